@@ -26,9 +26,9 @@ struct Surrogate {
     double mean_Q = 0.0, scale_Q = 1.0;
     std::vector<int> woff, boff;  // offsets of each layer in the flat parameter vector
     int nparam = 0;
-    DevBuf d_w, d_m, d_v, d_g, d_wb, d_wt, d_part, d_partb, d_loss, d_zero;
+    DevBuf d_w, d_m, d_v, d_g, d_wb, d_wt, d_part, d_loss;
     DevBuf d_act[SG_LAYERS + 1];  // x0 .. x5 (bf16 [B][N][C]); q (float [B][N]) in d_act[SG_LAYERS]
-    DevBuf d_dz[2];               // ping-pong gradient / tangent buffers (bf16 [B][N][64])
+    DevBuf d_dz[SG_LAYERS];       // gradient at each layer's output (bf16 [B][N][cout]); 0, 1: also tangents
     DevBuf d_bU, d_bQ, d_bF, d_idx;  // training minibatch gather buffers
     int capB = 0;
     long long adam_t = 0;

@@ -189,92 +189,223 @@ __global__ __launch_bounds__(COUT / 32 * 64) void sg_conv_kernel(int N, const __
     }
 }
 
-// Partial weight gradients of one tap over one chunk of (sample, site) rows:
-//   P[k][co][tap][ci] = sum_{s in chunk k} dZ[s][co] X[s + tap - 4][ci]
-// (X rows outside the sample read as zero), as an MFMA GEMM with M = co,
-// N = ci, K = sites.  Both tiles are staged transposed ([c][site]) so that
-// the eight consecutive sites of an operand fragment are contiguous.
-// grid (9, chunks); COUT/16 wavefronts.
-template <int CIN, int COUT>
-__global__ __launch_bounds__(COUT / 16 * 64) void sg_wgrad_kernel(int N, long long total, int sites_per_chunk,
-                                                                  const __bf16* __restrict__ dZ,
-                                                                  const __bf16* __restrict__ X,
-                                                                  float* __restrict__ P)
+// ---- parameter gradients of all layers in one launch
+//   dW_l[co][tap][ci] = sum_s dZ_l[s][co] X_l[s + tap - 4][ci],  db_l[co] = sum_s dZ_l[s][co]
+// (s over the sites of all samples, X = 0 outside a sample) as MFMA GEMMs with
+// M = co, N = ci, K = sites.  K runs over channels-fastest arrays, so an
+// operand fragment needs eight sites of one channel: a thread loads 8 sites x
+// 8 channels (eight 16-byte loads) and transposes them with v_perm_b32, half
+// an instruction per value.  A chunk of 256 sites is kept in LDS as 32 rows
+// with element e of row r the site r + 32 e: the tap shift s + tap - 4 is then
+// another row, never another element, so every fragment is one aligned
+// 16-byte read and the rows of tap 4..8 are those of tap 0..4 four rows on
+// (one K step of 32 sites), held in registers: 45 reads feed 72 MFMAs.
+// Jobs (blockIdx.y): 4 hidden layers x 4 tiles of 16 input channels (wavefront
+// w: output channels 16 w..16 w + 15, nine taps), then the first layer (3 real
+// inputs x 9 taps as the 27 columns of two tiles) and the last (9 taps as the
+// rows, one output channel).  Each workgroup walks a run of chunks and writes
+// one partial copy; sg_wreduce_kernel sums the copies in order.
+// At 32 x 2048 sites all six layers take 50 us (MFMA time 9 us; the rest is
+// the global loads and transposes of each chunk, three workgroups per CU
+// covering for each other) and the sum of the copies 7 us.  One launch per
+// layer with 2-byte transposing loads and a serial bias sum took 4.7 ms.
+constexpr int WG_R = 32;                 // rows of a chunk
+constexpr int WG_SITES = 8 * WG_R;       // sites of a chunk
+constexpr int WG_XR = WG_R + 2 * SG_HALO;
+constexpr int WG_JOBS = 4 * (SG_LAYERS - 2) + 2;
+constexpr int WG_GROUPS = 42;            // partial copies at most: 18 jobs x 42 workgroups fill 256 CUs three deep
+
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+
+struct SgWgradArgs {
+    const __bf16* dz[SG_LAYERS];  // gradient at layer l's output [site][cout]
+    const __bf16* x[SG_LAYERS];   // layer l's input [site][cin]
+    int woff[SG_LAYERS], boff[SG_LAYERS];
+    int N, cps, nchunks, per;     // sites and chunks per sample, chunks, chunks per workgroup
+    int nparam;
+    float* P;                     // [copy][nparam]
+};
+
+// eight channels of the eight sites n + 32 e of one sample (zero outside it)
+__device__ __forceinline__ void wg_load(const __bf16* __restrict__ src, int C, int n, int N, u32x4 (&v)[8])
 {
-    constexpr int NT = CIN / 16;  // 16-column tiles per wave
-    constexpr int KS = 32;        // sites per MFMA step
-    constexpr int LS = KS + 8;
-    __shared__ __attribute__((aligned(16))) __bf16 dzT[COUT * LS];
-    __shared__ __attribute__((aligned(16))) __bf16 xT[CIN * LS];
-    const int tap = blockIdx.x;
-    const int chunk = blockIdx.y;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int i = lane & 15, g = lane >> 4;
-    const long long s_begin = (long long)chunk * sites_per_chunk;
-    const long long s_end = std::min<long long>(total, s_begin + sites_per_chunk);
-    constexpr int NTHR = COUT / 16 * 64;
-    f4 acc[NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-    for (long long s0 = s_begin; s0 < s_end; s0 += KS) {
-        __syncthreads();
-        for (int q = threadIdx.x; q < KS * COUT; q += NTHR) {
-            const int s = q / COUT, c = q - s * COUT;
-            const long long gs = s0 + s;
-            dzT[c * LS + s] = gs < s_end ? dZ[gs * COUT + c] : (__bf16)0.0f;
-        }
-        for (int q = threadIdx.x; q < KS * CIN; q += NTHR) {
-            const int s = q / CIN, c = q - s * CIN;
-            const long long gs = s0 + s;
-            __bf16 v = (__bf16)0.0f;
-            if (gs < s_end) {
-                const long long bb = gs / N;
-                const long long n = gs - bb * N + tap - SG_HALO;
-                if (n >= 0 && n < N) v = X[(bb * N + n) * CIN + c];
-            }
-            xT[c * LS + s] = v;
-        }
-        __syncthreads();
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&dzT[(w * 16 + i) * LS + 8 * g]);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const bf16x8 bb = *reinterpret_cast<const bf16x8*>(&xT[(t * 16 + i) * LS + 8 * g]);
-            acc[t] = mfma_bf16(a, bb, acc[t]);
-        }
+    for (int e = 0; e < 8; ++e) {
+        const int m = n + WG_R * e;
+        v[e] = *reinterpret_cast<const u32x4*>(src + (size_t)min(max(m, 0), N - 1) * C);
     }
-    float* Pk = P + (size_t)chunk * COUT * SG_KW * CIN;
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int e = 0; e < 8; ++e) {
+        const int m = n + WG_R * e;
+        if (m < 0 || m >= N) v[e] = u32x4{0u, 0u, 0u, 0u};
+    }
+}
+
+// transposed: channel c of the eight at row[(c ^ swz) * 8], its eight sites together
+__device__ __forceinline__ void wg_store(const u32x4 (&v)[8], __bf16* row, int swz)
+{
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        u32x4 o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            o[q] = __builtin_amdgcn_perm(v[2 * q + 1][c >> 1], v[2 * q][c >> 1], c & 1 ? 0x07060302u : 0x05040100u);
+        *reinterpret_cast<u32x4*>(row + (c ^ swz) * 8) = o;
+    }
+}
+
+__global__ __launch_bounds__(256, 3) void sg_wgrad_kernel(SgWgradArgs a)
+{
+    __shared__ __attribute__((aligned(16))) __bf16 wide[WG_R * SG_C * 8];      // 64 channels, no halo
+    __shared__ __attribute__((aligned(16))) __bf16 halo[WG_XR * 16 * 8];       // 16 channels or 3 planes, with halo
+    const int job = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, g = lane >> 4;
+    const int c0 = blockIdx.x * a.per, c1 = min(a.nchunks, c0 + a.per);
+    const int N = a.N;
+    float* P = a.P + (size_t)blockIdx.x * a.nparam;
+    // wide tile: thread = (row tid / 8, channel octet tid % 8); the octet's number
+    // is mixed into the position inside it, so that 8 threads write 8 bank groups
+    const int wr = tid >> 3, wo = tid & 7;
+    __bf16* wdst = wide + (wr * SG_C + wo * 8) * 8;
+    const int wcol = 16 * w + i;                              // this lane's channel of the wide tile
+    const __bf16* wsrc = wide + (g * SG_C + (wcol & ~7) + ((wcol & 7) ^ (wcol >> 3))) * 8;
+    __attribute__((aligned(16))) __bf16 one8[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) one8[e] = (__bf16)1.0f;
+    const bf16x8 ones = *reinterpret_cast<const bf16x8*>(one8);
+
+    if (job < WG_JOBS - 2) {
+        const int l = 1 + (job >> 2), tile = job & 3;
+        const __bf16* dz = a.dz[l];
+        const __bf16* x = a.x[l] + tile * 16;
+        // halo tile: thread < 80 = (row tid / 2, octet tid % 2)
+        const int hr = tid >> 1, ho = tid & 1;
+        const bool hx = tid < 2 * WG_XR;
+        u32x4 vw[8];
+        auto load = [&](int c) {
+            const int b = c / a.cps, n0 = (c - b * a.cps) * WG_SITES;
+            wg_load(dz + (size_t)b * N * SG_C + wo * 8, SG_C, n0 + wr, N, vw);
+        };
+        f4 acc[SG_KW], accb = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < SG_KW; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+        if (c0 < c1) load(c0);
+        for (int c = c0; c < c1; ++c) {
+            wg_store(vw, wdst, wo);
+            if (hx) {
+                const int b = c / a.cps, n0 = (c - b * a.cps) * WG_SITES;
+                u32x4 vh[8];
+                wg_load(x + (size_t)b * N * SG_C + ho * 8, SG_C, n0 + hr - SG_HALO, N, vh);
+                wg_store(vh, halo + (hr * 16 + ho * 8) * 8, hr & 7);
+            }
+            __syncthreads();
+            if (c + 1 < c1) load(c + 1);
+            // fragment rho: row rho + g of the halo tile (tap t of step st: rho = 4 st + t)
+            auto frag = [&](int rho) {
+                const int row = rho + g;
+                return *reinterpret_cast<const bf16x8*>(halo + (row * 16 + (i ^ (row & 7))) * 8);
+            };
+            bf16x8 win[SG_KW];
+#pragma unroll
+            for (int t = 0; t < 5; ++t) win[t] = frag(t);
+#pragma unroll
+            for (int st = 0; st < WG_R / 4; ++st) {
+#pragma unroll
+                for (int t = 5; t < SG_KW; ++t) win[t] = frag(4 * st + t);
+                const bf16x8 av = *reinterpret_cast<const bf16x8*>(wsrc + 4 * st * SG_C * 8);
+#pragma unroll
+                for (int t = 0; t < SG_KW; ++t) acc[t] = mfma_bf16(av, win[t], acc[t]);
+                if (tile == 0) accb = mfma_bf16(av, ones, accb);
+#pragma unroll
+                for (int t = 0; t < 5; ++t) win[t] = win[t + 4];
+            }
+            __syncthreads();
+        }
+        float* Pw = P + a.woff[l];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int co = w * 16 + 4 * g + v;
-            const int ci = t * 16 + i;
-            Pk[((size_t)co * SG_KW + tap) * CIN + ci] = acc[t][v];
+            const int co = 16 * w + 4 * g + v;
+#pragma unroll
+            for (int t = 0; t < SG_KW; ++t) Pw[(co * SG_KW + t) * SG_C + tile * 16 + i] = acc[t][v];
+            if (tile == 0 && i == 0) P[a.boff[l] + co] = accb[v];
         }
+        return;
+    }
+    // first and last layer: one tile of 64 channels without halo, and planes of
+    // single channels with halo (3 inputs, or the one output gradient)
+    const bool first = job == WG_JOBS - 2;
+    const int l = first ? 0 : SG_LAYERS - 1;
+    const __bf16* wsr = first ? a.dz[0] : a.x[SG_LAYERS - 1];
+    const __bf16* psr = first ? a.x[0] : a.dz[SG_LAYERS - 1];
+    const int np = first ? SG_IN : 1;
+    u32x4 vw[8];
+    f4 acc[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}}, accb = acc[0];
+    // first layer: this lane's columns (input, tap) of the two tiles; last: its row (tap)
+    int prow[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int col = min(16 * t + i, SG_IN * SG_KW - 1);
+        prow[t] = first ? col / SG_KW * WG_XR + col % SG_KW : 2 * SG_HALO - min(i, SG_KW - 1);
+    }
+    for (int c = c0; c < c1; ++c) {
+        const int b = c / a.cps, n0 = (c - b * a.cps) * WG_SITES;
+        wg_load(wsr + (size_t)b * N * SG_C + wo * 8, SG_C, n0 + wr, N, vw);
+        wg_store(vw, wdst, wo);
+        for (int q = tid; q < np * WG_XR * 8; q += 256) {
+            const int p = q / (WG_XR * 8), r = q - p * WG_XR * 8, row = r >> 3, e = r & 7;
+            const int n = n0 + row - SG_HALO + WG_R * e;
+            const __bf16 v = psr[((size_t)b * N + min(max(n, 0), N - 1)) * SG_CP + p];
+            halo[q] = n >= 0 && n < N ? v : (__bf16)0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int st = 0; st < WG_R / 4; ++st) {
+            const bf16x8 wv = *reinterpret_cast<const bf16x8*>(wsrc + 4 * st * SG_C * 8);
+            const bf16x8 p0 = *reinterpret_cast<const bf16x8*>(halo + (prow[0] + 4 * st + g) * 8);
+            if (first) {
+                const bf16x8 p1 = *reinterpret_cast<const bf16x8*>(halo + (prow[1] + 4 * st + g) * 8);
+                acc[0] = mfma_bf16(wv, p0, acc[0]);
+                acc[1] = mfma_bf16(wv, p1, acc[1]);
+                accb = mfma_bf16(wv, ones, accb);
+            } else {
+                acc[0] = mfma_bf16(p0, wv, acc[0]);
+                accb = mfma_bf16(p0, ones, accb);
+            }
+        }
+        __syncthreads();
+    }
+    float* Pw = P + a.woff[l];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int m = 4 * g + v;
+        if (first) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int col = 16 * t + i;
+                if (col < SG_IN * SG_KW) Pw[((16 * w + m) * SG_KW + col % SG_KW) * SG_CP + col / SG_KW] = acc[t][v];
+            }
+            if (i == 0) P[a.boff[0] + 16 * w + m] = accb[v];
+        } else {
+            if (m < SG_KW) Pw[m * SG_C + 16 * w + i] = acc[0][v];
+            if (w == 0 && i == 0 && m == SG_HALO) P[a.boff[l]] = accb[v];  // tap 4: the sum of dq itself
+        }
+    }
 }
 
-// Partial bias gradients: Pb[k][co] = sum over chunk k's rows of dZ[s][co].
-__global__ void sg_bgrad_kernel(long long total, int sites_per_chunk, int cout, const __bf16* __restrict__ dZ,
-                                float* __restrict__ Pb)
-{
-    const int chunk = blockIdx.x;
-    const int co = threadIdx.x;
-    if (co >= cout) return;
-    const long long s0 = (long long)chunk * sites_per_chunk;
-    const long long s1 = std::min<long long>(total, s0 + sites_per_chunk);
-    float a = 0.f;
-    for (long long s = s0; s < s1; ++s) a += (float)dZ[s * cout + co];
-    Pb[(size_t)chunk * cout + co] = a;
-}
-
-// out[j] = sum_k P[k][j] in chunk order (deterministic).
-__global__ void sg_reduce_kernel(int nchunks, int len, const float* __restrict__ P, float* __restrict__ out)
+// out[j] = sum_k P[k][j] in copy order; entries of padding channels are 0.
+__global__ __launch_bounds__(256) void sg_wreduce_kernel(int ncopies, SgWgradArgs a, float* __restrict__ out)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= len) return;
-    float a = 0.f;
-    for (int k = 0; k < nchunks; ++k) a += P[(size_t)k * len + j];
-    out[j] = a;
+    if (j >= a.nparam) return;
+    const int r5 = j - a.woff[SG_LAYERS - 1], b5 = j - a.boff[SG_LAYERS - 1];
+    const bool pad = (j < a.boff[0] && j % SG_CP >= SG_IN) || (r5 >= SG_KW * SG_C && b5 < 0) || b5 > 0;
+    float s = 0.f;
+    if (!pad) {
+#pragma unroll 8
+        for (int k = 0; k < ncopies; ++k) s += a.P[(size_t)k * a.nparam + j];
+    }
+    out[j] = s;
 }
 
 __global__ void sg_input_kernel(int N, long long total, const double* __restrict__ U,
@@ -458,8 +589,8 @@ int Surrogate::ensure_batch(int B)
     for (int l = 0; l < SG_LAYERS; ++l)
         if ((rc = d_act[l].ensure(2 * sites * sg_cin(l)))) return rc;
     if ((rc = d_act[SG_LAYERS].ensure(sizeof(float) * sites))) return rc;
-    for (DevBuf* b : {&d_dz[0], &d_dz[1]})
-        if ((rc = b->ensure(2 * sites * SG_C))) return rc;
+    for (int l = 0; l < 2; ++l)
+        if ((rc = d_dz[l].ensure(2 * sites * SG_C))) return rc;
     capB = B;
     return NEGF_OK;
 }
@@ -533,42 +664,38 @@ int Surrogate::backward(int B, const double* dQt, double* loss, hipStream_t s)
     const long long sites = (long long)B * N;
     const int lblocks = (int)((sites + 255) / 256);
     if ((rc = d_loss.ensure(sizeof(float) * lblocks))) return rc;
+    for (int l = 0; l < SG_LAYERS; ++l)
+        if ((rc = d_dz[l].ensure(2 * (size_t)sites * sg_cout(l)))) return rc;
     hipLaunchKernelGGL(sg_loss_kernel, dim3(lblocks), dim3(256), 0, s, sites, d_act[SG_LAYERS].as<float>(), dQt,
-                       mean_Q, 1.0 / scale_Q, d_dz[0].as<__bf16>(), d_loss.as<float>());
-    const int spc = 2048;  // rows per gradient chunk
-    const int nchunks = (int)((sites + spc - 1) / spc);
-    if ((rc = d_part.ensure(sizeof(float) * (size_t)nchunks * SG_C * SG_KW * SG_C))) return rc;
-    if ((rc = d_partb.ensure(sizeof(float) * (size_t)nchunks * SG_C))) return rc;
-    int cur = 0;
-    for (int l = SG_LAYERS - 1; l >= 0; --l) {
-        const int cin = sg_cin(l), cout = sg_cout(l);
-        const __bf16* dz = d_dz[cur].as<__bf16>();
-        const __bf16* x = d_act[l].as<__bf16>();
-        if (cin == SG_C && cout == SG_C)
-            hipLaunchKernelGGL((sg_wgrad_kernel<SG_C, SG_C>), dim3(SG_KW, nchunks), dim3(256), 0, s, N, sites, spc,
-                               dz, x, d_part.as<float>());
-        else if (cin == SG_C)
-            hipLaunchKernelGGL((sg_wgrad_kernel<SG_C, SG_CP>), dim3(SG_KW, nchunks), dim3(128), 0, s, N, sites, spc,
-                               dz, x, d_part.as<float>());
-        else
-            hipLaunchKernelGGL((sg_wgrad_kernel<SG_CP, SG_C>), dim3(SG_KW, nchunks), dim3(256), 0, s, N, sites, spc,
-                               dz, x, d_part.as<float>());
-        const int lw = cout * SG_KW * cin;
-        hipLaunchKernelGGL(sg_reduce_kernel, dim3((lw + 255) / 256), dim3(256), 0, s, nchunks, lw,
-                           d_part.as<float>(), d_g.as<float>() + woff[l]);
-        hipLaunchKernelGGL(sg_bgrad_kernel, dim3(nchunks), dim3(64), 0, s, sites, spc, cout, dz, d_partb.as<float>());
-        hipLaunchKernelGGL(sg_reduce_kernel, dim3(1), dim3(64), 0, s, nchunks, cout, d_partb.as<float>(),
-                           d_g.as<float>() + boff[l]);
-        if (l == 0) break;
+                       mean_Q, 1.0 / scale_Q, d_dz[SG_LAYERS - 1].as<__bf16>(), d_loss.as<float>());
+    // every layer's gradient stays until the one launch that forms all weight gradients
+    for (int l = SG_LAYERS - 1; l > 0; --l) {
         // data gradient into layer l's input, through the tanh that made it
         const __bf16* wt = d_wt.as<__bf16>() + woff[l];
-        __bf16* dzn = d_dz[1 - cur].as<__bf16>();
-        if (cout == SG_C)
-            conv<SG_C, SG_C, EPI_DTANH>(N, B, dz, wt, nullptr, dzn, nullptr, x, s);
+        if (l == SG_LAYERS - 1)
+            conv<SG_CP, SG_C, EPI_DTANH>(N, B, d_dz[l].as<__bf16>(), wt, nullptr, d_dz[l - 1].as<__bf16>(), nullptr,
+                                         d_act[l].as<__bf16>(), s);
         else
-            conv<SG_CP, SG_C, EPI_DTANH>(N, B, dz, wt, nullptr, dzn, nullptr, x, s);
-        cur = 1 - cur;
+            conv<SG_C, SG_C, EPI_DTANH>(N, B, d_dz[l].as<__bf16>(), wt, nullptr, d_dz[l - 1].as<__bf16>(), nullptr,
+                                        d_act[l].as<__bf16>(), s);
     }
+    SgWgradArgs a;
+    for (int l = 0; l < SG_LAYERS; ++l) {
+        a.dz[l] = d_dz[l].as<__bf16>();
+        a.x[l] = d_act[l].as<__bf16>();
+        a.woff[l] = woff[l];
+        a.boff[l] = boff[l];
+    }
+    a.N = N;
+    a.cps = (N + WG_SITES - 1) / WG_SITES;
+    a.nchunks = B * a.cps;
+    a.per = (a.nchunks + WG_GROUPS - 1) / WG_GROUPS;
+    a.nparam = nparam;
+    const int copies = (a.nchunks + a.per - 1) / a.per;
+    if ((rc = d_part.ensure(sizeof(float) * (size_t)copies * nparam))) return rc;
+    a.P = d_part.as<float>();
+    hipLaunchKernelGGL(sg_wgrad_kernel, dim3(copies, WG_JOBS), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(sg_wreduce_kernel, dim3((nparam + 255) / 256), dim3(256), 0, s, copies, a, d_g.as<float>());
     NEGF_HIP_TRY(hipGetLastError());
     if (loss) {
         std::vector<float> h(lblocks);

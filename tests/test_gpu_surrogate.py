@@ -76,6 +76,26 @@ def test_gradient_matches_cpu_model(dev):
     sg.close()
 
 
+@pytest.mark.parametrize("N,B", [(16, 1), (255, 2), (256, 1), (257, 3), (40, 50), (600, 30)])
+def test_gradient_at_chunk_edges(dev, N, B):
+    """Samples shorter than, equal to and just past a 256-site chunk, one
+    sample, and more chunks than partial copies; tolerance as above."""
+    sg = Surrogate(N, seed=2)
+    p = S.init_params(seed=N)
+    norm = np.array([0.01, 0.2])
+    sg.set_params(p, norm)
+    U = smooth_U(B, N, seed=N + 1)
+    Q = norm[0] + norm[1] * np.random.default_rng(B).standard_normal((B, N))
+    _, gg = sg.gradient(U, Q)
+    _, gc = S.loss_and_grad(p, U, Q, norm[0], norm[1], None, bf=True)
+    lay, _ = S.layout()
+    for l, (wo, bo) in enumerate(lay):
+        for lo, hi in ((wo, bo), (bo, bo + S.cout(l))):
+            a, b = gg[lo:hi].astype(np.float64), gc[lo:hi]
+            assert np.linalg.norm(a - b) <= 5e-2 * np.linalg.norm(b), (l, lo)
+    sg.close()
+
+
 def test_jvp_matches_cpu_model_and_differences(dev):
     N, B = 180, 2
     sg = Surrogate(N, seed=3)
