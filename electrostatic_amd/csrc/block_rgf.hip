@@ -15,6 +15,10 @@
 // functions are then complex symmetric, which the backward step uses:
 //   G_bb = g_b + X G_{b+1,b+1} X^T,   X = g_b T.
 //
+// A chain whose T joins only the second part of a block with the first part of
+// the next (a tube cut into blocks of two rings), parts of 1..16 orbitals, is
+// swept part by part in block_split.hip; the kernels here take every other T.
+//
 // Layout.  Products run on v_mfma_f64_16x16x4f64 (lane l: A[i][k] with
 // i = l % 16, k = l / 16; B[k][j] with j = l % 16; result register v holds
 // D[l / 16 + 4 v][l % 16], as a GPU probe against numpy established for this
@@ -31,23 +35,13 @@
 #include <cmath>
 #include <vector>
 
+#include "block_device.h"
+#include "block_split.h"
 #include "negf_internal.h"
 
 namespace negf {
 
-typedef __attribute__((ext_vector_type(4))) double d4;
-
-constexpr int BM = 32;               // orbitals per block
-constexpr int BLD = 33;              // LDS row stride (doubles)
-constexpr int BPL = BM * BLD;        // doubles per LDS plane
 constexpr int BTHREADS = 256;        // 4 wavefronts (Sancho-Rubio: one quadrant each)
-constexpr int BGL = BM * BM;         // doubles per plane in global memory (row-major, unpadded)
-
-__device__ __forceinline__ d4 mfma64(double a, double b, d4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
 struct Quad {
     int lane, qi, qj;
     __device__ Quad()
@@ -104,11 +98,6 @@ __device__ __forceinline__ void store_quad(double* Mre, double* Mim, const d4& c
     }
 }
 
-__device__ __forceinline__ double mag2(double re, double im) { return re * re + im * im; }
-
-// max that keeps a NaN (so that a NaN never reads as converged)
-__device__ __forceinline__ double nan_max(double a, double b) { return (a > b || a != a) ? a : b; }
-
 // Pivot candidate key: |a|^2 (non-negative, so its bits order as an
 // unsigned integer) with the low 5 mantissa bits replaced by 31 - row, so
 // that the largest key is the largest magnitude and, among equal ones, the
@@ -116,16 +105,6 @@ __device__ __forceinline__ double nan_max(double a, double b) { return (a > b ||
 __device__ __forceinline__ unsigned long long pivot_key(double m, int i)
 {
     return ((unsigned long long)__double_as_longlong(m) & ~31ull) | (unsigned long long)(31 - i);
-}
-
-// 64-bit value of another lane by a DPP move (CTRL: a compile-time DPP
-// control word; all lanes active).
-template <int CTRL>
-__device__ __forceinline__ unsigned long long dpp64(unsigned long long v)
-{
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(v & 0xffffffffull), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), CTRL, 0xF, 0xF, false);
-    return ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo;
 }
 
 // max over each aligned group of 8 lanes: quad_perm [1,0,3,2], quad_perm
@@ -286,15 +265,6 @@ __device__ __forceinline__ void zero(Quad4& c)
     }
 }
 
-// LDS written by lanes of this wavefront is visible to its later reads.
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // c += A B over all four quadrants (same operand conventions as mm); SYM:
 // the product is known to be symmetric and quadrant (1, 0) is skipped.
 template <bool AC, bool BC, bool TA, bool TB, int LA = BLD, int LB = BLD, bool SYM = false>
@@ -371,155 +341,6 @@ __device__ __forceinline__ void store_quad4_sym(double* Mre, double* Mim, const 
             }
         }
     }
-}
-
-// 32-bit pivot key: |a|^2 rounded to float (non-negative, so its bits order
-// as an unsigned integer) with the low 5 mantissa bits replaced by 31 - row:
-// the largest key is a largest magnitude (to float precision, enough for a
-// pivot choice) and, among equal ones, the smallest row.  0: no candidate.
-__device__ __forceinline__ unsigned pivot_key32(double m, int i)
-{
-    return (__float_as_uint((float)m) & ~31u) | (unsigned)(31 - i);
-}
-
-template <int CTRL>
-__device__ __forceinline__ unsigned max_dpp(unsigned v)
-{
-    const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false);
-    return o > v ? o : v;
-}
-
-// max over the 64 lanes, read from lane 63: quad_perm [1,0,3,2], quad_perm
-// [2,3,0,1], row_half_mirror and row_mirror give every lane its row's
-// maximum; row_bcast:15 and row_bcast:31 carry the rows into lane 63.
-__device__ __forceinline__ unsigned wave_max32(unsigned v)
-{
-    v = max_dpp<0xB1>(v);
-    v = max_dpp<0x4E>(v);
-    v = max_dpp<0x141>(v);
-    v = max_dpp<0x140>(v);
-    v = max_dpp<0x142>(v);
-    v = max_dpp<0x143>(v);
-    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
-
-__device__ __forceinline__ double dpp_swap1(double x)
-{
-    return __longlong_as_double((long long)dpp64<0xB1>((unsigned long long)__double_as_longlong(x)));
-}
-
-__device__ __forceinline__ double readlane_f64(double x, int src)
-{
-    const long long b = __double_as_longlong(x);
-    const unsigned lo = __builtin_amdgcn_readlane((unsigned)(b & 0xffffffffll), src);
-    const unsigned hi = __builtin_amdgcn_readlane((unsigned)((unsigned long long)b >> 32), src);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// 1 / d for d > 0: hardware reciprocal estimate refined by two Newton-Raphson
-// steps y <- y + y (1 - d y), each of which squares the relative error.
-__device__ __forceinline__ double recip_nr(double d)
-{
-    double y = __builtin_amdgcn_rcp(d);
-    y = fma(y, fma(-d, y, 1.0), y);
-    return fma(y, fma(-d, y, 1.0), y);
-}
-
-// Inverse of the complex matrix (Mre, Mim) (LDS planes, row stride BLD) by
-// one wavefront, in place: Gauss-Jordan with partial pivoting.  Lane l holds
-// row i = l / 2, columns h * 16 .. h * 16 + 15 (h = l % 2) in registers.
-// Rows are never swapped: step k takes as pivot the largest |a_ik| among the
-// rows not yet used (|a_ik|^2 compared in float precision, ties to the
-// smallest row), found by a 64-lane maximum.
-// A pivot row is not divided by its pivot: each row keeps a scale s_i (1 until
-// it is the pivot, then 1 / pivot) and holds M / s_i, which leaves every
-// update in the form a_ij -= (a_ik / pivot) a_pj with the stored values; the
-// scales are applied once at the end.  The pivot element and the pivot row's
-// entries in column k + 1 are read from their lanes (v_readlane), so the next
-// pivot search waits on no memory; every lane fetches the pivot row's other
-// entries of its columns from the pivot row's lane of the same half by lane
-// shuffles (ds_bpermute), so no LDS store, wait and reload sits in a step.
-// perm (32 ints of LDS) records the pivot order.  The result is written back
-// through the pivot order: A^-1[q(i)][perm[j]] = s_i M[i][j], with q(i) the
-// step whose pivot was row i.
-__device__ __forceinline__ void gj_inverse_wave(double* Mre, double* Mim, int* perm, int lane)
-{
-    const int i = lane >> 1, h = lane & 1;
-    double ar[16], ai[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        ar[r] = Mre[i * BLD + h * 16 + r];
-        ai[r] = Mim[i * BLD + h * 16 + r];
-    }
-    unsigned used = 0u;  // bit x: row x has been a pivot (wave-uniform)
-    int qrow = 0;
-    double sr = 1.0, si = 0.0;
-    for (int kh = 0; kh < 2; ++kh) {
-#pragma unroll
-        for (int kr = 0; kr < 16; ++kr) {
-            const int k = kh * 16 + kr;
-            // pivot: column k is register kr of the lanes with h == kh
-            unsigned key = 0u;
-            if (h == kh && !((used >> i) & 1u)) key = pivot_key32(mag2(ar[kr], ai[kr]), i);
-            key = wave_max32(key);
-            const int p = key == 0u ? __builtin_ctz(~used) : 31 - (int)(key & 31u);
-            used |= 1u << p;
-            if (i == p) {
-                if (h == 0) perm[k] = p;
-                qrow = k;
-            }
-            // 1 / pivot from the lane holding (p, k)
-            const double pr = readlane_f64(ar[kr], 2 * p + kh), pim = readlane_f64(ai[kr], 2 * p + kh);
-            const double iv = recip_nr(pr * pr + pim * pim);
-            const double ir = pr * iv, ii = -pim * iv;
-            // multiplier of this row: a_ik / pivot (a_ik from the lane of this row holding column k)
-            const double orr = dpp_swap1(ar[kr]), oi = dpp_swap1(ai[kr]);
-            const double fr = (h == kh) ? ar[kr] : orr, fi = (h == kh) ? ai[kr] : oi;
-            double mr = fr * ir - fi * ii, mi = fr * ii + fi * ir;
-            if (i == p) {
-                mr = 0.0;
-                mi = 0.0;
-                sr = ir;
-                si = ii;
-            }
-            // register c (column k + 1 in the lanes of its half) first, with the
-            // pivot row's entries read from its two lanes: the next pivot search
-            // then waits on no shuffle
-            const int c = (kr + 1) & 15;
-            {
-                const double x0r = readlane_f64(ar[c], 2 * p), x0i = readlane_f64(ai[c], 2 * p);
-                const double x1r = readlane_f64(ar[c], 2 * p + 1), x1i = readlane_f64(ai[c], 2 * p + 1);
-                const double xr = h ? x1r : x0r, xi = h ? x1i : x0i;
-                ar[c] = fma(-mr, xr, fma(mi, xi, ar[c]));
-                ai[c] = fma(-mr, xi, fma(-mi, xr, ai[c]));
-            }
-            // the other entries of the pivot row, from the lane of its same half
-            // (the pivot row itself is not updated: m = 0)
-            const int src = 2 * p + h;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                if (r == c) continue;
-                const double2 x = make_double2(__shfl(ar[r], src, 64), __shfl(ai[r], src, 64));
-                ar[r] = fma(-mr, x.x, fma(mi, x.y, ar[r]));
-                ai[r] = fma(-mr, x.y, fma(-mi, x.x, ai[r]));
-            }
-            if (h == kh) {
-                ar[kr] = (i == p) ? 1.0 : -mr;
-                ai[kr] = (i == p) ? 0.0 : -mi;
-            }
-        }
-    }
-    wave_sync();
-    int pj[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) pj[r] = perm[h * 16 + r];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int o = qrow * BLD + pj[r];
-        Mre[o] = sr * ar[r] - si * ai[r];
-        Mim[o] = sr * ai[r] + si * ar[r];
-    }
-    wave_sync();
 }
 
 // Sancho-Rubio decimation for one energy (blockIdx.x) and one lead
@@ -804,22 +625,39 @@ __global__ __launch_bounds__(64 * WPB, 1) void block_rgf_kernel(int e0, int n, i
     }
 }
 
-// out[j] = sum_e part[e][j] in energy order.
-__global__ void block_reduce_kernel(int nE, int len, const double* __restrict__ part, double* __restrict__ out)
+// out[j] = sum_e part[e][j] in a fixed order: a workgroup covers 32 values x 8
+// slices of the energies (slice k: e = k, k + 8, ..., eight loads in flight),
+// the slices are then added in order.  One thread per value summing all
+// energies kept one wavefront's loads in flight per 64 values: 403 us for
+// 1024 energies x 16000 values (131 MB) against 22 us.
+__global__ __launch_bounds__(256) void block_reduce_kernel(int nE, int len, const double* __restrict__ part,
+                                                           double* __restrict__ out)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= len) return;
+    __shared__ double red[8][33];
+    const int x = threadIdx.x & 31, k = threadIdx.x >> 5;
+    const int j = blockIdx.x * 32 + x;
     double a = 0.0;
-    for (int e = 0; e < nE; ++e) a += part[(size_t)e * len + j];
-    out[j] = a;
+    if (j < len) {
+#pragma unroll 8
+        for (int e = k; e < nE; e += 8) a += part[(size_t)e * len + j];
+    }
+    red[k][x] = a;
+    __syncthreads();
+    if (k == 0 && j < len) {
+        double s = 0.0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s += red[q][x];
+        out[j] = s;
+    }
 }
 
 struct BlockChain {
     int nb = 0;
     int m = BM;  // orbitals per block of the caller; the device blocks are BM wide (padded)
     std::vector<double> H0, T;
+    SplitChain sp;  // h > 0: T joins only the second part of a block with the first of the next
     double Uc[2] = {0.0, 0.0};
-    DevBuf d_H0, d_T, d_v, d_E, d_coef, d_Sigma, d_iters, d_g, d_part, d_out, d_diag;
+    DevBuf d_mats, d_H0, d_T, d_v, d_E, d_coef, d_Sigma, d_iters, d_g, d_part, d_out, d_diag;
     size_t scratch_limit = (size_t)80 << 30;  // bytes of g_b (and g_b T) storage per launch
     float ms_sr = 0.f, ms_rgf = 0.f;
     hipStream_t st = nullptr;
@@ -834,6 +672,22 @@ struct BlockChain {
             if (x) (void)hipEventDestroy(x);
     }
 };
+
+// Lead self-energies into d_Sigma: [nE][2][re, im][32 x 32], or the split form.
+static int enqueue_sancho_rubio(BlockChain& c, int nE, double sr_tol, int sr_max_iter)
+{
+    if (c.sp.h) {
+        NEGF_HIP_TRY(split_sancho_rubio(c.sp, nE, c.d_E.as<double2>(), c.Uc[0], c.Uc[1], sr_tol, sr_max_iter,
+                                        c.d_Sigma.as<double>(), c.d_iters.as<int>(), c.st));
+        return NEGF_OK;
+    }
+    NEGF_HIP_TRY(hipMemsetAsync(c.d_iters.p, 0, sizeof(int) * 2 * nE, c.st));
+    hipLaunchKernelGGL(sancho_rubio_kernel, dim3(nE, 2), dim3(BTHREADS), 0, c.st, nE, c.d_E.as<double2>(),
+                       c.d_H0.as<double>(), c.d_T.as<double>(), c.Uc[0], c.Uc[1], sr_tol, sr_max_iter,
+                       c.d_Sigma.as<double>(), c.d_iters.as<int>());
+    NEGF_HIP_TRY(hipGetLastError());
+    return NEGF_OK;
+}
 
 }  // namespace negf
 
@@ -901,6 +755,20 @@ int negf_block_chain_create(int m, int nblocks, const double* H0, const double* 
         set_error("block chain upload failed");
         return fail(NEGF_EDEVICE);
     }
+    c.sp.m = m;
+    c.sp.nb = nblocks;
+    c.sp.h = split_part_size(m, T, BM);
+    if (c.sp.h) {
+        double mats[4 * 256];
+        split_matrices(m, c.sp.h, H0, T, BM, mats);
+        if ((rc = c.d_mats.ensure(sizeof(mats)))) return fail(rc);
+        if (hipMemcpy(c.d_mats.p, mats, sizeof(mats), hipMemcpyHostToDevice) != hipSuccess) {
+            set_error("block chain upload failed");
+            return fail(NEGF_EDEVICE);
+        }
+        c.sp.mats = c.d_mats.as<double>();
+        c.sp.v = c.d_v.as<double>();
+    }
     *out = h;
     return NEGF_OK;
 }
@@ -949,53 +817,57 @@ int negf_block_rgf(negf_block_chain* h, int nE, const negf_complex* E, const neg
         return NEGF_EARG;
     }
     BlockChain& c = h->c;
-    const int nb = c.nb;
-    const size_t len = (size_t)nb * BM;
+    const int nb = c.nb, m = c.m;
+    const bool split = c.sp.h > 0;
+    // the two-part sweep writes the caller's m orbitals only, the 32-wide one all of them
+    const int mw = split ? m : BM;
+    const size_t len = (size_t)nb * mw;
     int rc;
     if ((rc = c.d_E.ensure(sizeof(double2) * nE))) return rc;
     if ((rc = c.d_coef.ensure(sizeof(double2) * nE))) return rc;
-    if ((rc = c.d_Sigma.ensure(sizeof(double) * (size_t)nE * 4 * BGL))) return rc;
+    if ((rc = c.d_Sigma.ensure(sizeof(double) * (size_t)nE * (split ? 2 * SPLIT_SIGMA : 4 * BGL)))) return rc;
     if ((rc = c.d_iters.ensure(sizeof(int) * 2 * nE))) return rc;
     if ((rc = c.d_part.ensure(sizeof(double) * (size_t)nE * len))) return rc;
     if ((rc = c.d_out.ensure(sizeof(double) * len))) return rc;
     if (diagG && (rc = c.d_diag.ensure(sizeof(double2) * (size_t)nE * len))) return rc;
-    // g_b for every block and energy; also g_b T when all energies fit in one sweep that way
+    // g_b for every block and energy; 32-wide: also g_b T when all energies fit in one sweep that way
     const size_t per_g = (size_t)std::max(nb - 1, 1) * 2 * BGL * sizeof(double);
-    const bool keep_x = 2 * per_g * (size_t)nE <= c.scratch_limit;
-    const size_t per_energy = keep_x ? 2 * per_g : per_g;
+    const bool keep_x = !split && 2 * per_g * (size_t)nE <= c.scratch_limit;
+    const size_t per_energy = split ? split_scratch_per_energy(nb) : keep_x ? 2 * per_g : per_g;
     const int chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)nE, c.scratch_limit / per_energy));
     if ((rc = c.d_g.ensure(per_energy * chunk))) return rc;
+    double2* d_diag = diagG ? c.d_diag.as<double2>() : nullptr;
     NEGF_HIP_TRY(hipMemcpyAsync(c.d_E.p, E, sizeof(double2) * nE, hipMemcpyHostToDevice, c.st));
     NEGF_HIP_TRY(hipMemcpyAsync(c.d_coef.p, coef, sizeof(double2) * nE, hipMemcpyHostToDevice, c.st));
-    NEGF_HIP_TRY(hipMemsetAsync(c.d_iters.p, 0, sizeof(int) * 2 * nE, c.st));
     NEGF_HIP_TRY(hipEventRecord(c.ev[0], c.st));
-    hipLaunchKernelGGL(sancho_rubio_kernel, dim3(nE, 2), dim3(BTHREADS), 0, c.st, nE, c.d_E.as<double2>(),
-                       c.d_H0.as<double>(), c.d_T.as<double>(), c.Uc[0], c.Uc[1], sr_tol, sr_max_iter,
-                       c.d_Sigma.as<double>(), c.d_iters.as<int>());
-    NEGF_HIP_TRY(hipGetLastError());
+    if ((rc = enqueue_sancho_rubio(c, nE, sr_tol, sr_max_iter))) return rc;
     NEGF_HIP_TRY(hipEventRecord(c.ev[1], c.st));
     for (int e0 = 0; e0 < nE; e0 += chunk) {
         const int n = std::min(chunk, nE - e0);
+        if (split) {
+            NEGF_HIP_TRY(split_rgf(c.sp, e0, n, c.d_E.as<double2>(), c.d_coef.as<double2>(), c.d_Sigma.as<double>(),
+                                   c.d_g.as<double2>(), c.d_part.as<double>(), d_diag, c.st));
+            continue;
+        }
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((n + WPB - 1) / WPB), dim3(64 * WPB), 0, c.st, e0, n, nb,
+                               c.d_E.as<double2>(), c.d_coef.as<double2>(), c.d_H0.as<double>(), c.d_T.as<double>(),
+                               c.d_v.as<double>(), c.d_Sigma.as<double>(), c.d_g.as<double>(), c.d_part.as<double>(),
+                               d_diag);
+        };
         if (keep_x)
-            hipLaunchKernelGGL(block_rgf_kernel<true>, dim3((n + WPB - 1) / WPB), dim3(64 * WPB), 0, c.st, e0, n,
-                               nb, c.d_E.as<double2>(), c.d_coef.as<double2>(), c.d_H0.as<double>(),
-                               c.d_T.as<double>(), c.d_v.as<double>(), c.d_Sigma.as<double>(), c.d_g.as<double>(),
-                               c.d_part.as<double>(), diagG ? c.d_diag.as<double2>() : nullptr);
+            launch(block_rgf_kernel<true>);
         else
-            hipLaunchKernelGGL(block_rgf_kernel<false>, dim3((n + WPB - 1) / WPB), dim3(64 * WPB), 0, c.st, e0, n,
-                               nb, c.d_E.as<double2>(), c.d_coef.as<double2>(), c.d_H0.as<double>(),
-                               c.d_T.as<double>(), c.d_v.as<double>(), c.d_Sigma.as<double>(), c.d_g.as<double>(),
-                               c.d_part.as<double>(), diagG ? c.d_diag.as<double2>() : nullptr);
+            launch(block_rgf_kernel<false>);
         NEGF_HIP_TRY(hipGetLastError());
     }
     NEGF_HIP_TRY(hipEventRecord(c.ev[2], c.st));
-    hipLaunchKernelGGL(block_reduce_kernel, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, c.st, nE, (int)len,
+    hipLaunchKernelGGL(block_reduce_kernel, dim3((unsigned)((len + 31) / 32)), dim3(256), 0, c.st, nE, (int)len,
                        c.d_part.as<double>(), c.d_out.as<double>());
     NEGF_HIP_TRY(hipGetLastError());
     std::vector<int> it(2 * nE);
     NEGF_HIP_TRY(hipMemcpyAsync(it.data(), c.d_iters.p, sizeof(int) * 2 * nE, hipMemcpyDeviceToHost, c.st));
-    const int m = c.m;
-    if (m == BM) {
+    if (m == mw) {
         if (acc) NEGF_HIP_TRY(hipMemcpyAsync(acc, c.d_out.p, sizeof(double) * len, hipMemcpyDeviceToHost, c.st));
         if (diagG)
             NEGF_HIP_TRY(hipMemcpyAsync(diagG, c.d_diag.p, sizeof(double2) * (size_t)nE * len,
@@ -1033,28 +905,35 @@ int negf_block_self_energies(negf_block_chain* h, int nE, const negf_complex* E,
     BlockChain& c = h->c;
     int rc;
     if ((rc = c.d_E.ensure(sizeof(double2) * nE))) return rc;
-    if ((rc = c.d_Sigma.ensure(sizeof(double) * (size_t)nE * 4 * BGL))) return rc;
+    const int m = c.m;
+    const bool split = c.sp.h > 0;
+    const size_t n_sigma = (size_t)nE * (split ? 2 * SPLIT_SIGMA : 4 * BGL);
+    if ((rc = c.d_Sigma.ensure(sizeof(double) * n_sigma))) return rc;
     if ((rc = c.d_iters.ensure(sizeof(int) * 2 * nE))) return rc;
     NEGF_HIP_TRY(hipMemcpyAsync(c.d_E.p, E, sizeof(double2) * nE, hipMemcpyHostToDevice, c.st));
-    NEGF_HIP_TRY(hipMemsetAsync(c.d_iters.p, 0, sizeof(int) * 2 * nE, c.st));
-    hipLaunchKernelGGL(sancho_rubio_kernel, dim3(nE, 2), dim3(BTHREADS), 0, c.st, nE, c.d_E.as<double2>(),
-                       c.d_H0.as<double>(), c.d_T.as<double>(), c.Uc[0], c.Uc[1], sr_tol, sr_max_iter,
-                       c.d_Sigma.as<double>(), c.d_iters.as<int>());
-    NEGF_HIP_TRY(hipGetLastError());
+    if ((rc = enqueue_sancho_rubio(c, nE, sr_tol, sr_max_iter))) return rc;
     std::vector<int> it(2 * nE);
     NEGF_HIP_TRY(hipMemcpyAsync(it.data(), c.d_iters.p, sizeof(int) * 2 * nE, hipMemcpyDeviceToHost, c.st));
-    const int m = c.m;
-    if (m == BM) {
-        NEGF_HIP_TRY(hipMemcpyAsync(sigma, c.d_Sigma.p, sizeof(double) * (size_t)nE * 4 * BGL,
-                                    hipMemcpyDeviceToHost, c.st));
-    }
-    std::vector<double> full(m == BM ? 0 : (size_t)nE * 4 * BGL);
-    if (m != BM)
-        NEGF_HIP_TRY(hipMemcpyAsync(full.data(), c.d_Sigma.p, sizeof(double) * full.size(), hipMemcpyDeviceToHost,
-                                    c.st));
+    const bool direct = !split && m == BM;
+    std::vector<double> full(direct ? 0 : n_sigma);
+    NEGF_HIP_TRY(hipMemcpyAsync(direct ? sigma : full.data(), c.d_Sigma.p, sizeof(double) * n_sigma,
+                                hipMemcpyDeviceToHost, c.st));
     NEGF_HIP_TRY(hipStreamSynchronize(c.st));
+    if (split) {
+        // each lead's self-energy acts on the part next to it
+        std::fill(sigma, sigma + (size_t)nE * 4 * m * m, 0.0);
+        for (size_t q = 0; q < (size_t)nE * 2; ++q) {
+            const int o = q & 1 ? c.sp.h : 0, n = q & 1 ? m - c.sp.h : c.sp.h;
+            const double* src = full.data() + q * SPLIT_SIGMA;
+            double* dst = sigma + q * 2 * m * m;
+            for (int i = 0; i < n; ++i)
+                for (int j = 0; j < n; ++j)
+                    for (int pl = 0; pl < 2; ++pl)
+                        dst[((size_t)pl * m + o + i) * m + o + j] = src[2 * split_sigma_index(i, j) + pl];
+        }
+    }
     // the m x m leading submatrix of every [energy][lead][plane] matrix
-    for (size_t q = 0; m != BM && q < (size_t)nE * 4; ++q)
+    for (size_t q = 0; !split && m != BM && q < (size_t)nE * 4; ++q)
         for (int i = 0; i < m; ++i)
             std::copy(full.data() + q * BGL + (size_t)i * BM, full.data() + q * BGL + (size_t)i * BM + m,
                       sigma + q * m * m + (size_t)i * m);
