@@ -44,11 +44,14 @@
 // go on into the other half, where each inverts two matrices per part at once
 // (its own g and, with the other's stored self-energy, G).
 //
-// Bound by the FP64 VALU issue of the elimination steps (about 40 instructions
-// each).  Measured, 500 blocks of 32 orbitals, 1024 energies: sweep 9.0 ms against
-// 20.5 ms for the 32-orbital sweep (one wavefront per energy, pivoted inverse of
-// 1600 cycles per step), leads 0.88 ms against 4.5 ms (four wavefronts and a
-// barrier per pivot step); 40 blocks of 20 orbitals, 143 energies: 0.32 against
+// Bound by the FP64 VALU issue of the elimination steps (about 55 instructions
+// per pivot; row broadcasts as 64-bit DPP moves and a third-order reciprocal step).
+// One copy of the code serves blocks of both parities, 31 against 72 KB when it is
+// written out twice, at the same time.  Measured, 500 blocks of 32 orbitals, 1024
+// energies: sweep 8.6 ms against 20.5 ms for the 32-orbital sweep (one wavefront
+// per energy, pivoted inverse of 1600 cycles per step) and 9.0 ms with 32-bit DPP
+// moves and two Newton steps; leads 0.90 ms against 4.5 ms (four wavefronts and a
+// barrier per pivot step); 40 blocks of 20 orbitals, 143 energies: 0.31 against
 // 1.6 ms and 0.21 against 0.53 ms.
 #include "block_split.h"
 
@@ -257,10 +260,7 @@ __device__ __forceinline__ void inverse16s(M16 (&a)[NR][NR], double* lds, int la
 template <int K>
 __device__ __forceinline__ double row_lane(double x)
 {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
-    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, 0x150 + K, 0xF, 0xF, false);
-    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), 0x150 + K, 0xF, 0xF, false);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+    return __builtin_amdgcn_mov_dpp(x, 0x150 + K, 0xF, 0xF, true);
 }
 
 // A multiplier of a later row above the limit (squared here) sends the matrix to
@@ -268,17 +268,17 @@ __device__ __forceinline__ double row_lane(double x)
 // energies within the edge states of a disordered (16,0) tube, under 1%
 // elsewhere; the bits lost there are fewer than the condition of those blocks
 // costs (diag G within 1e-10 of the dense inverse given Sigma, as with a limit
-// of 8, which takes 16 instead of 9 ms for 500 x 1024 as half of those blocks
+// of 8, which took 16 instead of 9 ms for 500 x 1024 as half of those blocks
 // are inverted twice).  The leads (8): the doublings amplify every error, 256
 // costs up to four digits of Sigma.
 constexpr double CHAIN_GROW2 = 256.0 * 256.0, LEAD_GROW2 = 8.0 * 8.0;
 
 // Elimination step on column 4 T + K of a panel x (columns 4 T .. 4 T + 3; lane
 // (i, q): row i, column 4 T + q), pivot in row 4 T + K of the panel's own part.
-// y (if NR = 2): the panel's rows in the other part, CHECK: not yet pivots.
+// x[1] (if NR = 2): the panel's rows in the other part, check: not yet pivots.
 // Ends with -A_iJ P^-1 in the other rows and P^-1 in rows J.
-template <int T, int K, int NR, bool CHECK>
-__device__ __forceinline__ void panel_step(double2 (&x)[NR], int lane, bool& grow)
+template <int T, int K, int NR>
+__device__ __forceinline__ void panel_step(double2 (&x)[NR], int lane, bool& grow, bool check = false)
 {
     constexpr int row = 4 * T + K;
     asm volatile("" : "+v"(lane));  // the lane masks are made here: kept over all steps they spill
@@ -289,7 +289,9 @@ __device__ __forceinline__ void panel_step(double2 (&x)[NR], int lane, bool& gro
 #pragma unroll
     for (int r = 0; r < NR; ++r) c[r] = make_double2(bperm64(addr, x[r].x), bperm64(addr, x[r].y));
     const double pr = row_lane<row>(c[0].x), pi = row_lane<row>(c[0].y);
-    const double iv = recip_nr(fma(pr, pr, pi * pi));
+    // 1 / |pivot|^2: estimate and one third-order step y (1 + e + e^2), e = 1 - d y
+    const double d = fma(pr, pr, pi * pi), y = __builtin_amdgcn_rcp(d), ee = fma(-d, y, 1.0);
+    const double iv = fma(y, fma(ee, ee, ee), y);
     const double ir = pr * iv, ni = pi * iv;  // 1 / pivot = ir - i ni
     double rr = row_lane<row>(x[0].x), ri = row_lane<row>(x[0].y);
     rr = col ? 1.0 : rr;
@@ -299,7 +301,7 @@ __device__ __forceinline__ void panel_step(double2 (&x)[NR], int lane, bool& gro
         // -c / pivot
         double fr = -fma(c[r].x, ir, c[r].y * ni), fi = fma(c[r].x, ni, -c[r].y * ir);
         const bool big = !(fma(fr, fr, fi * fi) <= (NR == 1 ? CHAIN_GROW2 : LEAD_GROW2));
-        grow |= r == 0 ? big && i > row : CHECK && big;
+        grow |= r == 0 ? big && i > row : check && big;
         const bool p = r == 0 && prow;
         fr = p ? ir : fr;
         fi = p ? -ni : fi;
@@ -310,13 +312,13 @@ __device__ __forceinline__ void panel_step(double2 (&x)[NR], int lane, bool& gro
     }
 }
 
-template <int T, int NR, bool CHECK>
-__device__ __forceinline__ void panel_steps(double2 (&x)[NR], int lane, bool& grow)
+template <int T>
+__device__ __forceinline__ void panel_steps(double2 (&x)[2], int lane, bool& grow, bool check)
 {
-    panel_step<T, 0, NR, CHECK>(x, lane, grow);
-    panel_step<T, 1, NR, CHECK>(x, lane, grow);
-    panel_step<T, 2, NR, CHECK>(x, lane, grow);
-    panel_step<T, 3, NR, CHECK>(x, lane, grow);
+    panel_step<T, 0, 2>(x, lane, grow, check);
+    panel_step<T, 1, 2>(x, lane, grow, check);
+    panel_step<T, 2, 2>(x, lane, grow, check);
+    panel_step<T, 3, 2>(x, lane, grow, check);
 }
 
 // a(i, j) += sum_k o[j][k] b[i][k] for panels o and b
@@ -350,13 +352,13 @@ __device__ __forceinline__ void sweep16(M16 (&a)[NB], int lane, bool (&grow)[NB]
 #pragma unroll
     for (int n = 0; n < NB; ++n) x[n][0] = o[n] = make_double2(a[n].re[T], a[n].im[T]);
 #pragma unroll
-    for (int n = 0; n < NB; ++n) panel_step<T, 0, 1, false>(x[n], lane, grow[n]);
+    for (int n = 0; n < NB; ++n) panel_step<T, 0, 1>(x[n], lane, grow[n]);
 #pragma unroll
-    for (int n = 0; n < NB; ++n) panel_step<T, 1, 1, false>(x[n], lane, grow[n]);
+    for (int n = 0; n < NB; ++n) panel_step<T, 1, 1>(x[n], lane, grow[n]);
 #pragma unroll
-    for (int n = 0; n < NB; ++n) panel_step<T, 2, 1, false>(x[n], lane, grow[n]);
+    for (int n = 0; n < NB; ++n) panel_step<T, 2, 1>(x[n], lane, grow[n]);
 #pragma unroll
-    for (int n = 0; n < NB; ++n) panel_step<T, 3, 1, false>(x[n], lane, grow[n]);
+    for (int n = 0; n < NB; ++n) panel_step<T, 3, 1>(x[n], lane, grow[n]);
 #pragma unroll
     for (int n = 0; n < NB; ++n) {
         clear_rows<T>(a[n], lane);
@@ -379,14 +381,24 @@ __device__ __forceinline__ void neg_inverse16(M16 (&a)[NB], double* lds, int lan
         grow[n] = false;
     }
     sweep16<NS, NB>(a, lane, grow);
+    // (one copy of the elimination for all matrices)
+    bool any[NB];
+    bool some = false;
 #pragma unroll
-    for (int n = 0; n < NB; ++n)
-        if (__any(grow[n])) {
-            M16 b[1][1] = {{keep[n]}};
-            inverse16s<1, NS>(b, lds, lane);
-            a[n].re = -b[0][0].re;
-            a[n].im = -b[0][0].im;
-        }
+    for (int n = 0; n < NB; ++n) some |= any[n] = __any(grow[n]);
+    if (!some) return;
+#pragma unroll 1
+    for (int k = 0; k < NB; ++k) {
+        if (!any[NB == 1 ? 0 : k]) continue;
+        M16 b[1][1] = {{NB == 2 && k ? keep[NB - 1] : keep[0]}};
+        inverse16s<1, NS>(b, lds, lane);
+        b[0][0].re = -b[0][0].re;
+        b[0][0].im = -b[0][0].im;
+        if (NB == 2 && k)
+            a[NB - 1] = b[0][0];
+        else
+            a[0] = b[0][0];
+    }
 }
 
 constexpr int SLD = 17;            // row stride of a 16 x 16 LDS plane
@@ -429,10 +441,7 @@ __device__ __forceinline__ void sweep32_part(M16& own, M16& cross, M16& other, i
 {
     double2 x[2] = {make_double2(own.re[T], own.im[T]), make_double2(cross.re[T], cross.im[T])};
     const double2 o0 = x[0], o1 = x[1];
-    if (check)
-        panel_steps<T, 2, true>(x, lane, grow);
-    else
-        panel_steps<T, 2, false>(x, lane, grow);
+    panel_steps<T>(x, lane, grow, check);
     clear_rows<T>(own, lane);
     rank4(own, o0, x[0]);
     rank4(cross, o0, x[1]);
@@ -447,12 +456,18 @@ __device__ __forceinline__ void sweep32_part(M16& own, M16& cross, M16& other, i
 template <int NS>
 __device__ __forceinline__ bool sweep32(M16& pp, M16& rp, M16& rr, double* lds, int lane)
 {
-    bool grow = false;
-    sweep32_part<NS>(pp, rp, rr, lane, grow, true);
-    if (__any(grow)) return false;
-    rp = transpose16(rp, lds, lane);
-    sweep32_part<NS>(rr, rp, pp, lane, grow, false);
-    return !__any(grow);
+    // the columns of P, then (parts exchanged, one copy of the code) those of R
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+        bool grow = false;
+        sweep32_part<NS>(pp, rp, rr, lane, grow, half == 0);
+        if (__any(grow)) return false;
+        if (half == 0) rp = transpose16(rp, lds, lane);
+        const M16 t = pp;
+        pp = rr;
+        rr = t;
+    }
+    return true;
 }
 
 // E - H - diag(v) - ... of one part: the diagonal of rows i < np gets (er, ei)
@@ -531,58 +546,56 @@ __global__ __launch_bounds__(128, 2) void split_rgf_kernel(SplitChain c, int e0,
     Sn.re = -Sn.re;
     Sn.im = -Sn.im;
     double vj = pot(0);
-    // E - H - v + Sn of step j (parity p), and the potential of the next step
-    auto matrix = [&](int j, int p) {
+    // E - H - v + Sn of step j, and the potential of the next step.  H[0], Ct[0] are
+    // those of the present step: exchanged after each step, one copy of the code
+    // serves both parities (the inverses unrolled for each filled the
+    // instruction cache)
+    auto matrix = [&](int j) {
         M16 A;
-        A.re = Sn.re - H[p];
+        A.re = Sn.re - H[0];
         A.im = Sn.im;
-        add_diag(A, z.x - vj, z.y, (side ^ p) ? m - h : h, lane);
+        add_diag(A, z.x - vj, z.y, (side ^ (j & 1)) ? m - h : h, lane);
         vj = pot(min(j + 1, 2 * nb - 1));
         return A;
     };
-    auto advance = [&](const M16& gn, int p) {  // gn = -g
-        const M16 Q = prod_cr<NS>(gn, Ct[p], zero16());
-        Sn = symmetric16(prod_cr<NS>(Q, Ct[p], zero16()), lds, lane);
+    auto advance = [&](const M16& gn) {  // gn = -g
+        const M16 Q = prod_cr<NS>(gn, Ct[0], zero16());
+        Sn = symmetric16(prod_cr<NS>(Q, Ct[0], zero16()), lds, lane);
+        const d4 th = H[0], tc = Ct[0];
+        H[0] = H[1];
+        Ct[0] = Ct[1];
+        H[1] = th;
+        Ct[1] = tc;
     };
     // ---- to the middle
-    for (int j0 = 0; j0 < nb; j0 += 2) {
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const int j = j0 + p;
-            if (j < nb) {
-                store16(own + (size_t)j * 256, Sn, lane);
-                M16 a[1] = {matrix(j, p)};
-                neg_inverse16<NS, 1>(a, lds, lane);
-                advance(a[0], p);
-            }
-        }
+#pragma unroll 1
+    for (int j = 0; j < nb; ++j) {
+        store16(own + (size_t)j * 256, Sn, lane);
+        M16 a[1] = {matrix(j)};
+        neg_inverse16<NS, 1>(a, lds, lane);
+        advance(a[0]);
     }
     __syncthreads();  // the other side's self-energies are stored
     // ---- through the other half
     M16 So = load16(other + (size_t)(nb - 1) * 256, lane);
-    for (int j0 = nb & ~1; j0 < 2 * nb; j0 += 2) {
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const int j = j0 + p;
-            if (j >= nb) {
-                M16 a[2];
-                a[0] = matrix(j, p);
-                a[1] = M16{a[0].re + So.re, a[0].im + So.im};
-                So = load16(other + (size_t)max(2 * nb - 2 - j, 0) * 256, lane);
-                neg_inverse16<NS, 2>(a, lds, lane);
-                const int beta = side ? 2 * nb - 1 - j : j, bp = beta & 1;
-                if (i < (bp ? m - h : h) && (i & 3) == q) {
-                    const int v = i >> 2;
-                    const d4 re = a[1].re, im = a[1].im;
-                    const double gr = -(v == 0 ? re[0] : v == 1 ? re[1] : v == 2 ? re[2] : re[3]);
-                    const double gi = -(v == 0 ? im[0] : v == 1 ? im[1] : v == 2 ? im[2] : im[3]);
-                    const size_t o = (size_t)e * nb * m + (size_t)(beta >> 1) * m + bp * h + i;
-                    part[o] = fma(cf.x, gi, cf.y * gr);
-                    if (diag) diag[o] = make_double2(gr, gi);
-                }
-                if (j + 1 < 2 * nb) advance(a[0], p);
-            }
+#pragma unroll 1
+    for (int j = nb; j < 2 * nb; ++j) {
+        M16 a[2];
+        a[0] = matrix(j);
+        a[1] = M16{a[0].re + So.re, a[0].im + So.im};
+        So = load16(other + (size_t)max(2 * nb - 2 - j, 0) * 256, lane);
+        neg_inverse16<NS, 2>(a, lds, lane);
+        const int beta = side ? 2 * nb - 1 - j : j, bp = beta & 1;
+        if (i < (bp ? m - h : h) && (i & 3) == q) {
+            const int v = i >> 2;
+            const d4 re = a[1].re, im = a[1].im;
+            const double gr = -(v == 0 ? re[0] : v == 1 ? re[1] : v == 2 ? re[2] : re[3]);
+            const double gi = -(v == 0 ? im[0] : v == 1 ? im[1] : v == 2 ? im[2] : im[3]);
+            const size_t o = (size_t)e * nb * m + (size_t)(beta >> 1) * m + bp * h + i;
+            part[o] = fma(cf.x, gi, cf.y * gr);
+            if (diag) diag[o] = make_double2(gr, gi);
         }
+        advance(a[0]);
     }
 }
 
@@ -633,12 +646,21 @@ __global__ __launch_bounds__(128, 1) void split_sr_kernel(SplitChain c, const do
         gpr = M16{-G[0][1].re, -G[0][1].im};
         grr = M16{-G[1][1].re, -G[1][1].im};
     };
+    // the last pass (conv or it == max_iter) is the surface's own G, of es; one
+    // copy of the elimination serves both
     int it = 0;
     bool conv = false;
-    while (it < max_iter) {
-        ++it;
+    M16 sg;
+    for (;;) {
+        const bool last = conv || it >= max_iter;
         M16 gpp, gpr, grr;
-        green(eP, eR, gpp, gpr, grr);
+        green(last ? es : eP, last ? M16{HR, zr} : eR, gpp, gpr, grr);
+        if (last) {
+            const M16 Y = prod_cr<NS>(grr, a0, zero16());                   // -a0 g_RR
+            sg = symmetric16(prod_rc<NS>(a0, Y, zero16()), lds, lane);      // -a0 g_RR a0^T
+            break;
+        }
+        ++it;
         const M16 Y = prod_cc<NS>(grr, a, zero16());    // -a G_RR
         const M16 d = symmetric16(prod_cc<NS>(a, Y, zero16()), lds, lane);  // -a G_RR a^T
         es.re -= d.re;
@@ -659,15 +681,8 @@ __global__ __launch_bounds__(128, 1) void split_sr_kernel(SplitChain c, const do
         for (int v = 0; v < 4; ++v) mx = nan_max(mx, mag2(a.re[v], a.im[v]));
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) mx = nan_max(mx, __shfl_xor(mx, off));
-        if (mx < tol * tol) {
-            conv = true;
-            break;
-        }
+        conv = mx < tol * tol;
     }
-    M16 gpp, gpr, grr;
-    green(es, M16{HR, zr}, gpp, gpr, grr);
-    const M16 Y = prod_cr<NS>(grr, a0, zero16());  // -a0 g_RR
-    M16 sg = symmetric16(prod_rc<NS>(a0, Y, zero16()), lds, lane);  // -a0 g_RR a0^T
     sg.re = -sg.re;
     sg.im = -sg.im;
     store16(reinterpret_cast<double2*>(sigma) + ((size_t)e * 2 + side) * 256, sg, lane);
