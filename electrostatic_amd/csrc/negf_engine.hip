@@ -95,33 +95,28 @@ static void launch_sweep(int nblk, const WLaunch& lp, hipStream_t st)
     hipLaunchKernelGGL((sweep_kernel<NEGF_SUB_K, NEGF_SUB_NS, KIND, WG>), dim3(nblk), dim3(256), 0, st, lp);
 }
 
-static void launch_sweep_neq_full(int ns, int nblk, const WLaunch& lp, hipStream_t st)
-{
-    constexpr int K = NEGF_SUB_K;
-    switch (ns) {
-        case 1: hipLaunchKernelGGL((sweep_neq_full_kernel<K, 1>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 2: hipLaunchKernelGGL((sweep_neq_full_kernel<K, 2>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 3: hipLaunchKernelGGL((sweep_neq_full_kernel<K, 3>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 4: hipLaunchKernelGGL((sweep_neq_full_kernel<K, 4>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 5: hipLaunchKernelGGL((sweep_neq_full_kernel<K, 5>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 6: hipLaunchKernelGGL((sweep_neq_full_kernel<K, 6>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 7: hipLaunchKernelGGL((sweep_neq_full_kernel<K, 7>), dim3(nblk), dim3(256), 0, st, lp); break;
-        default: hipLaunchKernelGGL((sweep_neq_full_kernel<K, 8>), dim3(nblk), dim3(256), 0, st, lp); break;
-    }
-}
+#define SWEEP_TAIL_WAVES 2048  // two wavefronts per SIMD
 
-static void launch_sweep_eq_full(int ns, int nblk, const WLaunch& lp, hipStream_t st)
+// Sweep of full segments of ns sub-blocks (1 <= ns <= NS), partial segments beside them
+// when lp.ntail > 0.
+template <int NS>
+static void launch_sweep_full(int ns, int kind, const WLaunch& lp, hipStream_t st)
 {
+    if constexpr (NS > 1) {
+        if (ns < NS) return launch_sweep_full<NS - 1>(ns, kind, lp, st);
+    }
     constexpr int K = NEGF_SUB_K;
-    switch (ns) {
-        case 1: hipLaunchKernelGGL((sweep_eq_full_kernel<K, 1>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 2: hipLaunchKernelGGL((sweep_eq_full_kernel<K, 2>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 3: hipLaunchKernelGGL((sweep_eq_full_kernel<K, 3>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 4: hipLaunchKernelGGL((sweep_eq_full_kernel<K, 4>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 5: hipLaunchKernelGGL((sweep_eq_full_kernel<K, 5>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 6: hipLaunchKernelGGL((sweep_eq_full_kernel<K, 6>), dim3(nblk), dim3(256), 0, st, lp); break;
-        case 7: hipLaunchKernelGGL((sweep_eq_full_kernel<K, 7>), dim3(nblk), dim3(256), 0, st, lp); break;
-        default: hipLaunchKernelGGL((sweep_eq_full_kernel<K, 8>), dim3(nblk), dim3(256), 0, st, lp); break;
+    const dim3 grid((lp.nlist + lp.ntail + 3) / 4), block(256);
+    if (kind == KIND_EQ) {
+        if (lp.ntail)
+            hipLaunchKernelGGL((sweep_eq_full_kernel<K, NS, true>), grid, block, 0, st, lp);
+        else
+            hipLaunchKernelGGL((sweep_eq_full_kernel<K, NS, false>), grid, block, 0, st, lp);
+    } else {
+        if (lp.ntail)
+            hipLaunchKernelGGL((sweep_neq_full_kernel<K, NS, true>), grid, block, 0, st, lp);
+        else
+            hipLaunchKernelGGL((sweep_neq_full_kernel<K, NS, false>), grid, block, 0, st, lp);
     }
 }
 
@@ -257,11 +252,11 @@ int RgfPlan::build(int kind, bool write_G, const std::vector<RgfTube>& tubes, Ch
         for (int i = 0; i < G * P; ++i) {
             item_tube.push_back(t);
             if (w.fused == 2) continue;  // no separate sweep
-            // full segments of the equilibrium charge go to the unrolled sweep
+            // full segments of the charge go to the unrolled sweep (a launch that
+            // is asked for integrand samples takes the general one for all items)
             const int sgi = i % P;
             const bool full = sgi * L + L <= tb.N;
-            const bool samples = tb.sample[0] >= 0 || tb.sample[1] >= 0 || tb.sample[2] >= 0;
-            if (full && ((kind == KIND_EQ && !write_G) || (kind == KIND_NONEQ && !samples)))
+            if (full && ((kind == KIND_EQ && !write_G) || kind == KIND_NONEQ))
                 fast_items[L / NEGF_SUB_K].push_back(items + i);
             else
                 slow_items.push_back(items + i);
@@ -409,22 +404,34 @@ static int launch_rgf_kernels(const RgfLayout& y, const WLaunch& lp, hipStream_t
     if (y.any_fused2)
         hipLaunchKernelGGL((rgf_eq_fused_kernel<NEGF_SUB_K, NEGF_SUB_NS>), dim3(2 * y.nsblk), dim3(64 * EQF_WAVES), 0,
                            st, lp, y.nsblk);
+    // Partial segments run beside the longest full ones, in their launch; on their own
+    // they leave the chip to a few wavefronts for as long as a full sweep takes.  Their
+    // general form needs 256 registers: where the full sweep runs three wavefronts per
+    // SIMD (up to 4 sub-blocks) and its items need them, they keep a launch of their own.
+    // Measured, 143 energies x 4012 sites (44 in the last segment): equilibrium sweep 11.4
+    // us against 11.1 + 9.4 in series; non-equilibrium 13.7 us against 20.8 by the general
+    // sweep for every segment.
+    int tail_ns = 0;
+    for (int ns = 1; ns <= NEGF_SUB_NS; ++ns)
+        if (y.fast_n[ns] > 0 && (ns > 4 || y.fast_n[ns] + y.slow_n <= SWEEP_TAIL_WAVES)) tail_ns = ns;
+    if (y.kind == KIND_DOS || y.write_G) tail_ns = 0;
     for (int ns = 1; ns <= NEGF_SUB_NS; ++ns) {
         if (y.fast_n[ns] == 0) continue;
         WLaunch lf = lp;
         lf.item_list = y.item_list + y.fast_off[ns];
         lf.nlist = y.fast_n[ns];
-        if (y.kind == KIND_EQ)
-            launch_sweep_eq_full(ns, (y.fast_n[ns] + 3) / 4, lf, st);
-        else
-            launch_sweep_neq_full(ns, (y.fast_n[ns] + 3) / 4, lf, st);
+        if (ns == tail_ns) {
+            lf.tail_list = y.item_list + y.slow_off;
+            lf.ntail = y.slow_n;
+        }
+        launch_sweep_full<NEGF_SUB_NS>(ns, y.kind, lf, st);
     }
     WLaunch ls = lp;
     ls.item_list = y.item_list + y.slow_off;
     ls.nlist = y.slow_n;
     const int nblk_slow = (y.slow_n + 3) / 4;
-    if (y.slow_n == 0) {
-        // nothing left for the general sweep
+    if (y.slow_n == 0 || tail_ns) {
+        // nothing left for a launch of the general sweep
     } else if (y.kind == KIND_EQ) {
         if (y.write_G)
             launch_sweep<KIND_EQ, true>(nblk_slow, ls, st);
@@ -517,6 +524,15 @@ int RgfPlan::enqueue(double* d_out, double2* d_diagG, double* d_chain_out, hipSt
     y.any_fused2 = any_fused2_;
     y.any_unfused = any_unfused_;
     if (ntubes_ == 1 && tube0_.size() == sizeof(WTube)) y.tube1 = reinterpret_cast<const WTube*>(tube0_.data());
+    if (kind_ == KIND_NONEQ && d_chain_out) {
+        // integrand samples: only the general sweep writes them.  The fast and the
+        // general items are one list.
+        y.slow_off = 0;
+        for (int ns = 0; ns <= NEGF_SUB_NS; ++ns) {
+            y.slow_n += y.fast_n[ns];
+            y.fast_n[ns] = 0;
+        }
+    }
     const WLaunch lp = launch_params(y, d_diagG, d_chain_out, tube_active, d_site_out);
 
     if (dec_.use) {

@@ -75,6 +75,8 @@ struct WLaunch {
     double2* diagG;           // optional [chain][N]
     double* site_out;         // KIND_DOS, optional [chain][N]: the site's spectral weight
     double* chain_out;        // per-chain outputs
+    const int* tail_list;     // full-segment sweeps: partial segments that share the launch
+    int ntail;
     double* dos_part;         // [item][64] per-segment DOS traces
     const int* sblk_tube;     // chain groups: tube
     const int* sblk_chain;    // chain groups: group index within the tube
@@ -1231,19 +1233,13 @@ __device__ __forceinline__ void site_loop(const Coefs& k, const double (&Us)[K],
     }
 }
 
-template <int K, int NS, int KIND, bool WRITE_G>
-__global__ __launch_bounds__(256, 2) void sweep_kernel(WLaunch lp)
+// Passes 2 and 3 of one item on a wavefront with LDS of its own: red (K x 65),
+// us (NEGF_SEG_MAX) and, for row outputs, rowst (1024).  SAMP: integrand samples
+// may be asked for (KIND_NONEQ).
+template <int K, int NS, int KIND, bool WRITE_G, bool SAMP>
+__device__ __forceinline__ void sweep_body(const WLaunch& lp, int item, int lane, double* red, double* us,
+                                           double* rowst)
 {
-    __shared__ double red_all[4][K * 65];
-    __shared__ double us_all[4][NEGF_SEG_MAX];
-    constexpr bool ROWS = WRITE_G || KIND == KIND_DOS;  // row outputs staged in LDS
-    __shared__ double rowst_all[ROWS ? 4 : 1][ROWS ? 1024 : 1];
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
-    const int idx = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);
-    if (idx >= lp.nlist) return;
-    const int item = lp.item_list ? __builtin_amdgcn_readfirstlane(lp.item_list[idx]) : idx;
-    double* red = red_all[wv];
     WTube tube;
     ItemCtx ic = item_ctx(lp, item, lane, tube);
     if (tube_skipped(lp, tube)) return;  // whole wavefront
@@ -1253,7 +1249,6 @@ __global__ __launch_bounds__(256, 2) void sweep_kernel(WLaunch lp)
     const int lo = min(N, ic.s * tube.L);
     const int hi = min(N, lo + tube.L);
     const int nsub = (hi - lo + K - 1) / K;  // wave-uniform
-    double* us = us_all[wv];
     stage_segment(us, tube.U, lo, hi, lane);
     const double* S = lp.St + (long long)item * 10 * 64 + lane;
     double2 ux = make_double2(S[0], S[64]), uy = make_double2(S[128], S[192]);
@@ -1305,9 +1300,9 @@ __global__ __launch_bounds__(256, 2) void sweep_kernel(WLaunch lp)
     {
         const long long row0 = (long long)(tube.chain0 + ic.g * 64) * N;
         const int nvalid = min(64, tube.nchain - ic.g * 64);
-        if (WRITE_G) go = RowOut{reinterpret_cast<char*>(lp.diagG + row0), N, nvalid, rowst_all[ROWS ? wv : 0]};
+        if (WRITE_G) go = RowOut{reinterpret_cast<char*>(lp.diagG + row0), N, nvalid, rowst};
         if (KIND == KIND_DOS && lp.site_out)
-            so = RowOut{reinterpret_cast<char*>(lp.site_out + row0), N, nvalid, rowst_all[ROWS ? wv : 0]};
+            so = RowOut{reinterpret_cast<char*>(lp.site_out + row0), N, nvalid, rowst};
     }
     for (int j = 0; j < nsub; ++j) {
         const int p0 = lo + j * K;
@@ -1373,12 +1368,12 @@ __global__ __launch_bounds__(256, 2) void sweep_kernel(WLaunch lp)
         sc.aL = aL;
         sc.aR = aR;
         bool samp = false;
-        if (KIND == KIND_NONEQ && lp.chain_out) {
+        if (SAMP && lp.chain_out) {
 #pragma unroll
             for (int w = 0; w < 3; ++w) samp |= (tube.sample[w] >= p0 && tube.sample[w] < p0 + len);
         }
-        if (samp)
-            site_loop<K, KIND, WRITE_G, false, true>(k, Us, vr, ux, uy, sc, p0, len, ic.valid, go, so, red, lane,
+        if (SAMP && samp)
+            site_loop<K, KIND, WRITE_G, false, SAMP>(k, Us, vr, ux, uy, sc, p0, len, ic.valid, go, so, red, lane,
                                                      dos_acc, tube, ch, lp.chain_out);
         else if (len == K)
             site_loop<K, KIND, WRITE_G, true, false>(k, Us, vr, ux, uy, sc, p0, len, ic.valid, go, so, red, lane,
@@ -1392,6 +1387,22 @@ __global__ __launch_bounds__(256, 2) void sweep_kernel(WLaunch lp)
         }
     }
     if (KIND == KIND_DOS) lp.dos_part[(long long)item * 64 + lane] = dos_acc;
+}
+
+template <int K, int NS, int KIND, bool WRITE_G>
+__global__ __launch_bounds__(256, 2) void sweep_kernel(WLaunch lp)
+{
+    __shared__ double red_all[4][K * 65];
+    __shared__ double us_all[4][NEGF_SEG_MAX];
+    constexpr bool ROWS = WRITE_G || KIND == KIND_DOS;  // row outputs staged in LDS
+    __shared__ double rowst_all[ROWS ? 4 : 1][ROWS ? 1024 : 1];
+    const int lane = threadIdx.x & 63;
+    const int wv = threadIdx.x >> 6;
+    const int idx = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);
+    if (idx >= lp.nlist) return;
+    const int item = lp.item_list ? __builtin_amdgcn_readfirstlane(lp.item_list[idx]) : idx;
+    sweep_body<K, NS, KIND, WRITE_G, KIND == KIND_NONEQ>(lp, item, lane, red_all[wv], us_all[wv],
+                                                         rowst_all[ROWS ? wv : 0]);
 }
 
 // Passes 2 and 3 of the equilibrium sweep over a full segment of K NS sites
@@ -1507,17 +1518,25 @@ __device__ __forceinline__ void eq_full_body(const KC& k, const double* us, doub
 // the entry states become w_lo = u_lo, w_{lo-1} = ai_{lo-1} u_{lo-1},
 // w'_{hi-1} = v_{hi-1}, w'_hi = ai_{hi-1} v_hi (u_n v_n = C w_n w'_n with the
 // segment constant C, which also divides W and so drops out).
-template <int K, int NS>
-__global__ __launch_bounds__(256, NS <= 4 ? 3 : 2) void sweep_eq_full_kernel(WLaunch lp)
+template <int K, int NS, bool TAIL>
+__global__ __launch_bounds__(256, NS <= 4 && !TAIL ? 3 : 2) void sweep_eq_full_kernel(WLaunch lp)
 {
     __shared__ double red_all[4][K * 65];
-    __shared__ double us_all[4][K * NS];
+    __shared__ double us_all[4][TAIL ? NEGF_SEG_MAX : K * NS];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    const int idx = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);
+    int idx = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);
+    double* red = red_all[wv];
+    if (TAIL) {
+        if (idx < lp.ntail) {
+            const int item = __builtin_amdgcn_readfirstlane(lp.tail_list[idx]);
+            sweep_body<K, NEGF_SUB_NS, KIND_EQ, false, false>(lp, item, lane, red, us_all[wv], nullptr);
+            return;
+        }
+        idx -= lp.ntail;
+    }
     if (idx >= lp.nlist) return;
     const int item = __builtin_amdgcn_readfirstlane(lp.item_list[idx]);
-    double* red = red_all[wv];
     WTube tube;
     ItemCtx ic = item_ctx(lp, item, lane, tube);
     if (tube_skipped(lp, tube)) return;  // whole wavefront
@@ -1920,17 +1939,25 @@ __device__ __forceinline__ void neq_full_scaled(const SCoefs& k, const double* u
 // recurrence, never renormalised: |ut_n| is |G_n,N-1| up to the constant) and,
 // per sub-block, vt = sqrt|kL Gamma_L| 2^(e_v - e_D) v / |D|; the signs of the
 // two weights multiply the squared moduli.
-template <int K, int NS>
-__global__ __launch_bounds__(256, NS <= 4 ? 3 : 2) void sweep_neq_full_kernel(WLaunch lp)
+template <int K, int NS, bool TAIL>
+__global__ __launch_bounds__(256, NS <= 4 && !TAIL ? 3 : 2) void sweep_neq_full_kernel(WLaunch lp)
 {
     __shared__ double red_all[4][K * 65];
-    __shared__ double us_all[4][K * NS];
+    __shared__ double us_all[4][TAIL ? NEGF_SEG_MAX : K * NS];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    const int idx = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);
+    int idx = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);
+    double* red = red_all[wv];
+    if (TAIL) {
+        if (idx < lp.ntail) {
+            const int item = __builtin_amdgcn_readfirstlane(lp.tail_list[idx]);
+            sweep_body<K, NEGF_SUB_NS, KIND_NONEQ, false, false>(lp, item, lane, red, us_all[wv], nullptr);
+            return;
+        }
+        idx -= lp.ntail;
+    }
     if (idx >= lp.nlist) return;
     const int item = __builtin_amdgcn_readfirstlane(lp.item_list[idx]);
-    double* red = red_all[wv];
     WTube tube;
     ItemCtx ic = item_ctx(lp, item, lane, tube);
     if (tube_skipped(lp, tube)) return;  // whole wavefront
