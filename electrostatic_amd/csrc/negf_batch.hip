@@ -97,14 +97,14 @@ class Batch {
         std::vector<RgfTube> teq, tneq;
         for (int i = 0; i < n; ++i) {
             Tube& t = *tubes[i];
-            RgfTube r = t.rgf_tube(t.d_U.as<double>(), t.d_Uc.as<double>(), (int)t.eq_host.size(), seg_len);
+            RgfTube r = t.rgf_tube(t.d_U.as<double>(), t.d_Uc(), (int)t.eq_host.size(), seg_len);
             r.chain0 = (int)eq.size();
             r.out_off = off[i];
             r.ext = i;
             eq.insert(eq.end(), t.eq_host.begin(), t.eq_host.end());
             teq.push_back(r);
             if (!t.neq_host.empty()) {
-                RgfTube q = t.rgf_tube(t.d_U.as<double>(), t.d_Uc.as<double>(), (int)t.neq_host.size(), seg_len);
+                RgfTube q = t.rgf_tube(t.d_U.as<double>(), t.d_Uc(), (int)t.neq_host.size(), seg_len);
                 q.chain0 = (int)neq.size();
                 q.out_off = off[i];
                 q.ext = i;

@@ -123,10 +123,7 @@ static void launch_sweep_full(int ns, int kind, const WLaunch& lp, hipStream_t s
 // ---------------------------------------------------------------- plan
 RgfPlan::~RgfPlan()
 {
-    DevBuf* bufs[] = {&d_item_list_, &d_tubes_,    &d_item_tube_, &d_chain_tube_,  &d_sblk_tube_,
-                      &d_sblk_chain_, &d_Tm_,       &d_St_,        &d_Dd_,          &d_part_,
-                      &d_dos_part_,   &d_status_,   &d_red_src_off_, &d_red_nrows_, &d_red_N_,
-                      &d_red_dst_off_};
+    DevBuf* bufs[] = {&d_tab_, &d_Tm_, &d_St_, &d_Dd_, &d_part_, &d_dos_part_};
     for (DevBuf* b : bufs) b->release();
     for (hipEvent_t e : ev_start_) (void)hipEventDestroy(e);
     for (hipEvent_t e : ev_stop_) (void)hipEventDestroy(e);
@@ -286,31 +283,43 @@ int RgfPlan::build(int kind, bool write_G, const std::vector<RgfTube>& tubes, Ch
     if ((rc = d_Dd_.ensure((size_t)nchains * 3 * sizeof(double)))) return rc;
     if ((rc = d_part_.ensure(std::max<long long>(1, poff) * sizeof(double)))) return rc;
     if (kind == KIND_DOS && (rc = d_dos_part_.ensure((size_t)items * 64 * sizeof(double)))) return rc;
-    if ((rc = upload(d_tubes_, wt))) return rc;
     tube0_.assign(reinterpret_cast<const unsigned char*>(wt.data()),
                   reinterpret_cast<const unsigned char*>(wt.data()) + sizeof(WTube));
-    if ((rc = upload(d_item_tube_, item_tube))) return rc;
-    {
-        std::vector<int> all;
-        for (int ns = 1; ns <= NEGF_SUB_NS; ++ns) {
-            fast_off_[ns] = (int)all.size();
-            fast_n_[ns] = (int)fast_items[ns].size();
-            all.insert(all.end(), fast_items[ns].begin(), fast_items[ns].end());
-        }
-        slow_off_ = (int)all.size();
-        slow_n_ = (int)slow_items.size();
-        all.insert(all.end(), slow_items.begin(), slow_items.end());
-        if ((rc = upload(d_item_list_, all))) return rc;
+    std::vector<int> all;
+    for (int ns = 1; ns <= NEGF_SUB_NS; ++ns) {
+        fast_off_[ns] = (int)all.size();
+        fast_n_[ns] = (int)fast_items[ns].size();
+        all.insert(all.end(), fast_items[ns].begin(), fast_items[ns].end());
     }
-    if ((rc = upload(d_chain_tube_, chain_tube))) return rc;
-    if ((rc = upload(d_sblk_tube_, sblk_tube))) return rc;
-    if ((rc = upload(d_sblk_chain_, sblk_chain))) return rc;
-    if ((rc = upload(d_red_src_off_, rsrc))) return rc;
-    if ((rc = upload(d_red_nrows_, rnrows))) return rc;
-    if ((rc = upload(d_red_N_, rN))) return rc;
-    if ((rc = upload(d_red_dst_off_, rdst))) return rc;
-    if ((rc = d_status_.ensure(sizeof(int)))) return rc;
-    NEGF_HIP_TRY(hipMemset(d_status_.p, 0, sizeof(int)));
+    slow_off_ = (int)all.size();
+    slow_n_ = (int)slow_items.size();
+    all.insert(all.end(), slow_items.begin(), slow_items.end());
+    // all tables and the cleared status word in one copy: each one is a round trip of
+    // its own to the device, and a plan of one short chain is otherwise mostly those
+    std::vector<unsigned char> tab;
+    auto put = [&tab](const auto& v) {
+        const size_t o = tab.size(), n = v.size() * sizeof(v[0]);
+        tab.resize(o + (n + 255) / 256 * 256);
+        if (n) std::memcpy(tab.data() + o, v.data(), n);
+        return o;
+    };
+    const size_t o_status = put(std::vector<int>{0}), o_tubes = put(wt), o_item_tube = put(item_tube);
+    const size_t o_items = put(all), o_chain_tube = put(chain_tube), o_sblk_tube = put(sblk_tube);
+    const size_t o_sblk_chain = put(sblk_chain), o_rsrc = put(rsrc), o_rnrows = put(rnrows), o_rN = put(rN);
+    const size_t o_rdst = put(rdst);
+    if ((rc = upload(d_tab_, tab))) return rc;
+    const unsigned char* d = d_tab_.as<const unsigned char>();
+    d_status_ = d_tab_.as<int>() + o_status / sizeof(int);
+    d_tubes_ = reinterpret_cast<const WTube*>(d + o_tubes);
+    d_item_tube_ = reinterpret_cast<const int*>(d + o_item_tube);
+    d_item_list_ = reinterpret_cast<const int*>(d + o_items);
+    d_chain_tube_ = reinterpret_cast<const int*>(d + o_chain_tube);
+    d_sblk_tube_ = reinterpret_cast<const int*>(d + o_sblk_tube);
+    d_sblk_chain_ = reinterpret_cast<const int*>(d + o_sblk_chain);
+    d_red_src_off_ = reinterpret_cast<const long long*>(d + o_rsrc);
+    d_red_nrows_ = reinterpret_cast<const int*>(d + o_rnrows);
+    d_red_N_ = reinterpret_cast<const int*>(d + o_rN);
+    d_red_dst_off_ = reinterpret_cast<const long long*>(d + o_rdst);
     return NEGF_OK;
 }
 
@@ -497,12 +506,12 @@ int RgfPlan::enqueue(double* d_out, double2* d_diagG, double* d_chain_out, hipSt
     y.max_N = max_N_;
     y.max_rows = max_rows_;
     y.chains = d_chains_;
-    y.tubes = d_tubes_.as<WTube>();
-    y.item_tube = d_item_tube_.as<int>();
-    y.chain_tube = d_chain_tube_.as<int>();
-    y.sblk_tube = d_sblk_tube_.as<int>();
-    y.sblk_chain = d_sblk_chain_.as<int>();
-    y.item_list = d_item_list_.as<int>();
+    y.tubes = d_tubes_;
+    y.item_tube = d_item_tube_;
+    y.chain_tube = d_chain_tube_;
+    y.sblk_tube = d_sblk_tube_;
+    y.sblk_chain = d_sblk_chain_;
+    y.item_list = d_item_list_;
     for (int ns = 0; ns <= NEGF_SUB_NS; ++ns) {
         y.fast_off[ns] = fast_off_[ns];
         y.fast_n[ns] = fast_n_[ns];
@@ -514,11 +523,11 @@ int RgfPlan::enqueue(double* d_out, double2* d_diagG, double* d_chain_out, hipSt
     y.Dd = d_Dd_.as<double>();
     y.part = d_part_.as<double>();
     y.dos_part = d_dos_part_.as<double>();
-    y.status = d_status_.as<int>();
-    y.red_src_off = d_red_src_off_.as<long long>();
-    y.red_nrows = d_red_nrows_.as<int>();
-    y.red_N = d_red_N_.as<int>();
-    y.red_dst_off = d_red_dst_off_.as<long long>();
+    y.status = d_status_;
+    y.red_src_off = d_red_src_off_;
+    y.red_nrows = d_red_nrows_;
+    y.red_N = d_red_N_;
+    y.red_dst_off = d_red_dst_off_;
     y.dec = dec_;
     y.any_fused = any_fused_;
     y.any_fused2 = any_fused2_;
@@ -566,9 +575,9 @@ int RgfPlan::enqueue(double* d_out, double2* d_diagG, double* d_chain_out, hipSt
 int RgfPlan::check_status(hipStream_t st, int* status)
 {
     int h = 0;
-    NEGF_HIP_TRY(hipMemcpyAsync(&h, d_status_.p, sizeof(int), hipMemcpyDeviceToHost, st));
+    NEGF_HIP_TRY(hipMemcpyAsync(&h, d_status_, sizeof(int), hipMemcpyDeviceToHost, st));
     NEGF_HIP_TRY(hipStreamSynchronize(st));
-    if (h) NEGF_HIP_TRY(hipMemsetAsync(d_status_.p, 0, sizeof(int), st));
+    if (h) NEGF_HIP_TRY(hipMemsetAsync(d_status_, 0, sizeof(int), st));
     *status = h;
     if (h & 2) {  // bit 1: set by rgf_eq_fused_kernel when a wait exceeded its bound
         set_error("fused RGF kernel: a wavefront's wait for the v walk exceeded its bound");

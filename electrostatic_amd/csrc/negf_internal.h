@@ -102,7 +102,7 @@ class RgfPlan {
     // Read and clear the device status word (synchronises the stream).
     int check_status(hipStream_t st, int* status);
     // The device status word itself (an int), for a copy enqueued by the caller.
-    const int* status_ptr() const { return d_status_.as<int>(); }
+    const int* status_ptr() const { return d_status_; }
     int num_items() const { return nitems_; }
     // hipEvent timing of the RGF kernels (transfer + scan + sweep)
     void enable_timing(bool on) { timing_ = on; }
@@ -119,11 +119,15 @@ class RgfPlan {
     ChainDesc* d_chains_ = nullptr;
     DecParams dec_;
     std::vector<RgfTube> tubes_;
-    DevBuf d_tubes_, d_item_tube_, d_chain_tube_, d_sblk_tube_, d_sblk_chain_, d_item_list_;
+    DevBuf d_tab_;  // status word and tables, and where each begins
+    int* d_status_ = nullptr;
+    const struct WTube* d_tubes_ = nullptr;
+    const int *d_item_tube_ = nullptr, *d_chain_tube_ = nullptr, *d_sblk_tube_ = nullptr, *d_sblk_chain_ = nullptr;
+    const int *d_item_list_ = nullptr, *d_red_nrows_ = nullptr, *d_red_N_ = nullptr;
+    const long long *d_red_src_off_ = nullptr, *d_red_dst_off_ = nullptr;  // fixed-order row reduction
     int fast_off_[NEGF_SUB_NS + 1] = {}, fast_n_[NEGF_SUB_NS + 1] = {};  // unrolled sweep items by sub-blocks
     int slow_off_ = 0, slow_n_ = 0;                                      // general sweep items
-    DevBuf d_Tm_, d_St_, d_Dd_, d_part_, d_dos_part_, d_status_;
-    DevBuf d_red_src_off_, d_red_nrows_, d_red_N_, d_red_dst_off_;  // fixed-order row reduction
+    DevBuf d_Tm_, d_St_, d_Dd_, d_part_, d_dos_part_;
     bool timing_ = false;
     std::vector<hipEvent_t> ev_start_, ev_stop_;
     size_t ev_used_ = 0;

@@ -90,12 +90,14 @@ class Tube {
     bool stream_pending = false;
     std::vector<double> U_host;
     double Uc_host[2] = {0, 0};
-    DevBuf d_U, d_Uc, d_zero, d_rho0, d_eq, d_neq, d_Q;
+    // d_U: the N site potentials, then the two contact potentials (one upload)
+    double* d_Uc() const { return d_U.as<double>() + N; }
+    DevBuf d_U, d_zero, d_rho0, d_eq, d_neq, d_Q;
     // d_neq holds zeros (filled, and no non-equilibrium launch since)
     bool neq_zero = false;
-    DevBuf eq_chains, neq_chains, d_integ, dos_chains, dos_pairs;
+    DevBuf eq_chains, neq_chains, d_integ, dos_chains, dos_pairs, dos_site;
     HostBuf h_stage;
-    RgfPlan eq_plan, neq_plan;
+    RgfPlan eq_plan, neq_plan, dos_plan;
 
     // RGF tube descriptor of this tube; seg_len < 0: the tube's own setting
     RgfTube rgf_tube(const double* dU, const double* dUc, int nchain, int seg_len = -1) const;

@@ -31,6 +31,9 @@ using cplx = std::complex<double>;
 static constexpr double kPi = 3.14159265358979323846;
 static constexpr double kKbEvPerK = 8.617333262e-5;   // PhysConst::kb_eVperK
 
+// per-site spectral functions of a DOS call kept for the next one up to this size
+static constexpr size_t kKeepBytes = size_t(256) << 20;
+
 // ---------------------------------------------------------------- kernels
 __global__ void combine_charge_kernel(int N, const double* __restrict__ eq, const double* __restrict__ neq,
                                       const double* __restrict__ rho0, double* __restrict__ Q)
@@ -205,8 +208,8 @@ void add_path(Path& out, cplx a, cplx b, int n, int type)
 Tube::~Tube()
 {
     if (stream) (void)hipStreamSynchronize(stream);
-    DevBuf* bufs[] = {&d_U, &d_Uc, &d_zero, &d_rho0, &d_eq, &d_neq, &d_Q, &eq_chains, &neq_chains, &d_integ,
-                      &dos_chains, &dos_pairs};
+    DevBuf* bufs[] = {&d_U, &d_zero, &d_rho0, &d_eq, &d_neq, &d_Q, &eq_chains, &neq_chains, &d_integ,
+                      &dos_chains, &dos_pairs, &dos_site};
     for (DevBuf* b : bufs) b->release();
     for (HostBuf* b : {&h_stage}) b->release();
     if (stream) (void)hipStreamDestroy(stream);
@@ -278,15 +281,14 @@ int Tube::init(const negf_tube_params& prm)
 
     NEGF_HIP_TRY(hipStreamCreate(&stream));
     int rc;
-    if ((rc = d_U.ensure(sizeof(double) * N))) return rc;
-    if ((rc = d_Uc.ensure(sizeof(double) * 2))) return rc;
+    if ((rc = d_U.ensure(sizeof(double) * (N + 2)))) return rc;
+    if ((rc = h_stage.ensure(sizeof(double) * (N + 2)))) return rc;
     if ((rc = d_zero.ensure(sizeof(double) * std::max(N, 2)))) return rc;
     if ((rc = d_rho0.ensure(sizeof(double) * N))) return rc;
     if ((rc = d_eq.ensure(sizeof(double) * N))) return rc;
     if ((rc = d_neq.ensure(sizeof(double) * N))) return rc;
     if ((rc = d_Q.ensure(sizeof(double) * N))) return rc;
-    if ((rc = fill_device(d_U.as<double>(), N, 0.0, stream))) return rc;
-    if ((rc = fill_device(d_Uc.as<double>(), 2, 0.0, stream))) return rc;
+    if ((rc = fill_device(d_U.as<double>(), N + 2, 0.0, stream))) return rc;
     if ((rc = fill_device(d_zero.as<double>(), std::max(N, 2), 0.0, stream))) return rc;
     if ((rc = fill_device(d_neq.as<double>(), N, 0.0, stream))) return rc;
     neq_zero = true;
@@ -449,7 +451,7 @@ int Tube::build_noneq_plan()
     n_neq = (int)ch.size();
     neq_host = ch;
     if ((rc = d_integ.ensure(sizeof(double) * 3 * n_neq))) return rc;
-    std::vector<RgfTube> tubes{rgf_tube(d_U.as<double>(), d_Uc.as<double>(), n_neq)};
+    std::vector<RgfTube> tubes{rgf_tube(d_U.as<double>(), d_Uc(), n_neq)};
     return neq_plan.build(KIND_NONEQ, false, tubes, neq_chains.as<ChainDesc>(), n_neq, dec());
 }
 
@@ -550,7 +552,7 @@ int Tube::update_paths(bool correct)
     n_eq = (int)ch.size();
     eq_host = ch;
     ++paths_version;
-    std::vector<RgfTube> tubes{rgf_tube(d_U.as<double>(), d_Uc.as<double>(), n_eq)};
+    std::vector<RgfTube> tubes{rgf_tube(d_U.as<double>(), d_Uc(), n_eq)};
     if ((rc = eq_plan.build(KIND_EQ, false, tubes, eq_chains.as<ChainDesc>(), n_eq, dec()))) return rc;
     if (L.noneq) {
         if ((rc = build_noneq_plan())) return rc;
@@ -573,15 +575,18 @@ int Tube::set_potential_host(const double* U, const double Uc[2])
     Uc_host[0] = Uc[0];
     Uc_host[1] = Uc[1];
     NEGF_HIP_TRY(hipStreamSynchronize(stream));
-    NEGF_HIP_TRY(hipMemcpy(d_U.p, U, sizeof(double) * N, hipMemcpyHostToDevice));
-    NEGF_HIP_TRY(hipMemcpy(d_Uc.p, Uc, sizeof(double) * 2, hipMemcpyHostToDevice));
+    double* h = h_stage.as<double>();
+    std::copy(U, U + N, h);
+    h[N] = Uc[0];
+    h[N + 1] = Uc[1];
+    NEGF_HIP_TRY(hipMemcpy(d_U.p, h, sizeof(double) * (N + 2), hipMemcpyHostToDevice));
     return NEGF_OK;
 }
 
 int Tube::set_potential_device(const double* dU, hipStream_t st)
 {
     NEGF_HIP_TRY(hipMemcpyAsync(d_U.p, dU, sizeof(double) * N, hipMemcpyDeviceToDevice, st));
-    hipLaunchKernelGGL(end_sites_kernel, dim3(1), dim3(64), 0, st, N, d_U.as<double>(), d_Uc.as<double>());
+    hipLaunchKernelGGL(end_sites_kernel, dim3(1), dim3(64), 0, st, N, d_U.as<double>(), d_Uc());
     NEGF_HIP_TRY(hipGetLastError());
     return NEGF_OK;
 }
@@ -722,25 +727,25 @@ int Tube::dos_complex(int nE, const cplx* E, double* dos_out, double* trans_out,
     int rc;
     if ((rc = upload_chains(dos_chains, ch))) return rc;
     if ((rc = dos_pairs.ensure(sizeof(double) * 2 * ch.size()))) return rc;
-    DevBuf d_site;
-    if (ldos && (rc = d_site.ensure(sizeof(double) * ch.size() * (size_t)N))) return rc;
-    RgfPlan plan;
-    std::vector<RgfTube> tubes{rgf_tube(d_U.as<double>(), d_Uc.as<double>(), (int)ch.size())};
-    if ((rc = plan.build(KIND_DOS, false, tubes, dos_chains.as<ChainDesc>(), (int)ch.size(), dec()))) return rc;
-    if ((rc = plan.enqueue(nullptr, nullptr, dos_pairs.as<double>(), stream, nullptr,
-                           ldos ? d_site.as<double>() : nullptr)))
+    if (ldos && (rc = dos_site.ensure(sizeof(double) * ch.size() * (size_t)N))) return rc;
+    std::vector<RgfTube> tubes{rgf_tube(d_U.as<double>(), d_Uc(), (int)ch.size())};
+    if ((rc = dos_plan.build(KIND_DOS, false, tubes, dos_chains.as<ChainDesc>(), (int)ch.size(), dec()))) return rc;
+    if ((rc = dos_plan.enqueue(nullptr, nullptr, dos_pairs.as<double>(), stream, nullptr,
+                               ldos ? dos_site.as<double>() : nullptr)))
         return rc;
     std::vector<double> h(2 * ch.size());
     NEGF_HIP_TRY(hipMemcpyAsync(h.data(), dos_pairs.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, stream));
     if (ldos) {
         const long long n = (long long)nE * N;
         hipLaunchKernelGGL(ldos_modes_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, n, nm, n,
-                           dos_chains.as<ChainDesc>(), nE, d_site.as<double>());
+                           dos_chains.as<ChainDesc>(), nE, dos_site.as<double>());
         NEGF_HIP_TRY(hipGetLastError());
-        NEGF_HIP_TRY(hipMemcpyAsync(ldos, d_site.p, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, stream));
+        NEGF_HIP_TRY(hipMemcpyAsync(ldos, dos_site.p, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, stream));
     }
     int status = 0;
-    if ((rc = plan.check_status(stream, &status))) return rc;
+    rc = dos_plan.check_status(stream, &status);
+    if (dos_site.cap > kKeepBytes) dos_site.release();
+    if (rc) return rc;
     root_flag |= status & 1;
     for (int e = 0; e < nE; ++e) {
         double tr = 0.0, tt = 0.0;
@@ -796,14 +801,13 @@ int Tube::current(double I[2])
     if (!L.noneq || n_neq == 0) return NEGF_OK;
     int rc;
     if ((rc = dos_pairs.ensure(sizeof(double) * 2 * (size_t)n_neq))) return rc;
-    RgfPlan plan;
-    std::vector<RgfTube> tubes{rgf_tube(d_U.as<double>(), d_Uc.as<double>(), n_neq)};
-    if ((rc = plan.build(KIND_DOS, false, tubes, neq_chains.as<ChainDesc>(), n_neq, dec()))) return rc;
-    if ((rc = plan.enqueue(nullptr, nullptr, dos_pairs.as<double>(), stream))) return rc;
+    std::vector<RgfTube> tubes{rgf_tube(d_U.as<double>(), d_Uc(), n_neq)};
+    if ((rc = dos_plan.build(KIND_DOS, false, tubes, neq_chains.as<ChainDesc>(), n_neq, dec()))) return rc;
+    if ((rc = dos_plan.enqueue(nullptr, nullptr, dos_pairs.as<double>(), stream))) return rc;
     std::vector<double> h(2 * (size_t)n_neq);
     NEGF_HIP_TRY(hipMemcpyAsync(h.data(), dos_pairs.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, stream));
     int status = 0;
-    if ((rc = plan.check_status(stream, &status))) return rc;
+    if ((rc = dos_plan.check_status(stream, &status))) return rc;
     root_flag |= status & 1;
     const double q_e = 1.602176634e-19, h_eVperHz = 4.135667696e-15;   // PhysConst
     const double cm = spin_degen * q_e / h_eVperHz;

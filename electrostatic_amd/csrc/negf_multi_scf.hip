@@ -355,7 +355,7 @@ class MultiScf {
             }
             Nmax = std::max(Nmax, tu.N);
             hU[t] = tu.d_U.as<double>();
-            hUc[t] = tu.d_Uc.as<double>();
+            hUc[t] = tu.d_Uc();
             const int C = (tu.N + MS_TILE - 1) / MS_TILE;
             for (int r = 0; r < tu.N; r += MS_ROWS)
                 for (int c = 0; c < C; ++c)

@@ -626,7 +626,7 @@ class BatchScf {
                 return NEGF_EARG;
             }
             hU.push_back(tubes[t]->t.d_U.as<double>());
-            hUc.push_back(tubes[t]->t.d_Uc.as<double>());
+            hUc.push_back(tubes[t]->t.d_Uc());
         }
         coulomb_kernel(tubes[0]->t.ptd, p, K);
         M = p.Broyden_threshold_maxstep;
@@ -1094,7 +1094,7 @@ static void scf_enqueue_potential(Scf& s, hipStream_t q)
     Tube& t = *s.tube;
     hipLaunchKernelGGL(scf_potential_kernel, dim3((t.N + 3) / 4), dim3(256), 0, q, t.N, s.d_K.as<double>(),
                        s.br.dev().n_in, s.has_ext ? s.d_Uext.as<double>() : nullptr, s.d_V.as<double>(),
-                       s.d_U.as<double>(), t.d_U.as<double>(), t.d_Uc.as<double>());
+                       s.d_U.as<double>(), t.d_U.as<double>(), t.d_Uc());
 }
 
 // With part: the tube's equilibrium charge from the plan's partial rows
