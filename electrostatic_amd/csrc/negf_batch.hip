@@ -141,7 +141,7 @@ class Batch {
     // runs on its own stream (forked from st and joined back before the
     // combine, a form that stream capture records too), so the latency-bound
     // walks of one overlap the other's sweeps.
-    int enqueue_on(double* dQ, hipStream_t st, const int* tube_active = nullptr)
+    int enqueue_on(double* dQ, hipStream_t st, const int* tube_active = nullptr, bool combine = true)
     {
         int rc;
         if (n_neq > 0) {
@@ -150,8 +150,9 @@ class Batch {
             if ((rc = neq_plan.enqueue(d_neq.as<double>(), nullptr, nullptr, stream_neq, tube_active))) return rc;
             NEGF_HIP_TRY(hipEventRecord(ev_join, stream_neq));
         }
-        if ((rc = eq_plan.enqueue(d_eq.as<double>(), nullptr, nullptr, st, tube_active))) return rc;
+        if ((rc = eq_plan.enqueue(d_eq.as<double>(), nullptr, nullptr, st, tube_active, nullptr, combine))) return rc;
         if (n_neq > 0) NEGF_HIP_TRY(hipStreamWaitEvent(st, ev_join, 0));
+        if (!combine) return NEGF_OK;
         const long long Nt = off.back();
         hipLaunchKernelGGL(batch_combine_kernel, dim3((unsigned)((Nt + 255) / 256)), dim3(256), 0, st, Nt,
                            d_eq.as<double>(), d_neq.as<double>(), d_rho0.as<double>(), dQ);
@@ -406,9 +407,17 @@ struct negf_batch {
 
 namespace negf {
 int batch_prepare(negf_batch* b, int iter, bool* rebuilt) { return b->b.prepare(iter, rebuilt); }
-int batch_enqueue(negf_batch* b, double* dQ, hipStream_t st, const int* tube_active)
+int batch_enqueue(negf_batch* b, double* dQ, hipStream_t st, const int* tube_active, bool combine)
 {
-    return b->b.enqueue_on(dQ, st, tube_active);
+    return b->b.enqueue_on(dQ, st, tube_active, combine);
+}
+bool batch_rows(const negf_batch* b, BatchRows* r)
+{
+    const Batch& x = b->b;
+    r->eq = x.d_eq.as<double>();
+    r->neq = x.d_neq.as<double>();
+    r->rho0 = x.d_rho0.as<double>();
+    return x.eq_plan.rows(&r->part, &r->off, &r->nrows);
 }
 long long batch_generation(const negf_batch* b) { return b->b.generation; }
 int batch_poll_status(negf_batch* b) { return b->b.poll_status(); }

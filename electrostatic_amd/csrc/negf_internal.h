@@ -99,6 +99,16 @@ class RgfPlan {
         *nrows = max_rows_;
         return true;
     }
+    // The partial rows of all tubes, in the order of build()'s list, for a caller
+    // that sums them itself; false unless every tube has at most 16.
+    bool rows(const double** part, const long long** off, const int** nrows) const
+    {
+        if (kind_ == KIND_DOS || max_rows_ > 16) return false;
+        *part = d_part_.as<const double>();
+        *off = d_red_src_off_;
+        *nrows = d_red_nrows_;
+        return true;
+    }
     // Read and clear the device status word (synchronises the stream).
     int check_status(hipStream_t st, int* status);
     // The device status word itself (an int), for a copy enqueued by the caller.
@@ -152,7 +162,22 @@ int lone_tube_segment_length(int N);
 // solve (rebuilding plans when paths changed) and the bare launch sequence
 // on a given stream (capturable).
 int batch_prepare(negf_batch* b, int iter, bool* rebuilt);
-int batch_enqueue(negf_batch* b, double* dQ, hipStream_t st, const int* tube_active = nullptr);
+// combine = false leaves out the last two steps, the equilibrium plan's row sum
+// into BatchRows::eq and Q = (eq + noneq) - rho0, for a caller that fuses both into
+// its next kernel (batch_rows says whether it may); dQ is then unused.
+int batch_enqueue(negf_batch* b, double* dQ, hipStream_t st, const int* tube_active = nullptr, bool combine = true);
+// The partial rows of the batch's equilibrium plan: tube t's row r of site n at
+// part[off[t] + r N_t + n], r < nrows[t], summed in order from 0.0; false where a
+// tube has more than 16 (the plan's row sum then adds in another order).  Valid until
+// the next rebuild.  The batch's tubes lie one after the other in eq, neq and rho0.
+struct BatchRows {
+    const double* part;
+    const long long* off;
+    const int* nrows;
+    double* eq;
+    const double *neq, *rho0;
+};
+bool batch_rows(const negf_batch* b, BatchRows* r);
 // Build counter of the batch's plans: a graph captured over batch_enqueue
 // is valid only while this value is unchanged.
 long long batch_generation(const negf_batch* b);

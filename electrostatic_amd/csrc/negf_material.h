@@ -47,7 +47,8 @@ class Tube {
     // two steps, the equilibrium plan's row sum into d_eq (eq_rows) and
     // Q = (eq + noneq) - rho0 (d_eq, d_neq, d_rho0), for a caller that fuses
     // both into its next kernel; dQ is then unused.
-    int enqueue_solve(double* dQ, hipStream_t st, bool combine = true);
+    // With active (a device flag), the launches do nothing while it is 0.
+    int enqueue_solve(double* dQ, hipStream_t st, bool combine = true, const int* active = nullptr);
     bool eq_rows(const double** part, int* nrows) const { return eq_plan.single_tube_rows(part, nrows); }
     // Device status words of the plans enqueue_solve() launches (nullptr for
     // a plan it does not launch); nonzero after a launch: check_status().

@@ -639,14 +639,14 @@ int Tube::solve(int iter, double* dQ, hipStream_t st)
     return NEGF_OK;
 }
 
-int Tube::enqueue_solve(double* dQ, hipStream_t st, bool combine)
+int Tube::enqueue_solve(double* dQ, hipStream_t st, bool combine, const int* active)
 {
     int rc;
-    if ((rc = eq_plan.enqueue(d_eq.as<double>(), nullptr, nullptr, st, nullptr, nullptr, combine))) return rc;
+    if ((rc = eq_plan.enqueue(d_eq.as<double>(), nullptr, nullptr, st, active, nullptr, combine))) return rc;
     const bool have_neq = L.noneq && n_neq > 0;
     if (have_neq) {
         neq_zero = false;
-        if ((rc = neq_plan.enqueue(d_neq.as<double>(), nullptr, nullptr, st))) return rc;
+        if ((rc = neq_plan.enqueue(d_neq.as<double>(), nullptr, nullptr, st, active))) return rc;
     } else if (!neq_zero) {
         // zeros once after the last non-equilibrium solve (the charge
         // components read them)

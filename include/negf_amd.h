@@ -341,10 +341,11 @@ int negf_scf_bias_point(negf_scf *s, double V_gate, double *U_out,
 int negf_scf_set_external_potential(negf_scf *s, const double *U_ext);
 /* Dense kernel K (N x N, row-major, V per e) used by the stand-in. */
 int negf_scf_kernel(const negf_scf *s, double *K);
-/* No reference counterpart (performance only): on (the default), each
- * iteration of negf_scf_bias_point replays one captured hipGraph (potential,
- * solve, Broyden update, read-back), recaptured when the tube's paths
- * change; off, the same launches are enqueued one by one.  Results are the
+/* No reference counterpart (performance only): on (the default), the
+ * iterations of negf_scf_bias_point (potential, solve, Broyden update with
+ * read-back) are launched one ahead of the host's convergence test, so the
+ * GPU does not wait for the host; off, the host waits for each one.  (The
+ * name is older: replays of a captured graph are slower.)  Results are the
  * same bit for bit. */
 int negf_scf_use_graph(negf_scf *s, int on);
 
@@ -353,7 +354,8 @@ int negf_scf_use_graph(negf_scf *s, int on);
  * electrostatic kernel K (N x N, as negf_scf); each tube t has its own
  * external potential U_ext[t], metal voltage V_gate[t] and Broyden history.
  * An iteration is one FP64 GEMM for all tubes, one batched NEGF solve and one
- * Broyden workgroup per tube, replayed from a captured hipGraph; a tube stops
+ * Broyden workgroup per tube, launched one iteration ahead of the host's
+ * convergence test (negf_batch_scf_use_graph off: not ahead); a tube stops
  * iterating once its Broyden_Norm <= Broyden_max_norm.  Arrays are host,
  * tube-major ([T][N]). */
 typedef struct negf_batch_scf negf_batch_scf;
