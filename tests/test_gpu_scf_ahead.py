@@ -77,3 +77,16 @@ def test_batch(T, cells, eq_pts, steps):
             t.close()
     assert (steps == 8) == isinstance(runs[0][0], str)
     same(*runs)
+
+
+@pytest.mark.parametrize("T,cells", [(1, 1), (2, 16), (5, 33)])
+def test_input_charge_round_trip(T, cells):
+    tubes = tubes_of(T, cells)
+    batch = negf.Batch(tubes)
+    scf = negf.BatchScf(batch, Broyden_max_norm=1e-6, Broyden_threshold_maxstep=20, **SP)
+    n = np.random.default_rng(T).normal(size=(T, tubes[0].N))
+    for k in (1.0, -2.0):
+        scf.set_input_charge(k * n)
+        assert np.array_equal(scf.get_input_charge(), k * n)
+    scf.close()
+    batch.close()
