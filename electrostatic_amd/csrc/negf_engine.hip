@@ -144,27 +144,38 @@ int RgfPlan::kernel_time(double* total_ms, int* launches)
     return NEGF_OK;
 }
 
-// Tubes of FUSED_MIN_SEGS..FUSED_SEGS segments take the fused transfer and
-// scan launch (NEGF_RGF_FUSED=0 in the environment turns it off, which leaves
-// the results the same up to rounding).
-static int fused_for(int P)
+// Tubes of FUSED_MIN_SEGS..FUSED_SEGS segments, and in a launch of few chain groups
+// those of fewer too, take the fused transfer and scan launch (NEGF_RGF_FUSED=0 in the
+// environment turns it off, which leaves the results the same up to rounding).  With
+// fewer segments a part of the fused launch's wavefronts is idle, which costs nothing
+// while its workgroups (two per group) do not wait for each other.
+static int fused_for(int P, int groups)
 {
     const char* e = std::getenv("NEGF_RGF_FUSED");
     if (e && e[0] == '0') return 0;
-    return P >= FUSED_MIN_SEGS && P <= FUSED_SEGS ? 1 : 0;
+    return P <= FUSED_SEGS && (P >= FUSED_MIN_SEGS || groups <= RGF_FEW_GROUPS) ? 1 : 0;
+}
+
+// Segment length of a tube of N sites when none is asked for.  A launch of few 64-chain
+// groups is short of wavefronts and as long as one segment takes: the shortest
+// multiple of NEGF_SUB_K that keeps the tube within the fused launch's segments, where
+// the default length would give fewer than it takes.  0 (the default) otherwise.
+// Measured, equilibrium charge with host part, short against default length: 64 to 4096
+// energies (1 to 64 groups) 46 .. 76 us against 49 .. 80 us at 40 to 1501 sites, diag G
+// of 1501 x 777 69 against 84 us; 96 groups (32 tubes of 1024, 600, 256 sites) 58.7,
+// 52.1, 40.4 against 62.2, 54.6, 50.5 us an SCF iteration; 128 groups (8192 energies)
+// 88 against 81 us at 1000 sites, 95 against 87 us at 1501.
+static int segment_length_for(int N, int groups)
+{
+    if (groups > RGF_FEW_GROUPS) return 0;
+    if ((N + NEGF_SEG_DEFAULT - 1) / NEGF_SEG_DEFAULT >= FUSED_MIN_SEGS) return 0;
+    const int L = (N + FUSED_SEGS - 1) / FUSED_SEGS;
+    return (L + NEGF_SUB_K - 1) / NEGF_SUB_K * NEGF_SUB_K;
 }
 
 // Kernel-side descriptor of one tube whose items start at item0 and whose
 // partial rows start at part_off.
-int lone_tube_segment_length(int N)
-{
-    if ((N + NEGF_SEG_DEFAULT - 1) / NEGF_SEG_DEFAULT >= FUSED_MIN_SEGS) return 0;
-    const int L = (N + FUSED_SEGS - 1) / FUSED_SEGS;
-    const int Lk = (L + NEGF_SUB_K - 1) / NEGF_SUB_K * NEGF_SUB_K;
-    return (N + Lk - 1) / Lk >= FUSED_MIN_SEGS ? Lk : 0;
-}
-
-static WTube make_wtube(const RgfTube& tb, int P, int L, int item0, long long part_off)
+static WTube make_wtube(const RgfTube& tb, int P, int L, int item0, long long part_off, int groups)
 {
     WTube w;
     std::memset(&w, 0, sizeof(w));
@@ -183,7 +194,7 @@ static WTube make_wtube(const RgfTube& tb, int P, int L, int item0, long long pa
     w.part_off = part_off;
     for (int q = 0; q < 3; ++q) w.sample[q] = tb.sample[q];
     w.ext = tb.ext;
-    w.fused = fused_for(P);
+    w.fused = fused_for(P, groups);
     return w;
 }
 
@@ -226,6 +237,8 @@ int RgfPlan::build(int kind, bool write_G, const std::vector<RgfTube>& tubes, Ch
     max_P_ = 0;
     max_groups_ = 0;
     any_fused_ = any_fused2_ = any_unfused_ = false;
+    int groups = 0;  // 64-chain groups of the launch
+    for (const RgfTube& tb : tubes) groups += (std::max(tb.nchain, 0) + 63) / 64;
     for (int t = 0; t < ntubes_; ++t) {
         const RgfTube& tb = tubes[t];
         if (tb.N < 2 || !tb.dU || tb.nchain <= 0 || tb.t_odd <= 0 || tb.chain0 < 0 ||
@@ -235,14 +248,15 @@ int RgfPlan::build(int kind, bool write_G, const std::vector<RgfTube>& tubes, Ch
             return NEGF_EARG;
         }
         int P, L;
-        if (!choose_segments(tb.N, tb.L, &P, &L)) {
+        if (!choose_segments(tb.N, tb.L > 0 ? tb.L : segment_length_for(tb.N, groups), &P, &L)) {
             set_error("chain of %d sites exceeds the supported maximum %d", tb.N, max_sites());
             return NEGF_ENOTSUP;
         }
         WTube& w = wt[t];
-        w = make_wtube(tb, P, L, items, poff);
+        w = make_wtube(tb, P, L, items, poff, groups);
         // equilibrium charge on full 128-site segments: the whole launch fused
-        if (w.fused && kind == KIND_EQ && !write_G && L == NEGF_SEG_MAX && tb.N % L == 0) w.fused = 2;
+        if (w.fused && P >= FUSED_MIN_SEGS && kind == KIND_EQ && !write_G && L == NEGF_SEG_MAX && tb.N % L == 0)
+            w.fused = 2;
         (w.fused == 2 ? any_fused2_ : w.fused ? any_fused_ : any_unfused_) = true;
         const int G = (tb.nchain + 63) / 64;
         const int rows = w.fused == 2 ? 2 * G : G;  // partial rows: one per 32 chains when fused
@@ -817,15 +831,15 @@ int negf_rgf_diag_accumulate_noalloc(const negf_chain_params* p, const double* d
         return NEGF_EARG;
     }
     int P, L;
-    if (!choose_segments(p->N, p->segment_length, &P, &L)) {
+    const size_t N = (size_t)p->N, E = (size_t)nE, G = (E + 63) / 64;
+    if (!choose_segments(p->N, p->segment_length > 0 ? p->segment_length : segment_length_for(p->N, (int)G), &P, &L)) {
         set_error("chain of %d sites exceeds the supported maximum %d", p->N, max_sites());
         return NEGF_ENOTSUP;
     }
-    const size_t N = (size_t)p->N, E = (size_t)nE;
-    const size_t G = (E + 63) / 64, items = G * (size_t)P;
+    const size_t items = G * (size_t)P;
     // the same launch forms as RgfPlan::build
-    WTube tb = make_wtube(one_tube(p, d_U, nE), P, L, 0, 0);
-    if (tb.fused && !d_diagG && L == NEGF_SEG_MAX && p->N % L == 0) tb.fused = 2;
+    WTube tb = make_wtube(one_tube(p, d_U, nE), P, L, 0, 0, (int)G);
+    if (tb.fused && P >= FUSED_MIN_SEGS && !d_diagG && L == NEGF_SEG_MAX && p->N % L == 0) tb.fused = 2;
     const size_t rows = tb.fused == 2 ? 2 * G : G;
     size_t off = 0;
     auto take = [&off](size_t bytes) {

@@ -64,7 +64,7 @@ struct RgfTube {
     const double* dUc = nullptr;  // or: device contact potentials (2 values)
     double t_odd = 0;             // gamma
     int sample[3] = {-1, -1, -1}; // integrand sample sites (KIND_NONEQ)
-    int L = 0;                    // requested segment length (0: default)
+    int L = 0;                    // requested segment length (0: chosen by the plan)
     int chain0 = 0, nchain = 0;   // chains [chain0, chain0+nchain) of d_chains
     long long out_off = 0;        // offset of this tube's N outputs in d_out
     int ext = 0;                  // index of the tube for an active mask
@@ -151,12 +151,6 @@ void gl_path(double ar, double ai, double br, double bi, int n, int type, double
 // Segmentation of a chain of N sites into P segments of L sites (L a
 // multiple of NEGF_SUB_K, at most NEGF_SEG_MAX); 0 if N is too long.
 int choose_segments(int N, int L_req, int* P, int* L);
-// Segment length for a lone tube when none is asked for: a lone tube has one
-// chain per energy, a few chain groups, so its launch is short of wavefronts;
-// where 128-site segments would give fewer segments than the fused transfer
-// and walk launch takes, the shortest multiple of NEGF_SUB_K that keeps the
-// count within that launch's range.  0 (the default) otherwise.
-int lone_tube_segment_length(int N);
 
 // Batched solve internals shared with the batched SCF: the host part of a
 // solve (rebuilding plans when paths changed) and the bare launch sequence

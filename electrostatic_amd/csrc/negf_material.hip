@@ -313,7 +313,7 @@ RgfTube Tube::rgf_tube(const double* dU, const double* dUc, int nchain, int seg_
     tb.chain0 = 0;
     tb.nchain = nchain;
     tb.out_off = 0;
-    tb.L = seg_len >= 0 ? seg_len : p.segment_length > 0 ? p.segment_length : lone_tube_segment_length(N);
+    tb.L = seg_len >= 0 ? seg_len : p.segment_length;
     // else-if order of the reference (NEGF_Common.cpp:3469-3495)
     tb.sample[0] = N / 2;
     tb.sample[1] = N / 4;

@@ -808,6 +808,7 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void scan_kernel(WLaunch lp, int n
 #define FUSED_WAVES 16
 #define FUSED_SEGS (2 * FUSED_WAVES)
 #define FUSED_MIN_SEGS 17
+#define RGF_FEW_GROUPS 96  // chain groups of a launch that counts as short of wavefronts
 
 
 // One walk over the segment matrices in LDS (V: the v walk), by the 32 lanes
