@@ -120,6 +120,15 @@ static void launch_sweep_full(int ns, int kind, const WLaunch& lp, hipStream_t s
     }
 }
 
+template <int NS>
+static void launch_sweep_pair(int ns, const WLaunch2& a, hipStream_t st)
+{
+    if constexpr (NS > 1) {
+        if (ns < NS) return launch_sweep_pair<NS - 1>(ns, a, st);
+    }
+    hipLaunchKernelGGL((sweep_pair_kernel<NEGF_SUB_K, NS>), dim3(a.n[0] + a.n[1]), dim3(256), 0, st, a);
+}
+
 // ---------------------------------------------------------------- plan
 RgfPlan::~RgfPlan()
 {
@@ -491,26 +500,9 @@ static int launch_rgf_finish(const RgfLayout& y, const WLaunch& lp, double* d_ou
     return NEGF_OK;
 }
 
-int RgfPlan::enqueue(double* d_out, double2* d_diagG, double* d_chain_out, hipStream_t st, const int* tube_active,
-                     double* d_site_out, bool finish)
+void RgfPlan::layout(RgfLayout* out) const
 {
-    if (nitems_ == 0) {
-        set_error("RgfPlan::enqueue: plan not built");
-        return NEGF_EARG;
-    }
-    if (write_G_ && !d_diagG) {
-        set_error("diag G output requested without a buffer");
-        return NEGF_EARG;
-    }
-    if (kind_ == KIND_DOS && !d_chain_out) {
-        set_error("DOS output buffer missing");
-        return NEGF_EARG;
-    }
-    if (kind_ != KIND_DOS && !d_out) {
-        set_error("output buffer missing");
-        return NEGF_EARG;
-    }
-    RgfLayout y;
+    RgfLayout& y = *out;
     y.kind = kind_;
     y.write_G = write_G_;
     y.nitems = nitems_;
@@ -547,6 +539,76 @@ int RgfPlan::enqueue(double* d_out, double2* d_diagG, double* d_chain_out, hipSt
     y.any_fused2 = any_fused2_;
     y.any_unfused = any_unfused_;
     if (ntubes_ == 1 && tube0_.size() == sizeof(WTube)) y.tube1 = reinterpret_cast<const WTube*>(tube0_.data());
+}
+
+// A plan that enqueue_pair takes: one tube, transfer and scan in the fused launch, all
+// full segments of one length and the partial one beside them.
+bool RgfPlan::pairs() const
+{
+    int full = 0;
+    for (int ns = 1; ns <= NEGF_SUB_NS; ++ns) full += fast_n_[ns] > 0;
+    return ntubes_ == 1 && any_fused_ && !any_fused2_ && !any_unfused_ && !dec_.use && !timing_ && full == 1;
+}
+
+int RgfPlan::enqueue_pair(const RgfPlan& eq, const RgfPlan& neq, hipStream_t st, const int* tube_active, bool* done)
+{
+    *done = false;
+    if (eq.kind_ != KIND_EQ || eq.write_G_ || neq.kind_ != KIND_NONEQ || !eq.pairs() || !neq.pairs()) return NEGF_OK;
+    int ns = 1;
+    while (eq.fast_n_[ns] == 0) ++ns;
+    const RgfPlan* pl[2] = {&eq, &neq};
+    int waves = 0;
+    for (const RgfPlan* p : pl) waves += p->nitems_;
+    // more items than two wavefronts per SIMD are better off at three (short segments)
+    if (neq.fast_n_[ns] == 0 || (ns <= 4 && waves > SWEEP_TAIL_WAVES)) return NEGF_OK;
+    WLaunch2 ts, sw;
+    for (int k = 0; k < 2; ++k) {
+        RgfLayout y;
+        pl[k]->layout(&y);
+        ts.lp[k] = sw.lp[k] = launch_params(y, nullptr, nullptr, tube_active);
+        ts.n[k] = y.nsblk;
+        WLaunch& l = sw.lp[k];
+        l.item_list = y.item_list + y.fast_off[ns];
+        l.nlist = y.fast_n[ns];
+        l.tail_list = y.item_list + y.slow_off;
+        l.ntail = y.slow_n;
+        sw.n[k] = (l.nlist + l.ntail + 3) / 4;
+    }
+    hipLaunchKernelGGL(transfer_scan_pair_kernel, dim3(2 * (ts.n[0] + ts.n[1])), dim3(64 * FUSED_WAVES), 0, st, ts);
+    launch_sweep_pair<NEGF_SUB_NS>(ns, sw, st);
+    NEGF_HIP_TRY(hipGetLastError());
+    *done = true;
+    return NEGF_OK;
+}
+
+int RgfPlan::sum_rows(double* d_out, hipStream_t st, const int* tube_active)
+{
+    RgfLayout y;
+    layout(&y);
+    return launch_rgf_finish(y, launch_params(y, nullptr, nullptr, tube_active), d_out, st, tube_active);
+}
+
+int RgfPlan::enqueue(double* d_out, double2* d_diagG, double* d_chain_out, hipStream_t st, const int* tube_active,
+                     double* d_site_out, bool finish)
+{
+    if (nitems_ == 0) {
+        set_error("RgfPlan::enqueue: plan not built");
+        return NEGF_EARG;
+    }
+    if (write_G_ && !d_diagG) {
+        set_error("diag G output requested without a buffer");
+        return NEGF_EARG;
+    }
+    if (kind_ == KIND_DOS && !d_chain_out) {
+        set_error("DOS output buffer missing");
+        return NEGF_EARG;
+    }
+    if (kind_ != KIND_DOS && !d_out) {
+        set_error("output buffer missing");
+        return NEGF_EARG;
+    }
+    RgfLayout y;
+    layout(&y);
     if (kind_ == KIND_NONEQ && d_chain_out) {
         // integrand samples: only the general sweep writes them.  The fast and the
         // general items are one list.

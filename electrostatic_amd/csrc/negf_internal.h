@@ -90,6 +90,13 @@ class RgfPlan {
     // into its next kernel (single_tube_rows).
     int enqueue(double* d_out, double2* d_diagG, double* d_chain_out, hipStream_t st,
                 const int* tube_active = nullptr, double* d_site_out = nullptr, bool finish = true);
+    // The transfer, scan and sweep of a tube's equilibrium and non-equilibrium plan up to
+    // their partial rows, as two launches for both; *done = false and nothing enqueued
+    // where the plans don't allow it.
+    static int enqueue_pair(const RgfPlan& eq, const RgfPlan& neq, hipStream_t st, const int* tube_active,
+                            bool* done);
+    // The last step of enqueue alone: the partial rows of a charge plan into d_out.
+    int sum_rows(double* d_out, hipStream_t st, const int* tube_active);
     // A one-tube plan's partial rows: row r of site n at part[r N + n], r <
     // nrows, summed in order r = 0, 1, ... from 0.0; false for other plans.
     bool single_tube_rows(const double** part, int* nrows) const
@@ -119,6 +126,8 @@ class RgfPlan {
     int kernel_time(double* total_ms, int* launches);
 
    private:
+    void layout(struct RgfLayout* y) const;
+    bool pairs() const;
     int kind_ = 0;
     bool write_G_ = false;
     int nitems_ = 0, nchains_ = 0, ntubes_ = 0, nsblk_ = 0;

@@ -41,14 +41,16 @@ class Tube {
     // Host part of a solve: limits and paths (plans rebuilt if needed).
     int prepare(int iter);
     // Enqueue one solve; Q (device, N) is ready on stream st when it returns.
-    int solve(int iter, double* dQ, hipStream_t st);
+    // With Q_host (st must be the tube's stream) it waits and gives the charge there too.
+    int solve(int iter, double* dQ, hipStream_t st, double* Q_host = nullptr);
     // The launches of a solve whose prepare() has run, all on stream st and
     // nothing on the host (capturable).  combine = false leaves out the last
     // two steps, the equilibrium plan's row sum into d_eq (eq_rows) and
     // Q = (eq + noneq) - rho0 (d_eq, d_neq, d_rho0), for a caller that fuses
     // both into its next kernel; dQ is then unused.
     // With active (a device flag), the launches do nothing while it is 0.
-    int enqueue_solve(double* dQ, hipStream_t st, bool combine = true, const int* active = nullptr);
+    int enqueue_solve(double* dQ, hipStream_t st, bool combine = true, const int* active = nullptr,
+                      bool to_host = false);
     bool eq_rows(const double** part, int* nrows) const { return eq_plan.single_tube_rows(part, nrows); }
     // Device status words of the plans enqueue_solve() launches (nullptr for
     // a plan it does not launch); nonzero after a launch: check_status().
@@ -98,6 +100,8 @@ class Tube {
     bool neq_zero = false;
     DevBuf eq_chains, neq_chains, d_integ, dos_chains, dos_pairs, dos_site;
     HostBuf h_stage;
+    HostBuf h_charge;             // charge and two status words of the last solve with Q_host
+    bool charge_on_host = false;  // that solve wrote them
     RgfPlan eq_plan, neq_plan, dos_plan;
 
     // RGF tube descriptor of this tube; seg_len < 0: the tube's own setting
@@ -106,6 +110,7 @@ class Tube {
     DecParams dec() const;
 
    private:
+    int take_charge(double* Q, const double* dQ);
     int upload_chains(DevBuf& buf, const std::vector<ChainDesc>& ch);
     void eq_chains_of(const Path& path, double cm, bool with_fermi, std::vector<ChainDesc>& out) const;
     int compute_rho0();

@@ -35,6 +35,45 @@ static constexpr double kKbEvPerK = 8.617333262e-5;   // PhysConst::kb_eVperK
 static constexpr size_t kKeepBytes = size_t(256) << 20;
 
 // ---------------------------------------------------------------- kernels
+// The charge of one tube from its plans' partial rows (row r of site n at part[r N + n]),
+// each sum in row order from 0.0 as the plans' own row sums of at most 16 rows are:
+// eq, neq (with neq_part) and Q = (eq + neq) - rho0.  With hQ, Q and the plans' status
+// words go to pinned host memory as well, so the caller waits once instead of for
+// a copy of each.  One launch instead of three; 4012 sites, 3 + 4 rows: 4.1 us against
+// 3.0 + 4.4 + 4.0 us, and 20 to 40 us less of copies and waits.
+__global__ __launch_bounds__(64) void tube_charge_kernel(int N, const double* __restrict__ eq_part, int eq_rows,
+                                                         const double* __restrict__ neq_part, int neq_rows,
+                                                         const double* __restrict__ rho0, double* __restrict__ eq,
+                                                         double* __restrict__ neq, double* __restrict__ Q,
+                                                         double* __restrict__ hQ, const int* __restrict__ st_eq,
+                                                         const int* __restrict__ st_neq, int* __restrict__ h_status)
+{
+    const int n = blockIdx.x * 64 + threadIdx.x;
+    if (n == 0 && h_status) {
+        h_status[0] = *st_eq;
+        h_status[1] = neq_part ? *st_neq : 0;
+    }
+    if (n >= N) return;
+    double v[16], w[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {  // the loads in flight together
+        v[r] = r < eq_rows ? eq_part[(size_t)r * N + n] : 0.0;
+        w[r] = r < neq_rows ? neq_part[(size_t)r * N + n] : 0.0;
+    }
+    const double r0 = rho0[n];
+    double e = 0.0, q = 0.0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        if (r < eq_rows) e += v[r];
+        if (r < neq_rows) q += w[r];
+    }
+    eq[n] = e;
+    if (neq_part) neq[n] = q;
+    const double c = (e + q) - r0;
+    Q[n] = c;
+    if (hQ) hQ[n] = c;
+}
+
 __global__ void combine_charge_kernel(int N, const double* __restrict__ eq, const double* __restrict__ neq,
                                       const double* __restrict__ rho0, double* __restrict__ Q)
 {
@@ -211,7 +250,7 @@ Tube::~Tube()
     DevBuf* bufs[] = {&d_U, &d_zero, &d_rho0, &d_eq, &d_neq, &d_Q, &eq_chains, &neq_chains, &d_integ,
                       &dos_chains, &dos_pairs, &dos_site};
     for (DevBuf* b : bufs) b->release();
-    for (HostBuf* b : {&h_stage}) b->release();
+    for (HostBuf* b : {&h_stage, &h_charge}) b->release();
     if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -283,6 +322,7 @@ int Tube::init(const negf_tube_params& prm)
     int rc;
     if ((rc = d_U.ensure(sizeof(double) * (N + 2)))) return rc;
     if ((rc = h_stage.ensure(sizeof(double) * (N + 2)))) return rc;
+    if ((rc = h_charge.ensure(sizeof(double) * (N + 1)))) return rc;
     if ((rc = d_zero.ensure(sizeof(double) * std::max(N, 2)))) return rc;
     if ((rc = d_rho0.ensure(sizeof(double) * N))) return rc;
     if ((rc = d_eq.ensure(sizeof(double) * N))) return rc;
@@ -615,7 +655,7 @@ int Tube::prepare(int iter)
     return NEGF_OK;
 }
 
-int Tube::solve(int iter, double* dQ, hipStream_t st)
+int Tube::solve(int iter, double* dQ, hipStream_t st, double* Q_host)
 {
     int rc;
     if (st != stream) {
@@ -627,8 +667,9 @@ int Tube::solve(int iter, double* dQ, hipStream_t st)
         NEGF_HIP_TRY(hipEventDestroy(ev));
     }
     if ((rc = prepare(iter))) return rc;
-    if ((rc = enqueue_solve(dQ, stream))) return rc;
+    if ((rc = enqueue_solve(dQ, stream, true, nullptr, Q_host != nullptr))) return rc;
     stream_pending = true;
+    if (Q_host) return take_charge(Q_host, dQ);
     if (st != stream) {
         hipEvent_t ev;
         NEGF_HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -639,14 +680,29 @@ int Tube::solve(int iter, double* dQ, hipStream_t st)
     return NEGF_OK;
 }
 
-int Tube::enqueue_solve(double* dQ, hipStream_t st, bool combine, const int* active)
+int Tube::enqueue_solve(double* dQ, hipStream_t st, bool combine, const int* active, bool to_host)
 {
     int rc;
-    if ((rc = eq_plan.enqueue(d_eq.as<double>(), nullptr, nullptr, st, active, nullptr, combine))) return rc;
     const bool have_neq = L.noneq && n_neq > 0;
+    const double *ep = nullptr, *np_ = nullptr;
+    int er = 0, nr = 0;
+    // the row sums and the charge are one kernel where the plans' own row sums are the
+    // in-order ones (at most 16 rows)
+    const bool rows = combine && eq_plan.single_tube_rows(&ep, &er) && er <= 16 &&
+                      (!have_neq || (neq_plan.single_tube_rows(&np_, &nr) && nr <= 16));
+    charge_on_host = rows && to_host;
+    bool paired = false;
+    if (have_neq && (rows || !combine) && (rc = RgfPlan::enqueue_pair(eq_plan, neq_plan, st, active, &paired)))
+        return rc;
+    if (!paired && (rc = eq_plan.enqueue(d_eq.as<double>(), nullptr, nullptr, st, active, nullptr, combine && !rows)))
+        return rc;
     if (have_neq) {
         neq_zero = false;
-        if ((rc = neq_plan.enqueue(d_neq.as<double>(), nullptr, nullptr, st, active))) return rc;
+        if (!paired)
+            rc = neq_plan.enqueue(d_neq.as<double>(), nullptr, nullptr, st, active, nullptr, !rows);
+        else if (!rows)
+            rc = neq_plan.sum_rows(d_neq.as<double>(), st, active);
+        if (rc) return rc;
     } else if (!neq_zero) {
         // zeros once after the last non-equilibrium solve (the charge
         // components read them)
@@ -654,10 +710,33 @@ int Tube::enqueue_solve(double* dQ, hipStream_t st, bool combine, const int* act
         neq_zero = true;
     }
     if (!combine) return NEGF_OK;
-    hipLaunchKernelGGL(combine_charge_kernel, dim3((N + 255) / 256), dim3(256), 0, st, N, d_eq.as<double>(),
-                       d_neq.as<double>(), d_rho0.as<double>(), dQ);
+    if (rows) {
+        double* hQ = charge_on_host ? h_charge.as<double>() : nullptr;
+        hipLaunchKernelGGL(tube_charge_kernel, dim3((N + 63) / 64), dim3(64), 0, st, N, ep, er, np_, nr,
+                           d_rho0.as<double>(), d_eq.as<double>(), d_neq.as<double>(), dQ, hQ, eq_status(),
+                           neq_status(), hQ ? reinterpret_cast<int*>(hQ + N) : nullptr);
+    } else {
+        hipLaunchKernelGGL(combine_charge_kernel, dim3((N + 255) / 256), dim3(256), 0, st, N, d_eq.as<double>(),
+                           d_neq.as<double>(), d_rho0.as<double>(), dQ);
+    }
     NEGF_HIP_TRY(hipGetLastError());
     return NEGF_OK;
+}
+
+// Wait for the solve that was enqueued with to_host; its charge to Q (host), the
+// plans' status words into root_flag.
+int Tube::take_charge(double* Q, const double* dQ)
+{
+    if (!charge_on_host) {
+        NEGF_HIP_TRY(hipMemcpyAsync(Q, dQ, sizeof(double) * N, hipMemcpyDeviceToHost, stream));
+        return check_status();
+    }
+    NEGF_HIP_TRY(hipStreamSynchronize(stream));
+    const double* h = h_charge.as<const double>();
+    const int* s = reinterpret_cast<const int*>(h + N);
+    const int rc = (s[0] | s[1]) ? check_status() : NEGF_OK;  // reads them again and clears them
+    if (!rc) std::copy(h, h + N, Q);
+    return rc;
 }
 
 int Tube::check_status()
@@ -998,10 +1077,8 @@ int negf_solve(negf_tube* t, int iter, double* Q, int* n_intg_pts)
         return NEGF_EARG;
     }
     Tube& tb = t->t;
-    int rc = tb.solve(iter, tb.d_Q.as<double>(), tb.stream);
+    int rc = tb.solve(iter, tb.d_Q.as<double>(), tb.stream, Q);
     if (rc) return rc;
-    NEGF_HIP_TRY(hipMemcpyAsync(Q, tb.d_Q.p, sizeof(double) * tb.N, hipMemcpyDeviceToHost, tb.stream));
-    if ((rc = tb.check_status())) return rc;
     if (n_intg_pts) *n_intg_pts = tb.total_integration_pts();
     return NEGF_OK;
 }

@@ -992,16 +992,20 @@ __device__ __forceinline__ void fused_walk_split(const WLaunch& lp, const double
     }
 }
 
-__global__ __launch_bounds__(64 * FUSED_WAVES, 1) void transfer_scan_kernel(WLaunch lp, int ngroups)
+struct FusedLds {
+    double Tl[FUSED_SEGS * 9 * 32];                // [segment][component][chain]
+    double us[FUSED_WAVES][2][NEGF_SEG_MAX];       // potentials of each wave's two segments
+    double sig[4][32];                             // SL, SR of the half's chains
+};
+
+// half hf of chain group gi of a launch, by one workgroup
+__device__ __forceinline__ void transfer_scan_block(const WLaunch& lp, int gi, int hf, FusedLds& lds)
 {
-    __shared__ double Tl[FUSED_SEGS * 9 * 32];                // [segment][component][chain]
-    __shared__ double us_all[FUSED_WAVES][2][NEGF_SEG_MAX];   // potentials of each wave's two segments
-    __shared__ double sig[4][32];                             // SL, SR of the half's chains
+    double* Tl = lds.Tl;
+    auto& us_all = lds.us;
+    auto& sig = lds.sig;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int gi = blockIdx.x >> 1;
-    const int hf = blockIdx.x & 1;
-    if (gi >= ngroups) return;  // uniform over the block
     int g;
     const int t = group_tube(lp, gi, g);
     WTube tube = tube_of(lp, t);
@@ -1099,6 +1103,31 @@ __global__ __launch_bounds__(64 * FUSED_WAVES, 1) void transfer_scan_kernel(WLau
         fused_walk<false>(lp, Tl, sig, tube, ch, g, hf, cl, valid, chain);
     else
         fused_walk<true>(lp, Tl, sig, tube, ch, g, hf, cl, valid, chain);
+}
+
+__global__ __launch_bounds__(64 * FUSED_WAVES, 1) void transfer_scan_kernel(WLaunch lp, int ngroups)
+{
+    __shared__ FusedLds lds;
+    const int gi = blockIdx.x >> 1;
+    if (gi >= ngroups) return;  // uniform over the block
+    transfer_scan_block(lp, gi, blockIdx.x & 1, lds);
+}
+
+// The equilibrium and the non-equilibrium plan of one tube are as long as their slowest
+// workgroup each and far from filling the chip: both in one launch, the first ngroups[0]
+// chain groups from lp[0].  143 + 256 chains x 4012 sites: 24 us against 23 + 23 us.
+struct WLaunch2 {
+    WLaunch lp[2];
+    int n[2];  // chain groups, or sweep workgroups, of each
+};
+__global__ __launch_bounds__(64 * FUSED_WAVES, 1) void transfer_scan_pair_kernel(WLaunch2 a)
+{
+    __shared__ FusedLds lds;
+    const int b = blockIdx.x >> 1, hf = blockIdx.x & 1;
+    const int k = b >= a.n[0] ? 1 : 0;
+    const int gi = b - (k ? a.n[0] : 0);
+    if (gi >= a.n[k]) return;  // uniform over the block
+    transfer_scan_block(a.lp[k], gi, hf, lds);
 }
 
 // ------------------------------------------------------------ sweep
@@ -1520,13 +1549,12 @@ __device__ __forceinline__ void eq_full_body(const KC& k, const double* us, doub
 // w'_{hi-1} = v_{hi-1}, w'_hi = ai_{hi-1} v_hi (u_n v_n = C w_n w'_n with the
 // segment constant C, which also divides W and so drops out).
 template <int K, int NS, bool TAIL>
-__global__ __launch_bounds__(256, NS <= 4 && !TAIL ? 3 : 2) void sweep_eq_full_kernel(WLaunch lp)
+__device__ __forceinline__ void sweep_eq_block(const WLaunch& lp, int block, double (*red_all)[K * 65],
+                                               double (*us_all)[TAIL ? NEGF_SEG_MAX : K * NS])
 {
-    __shared__ double red_all[4][K * 65];
-    __shared__ double us_all[4][TAIL ? NEGF_SEG_MAX : K * NS];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    int idx = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);
+    int idx = __builtin_amdgcn_readfirstlane(block * 4 + wv);
     double* red = red_all[wv];
     if (TAIL) {
         if (idx < lp.ntail) {
@@ -1565,6 +1593,14 @@ __global__ __launch_bounds__(256, NS <= 4 && !TAIL ? 3 : 2) void sweep_eq_full_k
         const Coefs k = make_coefs(E, ch.t_even, tube.t_odd);
         eq_full_body<K, NS>(k, us, ux, uy, x, y, e, coef, te, te, red, lane, prow);
     }
+}
+
+template <int K, int NS, bool TAIL>
+__global__ __launch_bounds__(256, NS <= 4 && !TAIL ? 3 : 2) void sweep_eq_full_kernel(WLaunch lp)
+{
+    __shared__ double red_all[4][K * 65];
+    __shared__ double us_all[4][TAIL ? NEGF_SEG_MAX : K * NS];
+    sweep_eq_block<K, NS, TAIL>(lp, blockIdx.x, red_all, us_all);
 }
 
 // ------------------------------------------------------------ fused equilibrium charge
@@ -1941,13 +1977,12 @@ __device__ __forceinline__ void neq_full_scaled(const SCoefs& k, const double* u
 // per sub-block, vt = sqrt|kL Gamma_L| 2^(e_v - e_D) v / |D|; the signs of the
 // two weights multiply the squared moduli.
 template <int K, int NS, bool TAIL>
-__global__ __launch_bounds__(256, NS <= 4 && !TAIL ? 3 : 2) void sweep_neq_full_kernel(WLaunch lp)
+__device__ __forceinline__ void sweep_neq_block(const WLaunch& lp, int block, double (*red_all)[K * 65],
+                                               double (*us_all)[TAIL ? NEGF_SEG_MAX : K * NS])
 {
-    __shared__ double red_all[4][K * 65];
-    __shared__ double us_all[4][TAIL ? NEGF_SEG_MAX : K * NS];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    int idx = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);
+    int idx = __builtin_amdgcn_readfirstlane(block * 4 + wv);
     double* red = red_all[wv];
     if (TAIL) {
         if (idx < lp.ntail) {
@@ -2038,6 +2073,27 @@ __global__ __launch_bounds__(256, NS <= 4 && !TAIL ? 3 : 2) void sweep_neq_full_
         const double r = lane_sum_transpose<K>(red, lane);
         if (lane < K) prow[j * K + lane] = r;
     }
+}
+
+template <int K, int NS, bool TAIL>
+__global__ __launch_bounds__(256, NS <= 4 && !TAIL ? 3 : 2) void sweep_neq_full_kernel(WLaunch lp)
+{
+    __shared__ double red_all[4][K * 65];
+    __shared__ double us_all[4][TAIL ? NEGF_SEG_MAX : K * NS];
+    sweep_neq_block<K, NS, TAIL>(lp, blockIdx.x, red_all, us_all);
+}
+
+// Both charge sweeps of one tube in one launch (see transfer_scan_pair_kernel): lp[0]
+// the equilibrium plan's, lp[1] the other's.
+template <int K, int NS>
+__global__ __launch_bounds__(256, 2) void sweep_pair_kernel(WLaunch2 a)
+{
+    __shared__ double red_all[4][K * 65];
+    __shared__ double us_all[4][NEGF_SEG_MAX];
+    if ((int)blockIdx.x < a.n[0])
+        sweep_eq_block<K, NS, true>(a.lp[0], blockIdx.x, red_all, us_all);
+    else
+        sweep_neq_block<K, NS, true>(a.lp[1], blockIdx.x - a.n[0], red_all, us_all);
 }
 
 // One-pass fixed-order sum of the group rows of every tube: a block covers
