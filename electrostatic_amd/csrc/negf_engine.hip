@@ -95,6 +95,32 @@ static void launch_sweep(int nblk, const WLaunch& lp, hipStream_t st)
     hipLaunchKernelGGL((sweep_kernel<NEGF_SUB_K, NEGF_SUB_NS, KIND, WG>), dim3(nblk), dim3(256), 0, st, lp);
 }
 
+template <int CW>
+static void launch_transfer_scan_cw(const WLaunch& lp, int groups, hipStream_t st)
+{
+    hipLaunchKernelGGL((transfer_scan_kernel<CW>), dim3(64 / CW * groups), dim3(FusedLds<CW>::kBlock), 0, st, lp, groups);
+}
+static void launch_transfer_scan(const WLaunch& lp, int groups, hipStream_t st)
+{
+    if (groups <= FUSED_FEW_GROUPS)
+        launch_transfer_scan_cw<FUSED_CHAINS_FEW>(lp, groups, st);
+    else
+        launch_transfer_scan_cw<FUSED_CHAINS_MANY>(lp, groups, st);
+}
+template <int CW>
+static void launch_transfer_scan_cw(const WLaunch2& a, hipStream_t st)
+{
+    hipLaunchKernelGGL((transfer_scan_pair_kernel<CW>), dim3(64 / CW * (a.n[0] + a.n[1])), dim3(FusedLds<CW>::kBlock), 0,
+                       st, a);
+}
+static void launch_transfer_scan(const WLaunch2& a, hipStream_t st)
+{
+    if (a.n[0] + a.n[1] <= FUSED_FEW_GROUPS)
+        launch_transfer_scan_cw<FUSED_CHAINS_FEW>(a, st);
+    else
+        launch_transfer_scan_cw<FUSED_CHAINS_MANY>(a, st);
+}
+
 #define SWEEP_TAIL_WAVES 2048  // two wavefronts per SIMD
 
 // Sweep of full segments of ns sub-blocks (1 <= ns <= NS), partial segments beside them
@@ -153,38 +179,42 @@ int RgfPlan::kernel_time(double* total_ms, int* launches)
     return NEGF_OK;
 }
 
-// Tubes of FUSED_MIN_SEGS..FUSED_SEGS segments, and in a launch of few chain groups
-// those of fewer too, take the fused transfer and scan launch (NEGF_RGF_FUSED=0 in the
-// environment turns it off, which leaves the results the same up to rounding).  With
-// fewer segments a part of the fused launch's wavefronts is idle, which costs nothing
-// while its workgroups (two per group) do not wait for each other.
-static int fused_for(int P, int groups)
+// Tubes of FUSED_MIN_SEGS..FUSED_SEGS segments take the fused transfer and scan launch (NEGF_RGF_FUSED=0 in the
+// environment turns it off, which leaves the results the same up to rounding).  In a
+// launch of few chain groups whose tubes all fit, those of fewer segments do too: a
+// part of the fused launch's wavefronts is then idle, which costs nothing while its
+// workgroups do not wait for each other.
+static int fused_for(int P, bool few)
 {
     const char* e = std::getenv("NEGF_RGF_FUSED");
     if (e && e[0] == '0') return 0;
-    return P <= FUSED_SEGS && (P >= FUSED_MIN_SEGS || groups <= RGF_FEW_GROUPS) ? 1 : 0;
+    return P <= FUSED_SEGS && (P >= FUSED_MIN_SEGS || few) ? 1 : 0;
 }
 
-// Segment length of a tube of N sites when none is asked for.  A launch of few 64-chain
+// Segment length when none is asked for, of a launch whose longest tube has N sites (one
+// length for all of them: every other one is a sweep launch more).  A launch of few 64-chain
 // groups is short of wavefronts and as long as one segment takes: the shortest
 // multiple of NEGF_SUB_K that keeps the tube within the fused launch's segments, where
 // the default length would give fewer than it takes.  0 (the default) otherwise.
 // Measured, equilibrium charge with host part, short against default length: 64 to 4096
 // energies (1 to 64 groups) 46 .. 76 us against 49 .. 80 us at 40 to 1501 sites, diag G
-// of 1501 x 777 69 against 84 us; 96 groups (32 tubes of 1024, 600, 256 sites) 58.7,
-// 52.1, 40.4 against 62.2, 54.6, 50.5 us an SCF iteration; 128 groups (8192 energies)
-// 88 against 81 us at 1000 sites, 95 against 87 us at 1501.
+// of 1501 x 777 69 against 84 us; 128 groups (8192 energies) 88 against 81 us at 1000
+// sites, 95 against 87 us at 1501.  Above FUSED_FEW_GROUPS, where workgroups share the
+// CUs, half the segments: 96 groups, 1024 / 600 / 256 sites, in us an SCF iteration: 16
+// segments 52.2 / 44.8 / 37.3, 32 segments 54.9 / 47.6 / - , the default length's
+// 59.0 / 54.6 / 48.9.
 static int segment_length_for(int N, int groups)
 {
     if (groups > RGF_FEW_GROUPS) return 0;
     if ((N + NEGF_SEG_DEFAULT - 1) / NEGF_SEG_DEFAULT >= FUSED_MIN_SEGS) return 0;
-    const int L = (N + FUSED_SEGS - 1) / FUSED_SEGS;
+    const int segs = groups <= FUSED_FEW_GROUPS ? FUSED_SEGS : FUSED_SEGS / 2;
+    const int L = (N + segs - 1) / segs;
     return (L + NEGF_SUB_K - 1) / NEGF_SUB_K * NEGF_SUB_K;
 }
 
 // Kernel-side descriptor of one tube whose items start at item0 and whose
 // partial rows start at part_off.
-static WTube make_wtube(const RgfTube& tb, int P, int L, int item0, long long part_off, int groups)
+static WTube make_wtube(const RgfTube& tb, int P, int L, int item0, long long part_off, bool few)
 {
     WTube w;
     std::memset(&w, 0, sizeof(w));
@@ -203,7 +233,7 @@ static WTube make_wtube(const RgfTube& tb, int P, int L, int item0, long long pa
     w.part_off = part_off;
     for (int q = 0; q < 3; ++q) w.sample[q] = tb.sample[q];
     w.ext = tb.ext;
-    w.fused = fused_for(P, groups);
+    w.fused = fused_for(P, few);
     return w;
 }
 
@@ -246,8 +276,17 @@ int RgfPlan::build(int kind, bool write_G, const std::vector<RgfTube>& tubes, Ch
     max_P_ = 0;
     max_groups_ = 0;
     any_fused_ = any_fused2_ = any_unfused_ = false;
-    int groups = 0;  // 64-chain groups of the launch
-    for (const RgfTube& tb : tubes) groups += (std::max(tb.nchain, 0) + 63) / 64;
+    int groups = 0, longest = 0;  // 64-chain groups of the launch, sites of its longest tube
+    for (const RgfTube& tb : tubes) {
+        groups += (std::max(tb.nchain, 0) + 63) / 64;
+        longest = std::max(longest, tb.N);
+    }
+    const int L_free = segment_length_for(longest, groups);
+    bool few = groups <= RGF_FEW_GROUPS;
+    for (const RgfTube& tb : tubes) {
+        int P, L;
+        few = few && choose_segments(tb.N, tb.L > 0 ? tb.L : L_free, &P, &L) && P <= FUSED_SEGS;
+    }
     for (int t = 0; t < ntubes_; ++t) {
         const RgfTube& tb = tubes[t];
         if (tb.N < 2 || !tb.dU || tb.nchain <= 0 || tb.t_odd <= 0 || tb.chain0 < 0 ||
@@ -257,12 +296,12 @@ int RgfPlan::build(int kind, bool write_G, const std::vector<RgfTube>& tubes, Ch
             return NEGF_EARG;
         }
         int P, L;
-        if (!choose_segments(tb.N, tb.L > 0 ? tb.L : segment_length_for(tb.N, groups), &P, &L)) {
+        if (!choose_segments(tb.N, tb.L > 0 ? tb.L : L_free, &P, &L)) {
             set_error("chain of %d sites exceeds the supported maximum %d", tb.N, max_sites());
             return NEGF_ENOTSUP;
         }
         WTube& w = wt[t];
-        w = make_wtube(tb, P, L, items, poff, groups);
+        w = make_wtube(tb, P, L, items, poff, few);
         // equilibrium charge on full 128-site segments: the whole launch fused
         if (w.fused && P >= FUSED_MIN_SEGS && kind == KIND_EQ && !write_G && L == NEGF_SEG_MAX && tb.N % L == 0)
             w.fused = 2;
@@ -432,7 +471,7 @@ static int launch_rgf_kernels(const RgfLayout& y, const WLaunch& lp, hipStream_t
         hipLaunchKernelGGL(scan_kernel, dim3(2 * y.nsblk), dim3(64 * SCAN_WAVES), 0, st, lp, y.nsblk);
     }
     if (y.any_fused)
-        hipLaunchKernelGGL(transfer_scan_kernel, dim3(2 * y.nsblk), dim3(64 * FUSED_WAVES), 0, st, lp, y.nsblk);
+        launch_transfer_scan(lp, y.nsblk, st);
     if (y.any_fused2)
         hipLaunchKernelGGL((rgf_eq_fused_kernel<NEGF_SUB_K, NEGF_SUB_NS>), dim3(2 * y.nsblk), dim3(64 * EQF_WAVES), 0,
                            st, lp, y.nsblk);
@@ -574,7 +613,7 @@ int RgfPlan::enqueue_pair(const RgfPlan& eq, const RgfPlan& neq, hipStream_t st,
         l.ntail = y.slow_n;
         sw.n[k] = (l.nlist + l.ntail + 3) / 4;
     }
-    hipLaunchKernelGGL(transfer_scan_pair_kernel, dim3(2 * (ts.n[0] + ts.n[1])), dim3(64 * FUSED_WAVES), 0, st, ts);
+    launch_transfer_scan(ts, st);
     launch_sweep_pair<NEGF_SUB_NS>(ns, sw, st);
     NEGF_HIP_TRY(hipGetLastError());
     *done = true;
@@ -900,7 +939,7 @@ int negf_rgf_diag_accumulate_noalloc(const negf_chain_params* p, const double* d
     }
     const size_t items = G * (size_t)P;
     // the same launch forms as RgfPlan::build
-    WTube tb = make_wtube(one_tube(p, d_U, nE), P, L, 0, 0, (int)G);
+    WTube tb = make_wtube(one_tube(p, d_U, nE), P, L, 0, 0, G <= RGF_FEW_GROUPS && P <= FUSED_SEGS);
     if (tb.fused && P >= FUSED_MIN_SEGS && !d_diagG && L == NEGF_SEG_MAX && p->N % L == 0) tb.fused = 2;
     const size_t rows = tb.fused == 2 ? 2 * G : G;
     size_t off = 0;

@@ -793,33 +793,42 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void scan_kernel(WLaunch lp, int n
 }
 
 // ------------------------------------------------------------ fused transfer + scan
-// Chain groups of tubes with FUSED_MIN_SEGS..FUSED_SEGS segments take one
-// launch for both steps, and their segment matrices never leave the CU (the
-// separate launches write them to memory and read them back twice, once per
-// walk).  One workgroup of FUSED_WAVES wavefronts per (64-chain group, half of
-// 32 chains).  Wave w computes the transfer matrices of segments w (lanes
-// 0-31) and w + FUSED_WAVES (lanes 32-63) of the half's chains into LDS, in
-// the arithmetic of transfer_kernel; then the first 32 lanes of wave 0 walk
-// them forward (u) and those of wave 1 backward (v), in the arithmetic of
-// scan_kernel, writing the same segment states and D.  The states are
-// renormalised every SCAN_RENORM steps of the walk (by exact powers of two,
-// so the stored (mantissa, exponent) pairs describe the same numbers for any
-// schedule).
-#define FUSED_WAVES 16
-#define FUSED_SEGS (2 * FUSED_WAVES)
+// Chain groups of tubes with FUSED_MIN_SEGS..FUSED_SEGS segments (in a launch of few
+// groups: any number up to FUSED_SEGS) take one launch for both steps, and their
+// segment matrices never leave the CU (the separate launches write them to memory and
+// read them back twice, once per walk).  One workgroup per CW chains of a 64-chain
+// group: CW / 2 wavefronts compute the transfer matrices of 64 / CW segments each into
+// LDS, in the arithmetic of transfer_kernel; the lead self-energies are one more
+// wavefront's (CW = 32: the first one's, the workgroup is full); then wavefront 0
+// walks the matrices forward (u) and wavefront 1 backward (v), in the arithmetic of
+// scan_kernel, writing the same segment states and D.  The states are renormalised
+// every FUSED_CHUNK steps of the walk (by exact powers of two, so the stored
+// (mantissa, exponent) pairs describe the same numbers for any schedule).
+//
+// Bound by latency: one segment's transfer (83 cycles a site for a wavefront alone on
+// its SIMD, 64 cycles a site each for four that share one), then the walk (about 400
+// cycles a step).  A launch of few groups takes 8 chains per workgroup: one wavefront
+// per SIMD, eight workgroups per group, the self-energies (4400 cycles) off the path.
+// Measured, 8 against 32 chains: 25 segments of 16 sites 10.2 against 11.4 us, 32 of
+// 128 sites 17.2 against 23.2 us, 32 of 48 sites 14.3 against 16.6 us.  Where the
+// groups fill the chip, 32 chains share one walk: 96 groups of 32 segments of 32 sites
+// 17.2 us against 20.0 (8 chains) and 21.8 us (16).
+#define FUSED_SEGS 32
+#define FUSED_CHAINS_FEW 8
+#define FUSED_CHAINS_MANY 32
+#define FUSED_FEW_GROUPS 32  // chain groups up to which FUSED_CHAINS_FEW is taken (one workgroup per CU)
 #define FUSED_MIN_SEGS 17
 #define RGF_FEW_GROUPS 96  // chain groups of a launch that counts as short of wavefronts
+#define FUSED_CHUNK 4
 
-
-// One walk over the segment matrices in LDS (V: the v walk), by the 32 lanes
-// of one wavefront, in chunks of CH steps whose matrices are read from LDS
+// One walk over the segment matrices in LDS (V: the v walk), by CW lanes of one
+// wavefront (c0: the first one's chain within its group), in chunks of CH steps whose matrices are read from LDS
 // together, the state renormalised once per chunk (by exact powers of two, so
 // the chunk length changes no value); the arithmetic is scan_kernel's.  The
 // states go to the segment-state array in memory, as scan_kernel writes them.
-#define FUSED_CHUNK 4
-template <bool V, int CH = FUSED_CHUNK>
-__device__ __forceinline__ void fused_walk(const WLaunch& lp, const double* Tl, const double (*sig)[32],
-                                           const WTube& tube, const ChainDesc& ch, int g, int hf, int cl,
+template <bool V, int CW, int CH = FUSED_CHUNK>
+__device__ __forceinline__ void fused_walk(const WLaunch& lp, const double* Tl, const double (*sig)[CW],
+                                           const WTube& tube, const ChainDesc& ch, int g, int c0, int cl,
                                            bool valid, int chain)
 {
     const int P = tube.P, L = tube.L, N = tube.N;
@@ -838,18 +847,18 @@ __device__ __forceinline__ void fused_walk(const WLaunch& lp, const double* Tl, 
     int ex = 0;
     const double idet_odd = te / to;  // 1/det T_s when hi - 1 is even
     const long long item0 = tube.item0 + (long long)g * P;
-    double* Sb = lp.St + item0 * 10 * 64 + (V ? 5 : 0) * 64 + hf * 32 + cl;
+    double* Sb = lp.St + item0 * 10 * 64 + (V ? 5 : 0) * 64 + c0 + cl;
     for (int i0 = 0; i0 < P; i0 += CH) {
         Mat2 m[CH];
 #pragma unroll
         for (int q = 0; q < CH; ++q) {
             const int i = min(i0 + q, P - 1);
-            const double* T = Tl + (V ? P - 1 - i : i) * 9 * 32 + cl;
-            m[q].a = make_double2(T[0 * 32], T[1 * 32]);
-            m[q].b = make_double2(T[2 * 32], T[3 * 32]);
-            m[q].c = make_double2(T[4 * 32], T[5 * 32]);
-            m[q].d = make_double2(T[6 * 32], T[7 * 32]);
-            m[q].e = T[8 * 32];
+            const double* T = Tl + (V ? P - 1 - i : i) * 9 * CW + cl;
+            m[q].a = make_double2(T[0 * CW], T[1 * CW]);
+            m[q].b = make_double2(T[2 * CW], T[3 * CW]);
+            m[q].c = make_double2(T[4 * CW], T[5 * CW]);
+            m[q].d = make_double2(T[6 * CW], T[7 * CW]);
+            m[q].e = T[8 * CW];
         }
 #pragma unroll
         for (int q = 0; q < CH; ++q) {
@@ -992,18 +1001,22 @@ __device__ __forceinline__ void fused_walk_split(const WLaunch& lp, const double
     }
 }
 
+template <int CW>
 struct FusedLds {
-    double Tl[FUSED_SEGS * 9 * 32];                // [segment][component][chain]
-    double us[FUSED_WAVES][2][NEGF_SEG_MAX];       // potentials of each wave's two segments
-    double sig[4][32];                             // SL, SR of the half's chains
+    // transfer wavefronts, and one for the self-energies where the workgroup has room
+    static constexpr int kWaves = FUSED_SEGS * CW / 64, kBlock = 64 * (kWaves + (kWaves < 16 ? 1 : 0));
+    double Tl[FUSED_SEGS * 9 * CW];                // [segment][component][chain]
+    // potentials, segment s at s (L + 2): the eight segments that a wavefront reads
+    // together lie in different banks
+    double us[FUSED_SEGS * (NEGF_SEG_MAX + 2)];
+    double sig[4][CW];                             // SL, SR of the workgroup's chains
 };
 
-// half hf of chain group gi of a launch, by one workgroup
-__device__ __forceinline__ void transfer_scan_block(const WLaunch& lp, int gi, int hf, FusedLds& lds)
+// chains [c0, c0 + CW) of chain group gi of a launch, by one workgroup
+template <int CW>
+__device__ __forceinline__ void transfer_scan_block(const WLaunch& lp, int gi, int c0, FusedLds<CW>& lds)
 {
-    double* Tl = lds.Tl;
-    auto& us_all = lds.us;
-    auto& sig = lds.sig;
+    constexpr int NW = FusedLds<CW>::kWaves;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int g;
@@ -1013,104 +1026,102 @@ __device__ __forceinline__ void transfer_scan_block(const WLaunch& lp, int gi, i
     tube.L = __builtin_amdgcn_readfirstlane(tube.L);
     tube.P = __builtin_amdgcn_readfirstlane(tube.P);
     tube.nchain = __builtin_amdgcn_readfirstlane(tube.nchain);
-    // (a half without chains still runs, on copies of the group's last chain:
+    // (a workgroup without chains still runs, on copies of the group's last chain:
     // the sweeps read the states of all 64 lanes and mask the contributions)
     if (tube.fused != 1 || tube_skipped(lp, tube)) return;  // uniform over the block
     const int P = tube.P, L = tube.L, N = tube.N;
-    const int h = lane >> 5, cl = lane & 31;
-    const int lc = g * 64 + hf * 32 + cl;
+    const int cl = lane & (CW - 1);
+    const int lc = g * 64 + c0 + cl;
     const bool valid = lc < tube.nchain;
     const int chain = tube.chain0 + (valid ? lc : tube.nchain - 1);
     const ChainDesc ch = lp.chains[chain];
     const double2 E = make_double2(ch.Er, ch.Ei);
     const double te = ch.t_even, to = tube.t_odd;
-
-    // potentials of the wave's two segments (zero past the end of the tube);
-    // every load is issued before the first LDS write
-    {
-        constexpr int R = 2 * NEGF_SEG_MAX / 64;
-        double uv[R];
+    double* Tl = lds.Tl;
+    double* us = lds.us;
+    if (w == (NW < 16 ? NW : 0)) {
+        // lead self-energies: closed form (also stored for the sweeps), or as the
+        // decimation launch left them in the chain table
+        if (lane < CW) {
+            double2 SL = make_double2(ch.SLr, ch.SLi), SR = make_double2(ch.SRr, ch.SRi);
+            if (!lp.dec_use) lead_sigma<false>(lp, valid ? lp.chains + chain : nullptr, ch, tube, &SL, &SR);
+            lds.sig[0][cl] = SL.x;
+            lds.sig[1][cl] = SL.y;
+            lds.sig[2][cl] = SR.x;
+            lds.sig[3][cl] = SR.y;
+        }
+    }
+    if (w < NW) {
+        // the wavefront's own segments, N <= P L <= FUSED_SEGS L
+        constexpr int SW = 64 / CW, R = NEGF_SEG_MAX / 64;
+        double uv[SW * R];
 #pragma unroll
-        for (int q = 0; q < R; ++q) {
-            const int i = lane + 64 * q;
-            const int hh = i >= L ? 1 : 0;
-            const int site = (w + FUSED_WAVES * hh) * L + (i - hh * L);
-            uv[q] = tube.U[min(site, N - 1)];
+        for (int q = 0; q < SW * R; ++q) {  // the loads in flight together
+            const int i = lane + 64 * (q % R);
+            uv[q] = tube.U[min((w * SW + q / R) * L + min(i, L - 1), N - 1)];
         }
 #pragma unroll
-        for (int q = 0; q < R; ++q) {
-            const int i = lane + 64 * q;
-            const int hh = i >= L ? 1 : 0;
-            const int site = (w + FUSED_WAVES * hh) * L + (i - hh * L);
-            if (i < 2 * L) us_all[w][hh][i - hh * L] = site < N ? uv[q] : 0.0;
+        for (int q = 0; q < SW * R; ++q) {
+            const int i = lane + 64 * (q % R);
+            if (i < L) us[(w * SW + q / R) * (L + 2) + i] = uv[q];
         }
-    }
-    // lead self-energies: the lanes of segment 0 (closed form, also stored for
-    // the sweeps), or as the decimation launch left them in the chain table
-    if (w == 0 && h == 0) {
-        double2 SL = make_double2(ch.SLr, ch.SLi), SR = make_double2(ch.SRr, ch.SRi);
-        if (!lp.dec_use) lead_sigma<false>(lp, valid ? lp.chains + chain : nullptr, ch, tube, &SL, &SR);
-        sig[0][cl] = SL.x;
-        sig[1][cl] = SL.y;
-        sig[2][cl] = SR.x;
-        sig[3][cl] = SR.y;
-    }
-    __builtin_amdgcn_wave_barrier();
-
-    const int s = w + FUSED_WAVES * h;  // this lane's segment
-    const int lo = min(N, s * L);
-    const int n = s < P ? min(N, lo + L) - lo : 0;
-    const double* us = us_all[w][h];
-    double2 m00 = make_double2(1.0, 0.0), m01 = make_double2(0.0, 0.0);
-    double2 m10 = make_double2(0.0, 0.0), m11 = make_double2(1.0, 0.0);
-    int eT = 0;
-    if (__all(scaled_ok(E, te, to))) {
-        const SCoefs ks = make_scoefs(E, te, to);
-        if (n > 0) {
-            const int hi = lo + n;
-            m11 = make_double2(((lo - 1) & 1) ? ks.ai[1] : ks.ai[0], 0.0);
-            transfer_loop<NEGF_SUB_K>(ks, us, n, m00, m01, m10, m11, eT);
-            double mC;
-            int eC;
-            scale_prod(ks, lo & 1, n - 1, mC, eC);
-            const double r0 = mC * (((hi - 1) & 1) ? ks.ai[1] : ks.ai[0]);
-            m00 = cscale(r0, m00);
-            m01 = cscale(r0, m01);
-            m10 = cscale(mC, m10);
-            m11 = cscale(mC, m11);
-            eT += eC;
-            renorm_mat(m00, m01, m10, m11, eT);
+        __builtin_amdgcn_wave_barrier();
+        const int s = w * SW + lane / CW;  // this lane's segment
+        const int lo = min(N, s * L);
+        const int n = s < P ? min(N, lo + L) - lo : 0;
+        const double* up = us + s * (L + 2);
+        double2 m00 = make_double2(1.0, 0.0), m01 = make_double2(0.0, 0.0);
+        double2 m10 = make_double2(0.0, 0.0), m11 = make_double2(1.0, 0.0);
+        int eT = 0;
+        if (__all(scaled_ok(E, te, to))) {
+            const SCoefs ks = make_scoefs(E, te, to);
+            if (n > 0) {
+                const int hi = lo + n;
+                m11 = make_double2(((lo - 1) & 1) ? ks.ai[1] : ks.ai[0], 0.0);
+                transfer_loop<NEGF_SUB_K>(ks, up, n, m00, m01, m10, m11, eT);
+                double mC;
+                int eC;
+                scale_prod(ks, lo & 1, n - 1, mC, eC);
+                const double r0 = mC * (((hi - 1) & 1) ? ks.ai[1] : ks.ai[0]);
+                m00 = cscale(r0, m00);
+                m01 = cscale(r0, m01);
+                m10 = cscale(mC, m10);
+                m11 = cscale(mC, m11);
+                eT += eC;
+                renorm_mat(m00, m01, m10, m11, eT);
+            }
+        } else {
+            const Coefs k = make_coefs(E, te, to);
+            if (n > 0) transfer_loop<NEGF_SUB_K>(k, up, n, m00, m01, m10, m11, eT);
         }
-    } else {
-        const Coefs k = make_coefs(E, te, to);
-        if (n > 0) transfer_loop<NEGF_SUB_K>(k, us, n, m00, m01, m10, m11, eT);
-    }
-    if (s < P) {
-        double* T = Tl + s * 9 * 32 + cl;
-        T[0 * 32] = m00.x;
-        T[1 * 32] = m00.y;
-        T[2 * 32] = m01.x;
-        T[3 * 32] = m01.y;
-        T[4 * 32] = m10.x;
-        T[5 * 32] = m10.y;
-        T[6 * 32] = m11.x;
-        T[7 * 32] = m11.y;
-        T[8 * 32] = (double)eT;
+        if (s < P) {
+            double* T = Tl + s * 9 * CW + cl;
+            T[0 * CW] = m00.x;
+            T[1 * CW] = m00.y;
+            T[2 * CW] = m01.x;
+            T[3 * CW] = m01.y;
+            T[4 * CW] = m10.x;
+            T[5 * CW] = m10.y;
+            T[6 * CW] = m11.x;
+            T[7 * CW] = m11.y;
+            T[8 * CW] = (double)eT;
+        }
     }
     __syncthreads();
-    if (w >= 2 || lane >= 32) return;
+    if (w >= 2 || lane >= CW) return;
     if (w == 0)
-        fused_walk<false>(lp, Tl, sig, tube, ch, g, hf, cl, valid, chain);
+        fused_walk<false, CW>(lp, Tl, lds.sig, tube, ch, g, c0, cl, valid, chain);
     else
-        fused_walk<true>(lp, Tl, sig, tube, ch, g, hf, cl, valid, chain);
+        fused_walk<true, CW>(lp, Tl, lds.sig, tube, ch, g, c0, cl, valid, chain);
 }
 
-__global__ __launch_bounds__(64 * FUSED_WAVES, 1) void transfer_scan_kernel(WLaunch lp, int ngroups)
+template <int CW>
+__global__ __launch_bounds__(FusedLds<CW>::kBlock) void transfer_scan_kernel(WLaunch lp, int ngroups)
 {
-    __shared__ FusedLds lds;
-    const int gi = blockIdx.x >> 1;
+    __shared__ __align__(16) FusedLds<CW> lds;
+    const int gi = blockIdx.x / (64 / CW);
     if (gi >= ngroups) return;  // uniform over the block
-    transfer_scan_block(lp, gi, blockIdx.x & 1, lds);
+    transfer_scan_block<CW>(lp, gi, blockIdx.x % (64 / CW) * CW, lds);
 }
 
 // The equilibrium and the non-equilibrium plan of one tube are as long as their slowest
@@ -1120,14 +1131,15 @@ struct WLaunch2 {
     WLaunch lp[2];
     int n[2];  // chain groups, or sweep workgroups, of each
 };
-__global__ __launch_bounds__(64 * FUSED_WAVES, 1) void transfer_scan_pair_kernel(WLaunch2 a)
+template <int CW>
+__global__ __launch_bounds__(FusedLds<CW>::kBlock) void transfer_scan_pair_kernel(WLaunch2 a)
 {
-    __shared__ FusedLds lds;
-    const int b = blockIdx.x >> 1, hf = blockIdx.x & 1;
+    __shared__ __align__(16) FusedLds<CW> lds;
+    const int b = blockIdx.x / (64 / CW);
     const int k = b >= a.n[0] ? 1 : 0;
     const int gi = b - (k ? a.n[0] : 0);
     if (gi >= a.n[k]) return;  // uniform over the block
-    transfer_scan_block(a.lp[k], gi, hf, lds);
+    transfer_scan_block<CW>(a.lp[k], gi, blockIdx.x % (64 / CW) * CW, lds);
 }
 
 // ------------------------------------------------------------ sweep
