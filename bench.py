@@ -390,7 +390,7 @@ def block_leg(steps=3, with_cpu=True):
            "flop_per_energy_block": 36 * m ** 3,
            "rgf_tflops": flops / (rg * 1e-3) / 1e12,
            "rgf_frac_fp64_peak": flops / (rg * 1e-3) / 1e12 / FP64_PEAK_TFLOPS,
-           "note": "fraction at the executed 36 m^3 flops per energy-block (real H0 and T); "
+           "note": "fraction at the general sweep's 36 m^3 flops per energy-block (real H0 and T); "
                    "a general complex block would need 56 m^3"}
     if with_cpu:
         from oracle import block_oracle as B
