@@ -1279,8 +1279,8 @@ class BatchScf {
         for (int k = 0; k < seed_iters; ++k) {
             // the capacitances follow the seed once, half way
             if (k > 0 && k == seed_iters / 2 && (rc = enqueue_capacitance())) return rc;
-            if ((rc = sg->evaluate(T, d_U.as<double>(), has_feat ? d_feat.as<double>() : nullptr, d_Q.as<double>(), st)))
-                return rc;
+            if ((rc = sg->forward(T, d_U.as<double>(), has_feat ? d_feat.as<double>() : nullptr, st))) return rc;
+            if ((rc = sg->output(T, d_Q.as<double>(), st))) return rc;
             if ((rc = enqueue_precondition(d_Q.as<double>()))) return rc;
             hipLaunchKernelGGL(batch_seed_step_kernel, dim3((unsigned)((NT + 255) / 256)), dim3(256), 0, st, N, T,
                                base().n_in, state_stride, d_PF.as<double>(), kSeedStep);

@@ -16,11 +16,10 @@
 // copy Wt[ci][tap][co] = W[co][8 - tap][ci] turns the data gradient into a
 // forward convolution.
 //
-// The five convolutions into 64 channels (forward, tangent, or the data
-// gradient of layers 5..1) and the last layer run as one launch over tiles of
-// sites, the activations in LDS (sg_chain_kernel).  Every convolution is an
-// implicit GEMM on v_mfma_f32_16x16x32_bf16: M = 16 output channels, N = 16
-// sites, K = 9 taps x input channels.  Operand layout: lane l
+// Every convolution is an implicit GEMM on v_mfma_f32_16x16x32_bf16:
+// M = 16 output channels per MFMA (two per wavefront), N = 16 sites per MFMA
+// tile (16 tiles = 256 sites per workgroup), K = 9 taps x input channels, with
+// the site tile and a 4-site halo on each side staged in LDS.  Operand layout: lane l
 // holds A[i][k] with i = l % 16 and B[k][j] with j = l % 16 for the same
 // eight k of its 16-lane group, and receives D[i][j] for i = 4 (l / 16) + v,
 // v = 0..3, j = l % 16.  (Which eight k a lane group holds does not matter:
@@ -31,345 +30,161 @@
 #include <cmath>
 #include <cstring>
 #include <random>
-#include <type_traits>
 
 #include "negf_material.h"
 
 namespace negf {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(4))) float f4;
+
+enum SgEpi { EPI_TANH = 0, EPI_LINEAR_OUT = 1, EPI_DTANH = 2 };
 
 __device__ __forceinline__ f4 mfma_bf16(const bf16x8& a, const bf16x8& b, const f4& c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// tanh for a result rounded to BF16: x P(x^2) / Q(x^2) with the coefficients of
-// a weighted least-squares fit to tanh(x) / x on [0, 4] (relative error below
-// 4e-7), beyond 4 the value at 4 (0.99933, which rounds to 1).  Nine
-// instructions and one v_rcp_f32; the epilogues of a layer take as long as its
-// MFMAs, so this is the other half of the kernel's time.
+// Y = epilogue(conv9(X, W) [+ bias]) for one sample (blockIdx.y) and
+// SG_TILE sites, as an implicit GEMM on v_mfma_f32_16x16x32_bf16
+// (A = weights [co][ci], B = staged inputs [ci][site], D [co][site]).
+// X bf16 [B][N][CIN], W bf16 [COUT][9][CIN]; COUT/32 wavefronts, each owning
+// 32 output channels whose 9 x CIN/32 x 2 weight fragments stay in its
+// registers across the tile's SG_TILE/16 site tiles, so that every input
+// fragment read from LDS feeds two MFMAs (one per 16-channel block) and the
+// weights are read once per workgroup.
+//   EPI_TANH:       Y bf16 [B][N][COUT] = tanh(acc + b)
+//   EPI_LINEAR_OUT: Yf float [B][N] = acc(co = 0) (+ b[0] if bias)
+//   EPI_DTANH:      Y bf16 [B][N][COUT] = acc * (1 - xp^2), xp bf16 [B][N][COUT]
+// tanh for a result rounded to BF16 (relative error below 1e-5, a
+// thousandth of a BF16 ulp): tanh|x| = (1 - e) / (1 + e) with e = exp(-2|x|)
+// from v_exp_f32 (2^y) and v_rcp_f32, and the odd Taylor series
+// x - x^3/3 + 2x^5/15 below |x| = 1/16, where 1 - e cancels (truncation
+// 17/315 x^7, below 4e-9 relative there).
 __device__ __forceinline__ float sg_tanh(float x)
 {
-    x = __builtin_amdgcn_fmed3f(x, -4.0f, 4.0f);
-    const float s = x * x;
-    const float p = fmaf(s, fmaf(s, 1.75496324e-3f, 1.18174323e-1f), 9.99999645e-1f);
-    const float q = fmaf(s, fmaf(s, fmaf(s, 7.30915899e-5f, 1.89287477e-2f), 4.51504160e-1f), 1.0f);
-    return x * p * __builtin_amdgcn_rcpf(q);
+    const float a = fabsf(x);
+    const float e = __builtin_amdgcn_exp2f(-2.8853900817779268f * a);  // -2 / ln 2
+    const float big = (1.0f - e) * __builtin_amdgcn_rcpf(1.0f + e);
+    const float x2 = a * a;
+    const float small = a * (1.0f - x2 * (1.0f / 3.0f - x2 * (2.0f / 15.0f)));
+    return copysignf(a < 0.0625f ? small : big, x);
 }
 
-// ---- the whole network on a tile of sites
-//   SG_FWD   x_1 = tanh(conv(x_0) + b_0), ..., x_5; q = conv(x_5) + b_5
-//   SG_TAN   the tangent of the same: t_{l+1} = conv(t_l) (1 - x_{l+1}^2)
-//   SG_BWD   data gradients: dz_4 = conv(dq; Wt_5) (1 - x_5^2), ..., dz_0
-// One workgroup of 8 wavefronts per (tile of T sites, sample).  All layers are
-// computed on the window of T + 40 sites (the last one needs four more sites on
-// each side per layer before it; what lies further out is not used), from one
-// LDS buffer into the other, so no activation makes a round trip through
-// memory; with STORE the tile's part of every layer is also written out.
-//
-// The window has 16 R sites and lane i of an operand holds site r + R i of row r:
-// the tap shift is then another row, not another lane, and the fragments of
-// rows r - 4 .. r + U + 3 serve U output rows: 2 (U + 8) LDS reads for 18 U
-// MFMAs (a layout with lane = neighbouring site needs 18 U).  Wavefront w makes
-// output channels 16 (w % 4) .. + 15 of half of the rows, its 18 weight
-// fragments in registers and those of the next layer on their way.
-// The first layer has one or three real channels: their nine taps fill one K
-// block (im2col in LDS).  The last layer has one output channel: its nine taps
-// are the M rows, z[tap][s] = sum_ci W[tap][ci] x[s][ci], summed as
-// q[n] = sum_tap z[tap][n + tap - 4].
-// Bound by MFMA and the epilogues' VALU (tanh): a row of a layer takes 500 cycles
-// of a CU, its MFMAs 290 and its epilogues about 350 (two wavefronts per SIMD,
-// partly overlapped; epilogues placed between the next rows' MFMAs by hand
-// and raised priorities for half of the wavefronts gained nothing), and about 15 us
-// per workgroup are latencies of the layers' first loads and barriers.
-// Measured, 128 x 2048 sites: 105 us for the forward pass against 185 us for one
-// launch per layer (each LDS fragment read for two MFMAs, activations through
-// memory); 32 x 2048 with the activations written: 50 against 107 us, the data
-// gradients of layers 5..1: 46 against 87 us.
-enum SgMode { SG_FWD = 0, SG_TAN = 1, SG_BWD = 2 };
-constexpr int CH_HALO = SG_HALO * (SG_LAYERS - 1);  // window sites beyond the tile, per side
-constexpr int CH_RMAX = 36;                         // rows of a window: 153 KiB of LDS
-constexpr int CH_WMAX = 16 * CH_RMAX;
-
-struct SgChainArgs {
-    int N, T, R;                        // sites per sample and tile, rows of a window (16 R >= T + 2 CH_HALO)
-    const double* in;                   // U or V [B][N]
-    const double* feat;                 // [B] or null
-    const __bf16* dq;                   // SG_BWD: gradient at the output [B][N]
-    const __bf16* w[SG_LAYERS];         // weights of step s: layer s, or layer 5 - s transposed
-    const float* bias[SG_LAYERS];
-    __bf16* x[SG_LAYERS];               // x_1 .. x_5 (index 1 ..): written (SG_FWD, STORE) or read
-    __bf16* dz[SG_LAYERS];              // SG_BWD: dz_0 .. dz_4, written
-    float* q;                           // output [B][N] (may be null)
-    double* Q;                          // mean + scale q (may be null)
-    double mean, scale;
-};
-
-template <int U>
-struct ChOut {
-    f4 acc[U];
-};
-
-// U output rows from r0 on: acc[u] += sum over taps and channels.  Row r = -4 ..
-// R + 3 of a lane (i, g) is the site s = r + R i; 16-byte chunk c of a site lies
-// at c ^ (s / R mod 8), and s / R is i - 1 (below row 0), i or i + 1 (from row R
-// on): olo, omid, ohi are the byte offsets of chunk g of site R i in those cases.
-template <int U>
-__device__ __forceinline__ void ch_rows(const char* buf, int olo, int omid, int ohi, int r0, int R,
-                                        const bf16x8 (&a)[SG_KW][2], ChOut<U>& o)
+template <int EPI>
+__device__ __forceinline__ void sg_epilogue(const f4& acc, int cb, size_t site, int COUT, const float* bias,
+                                            __bf16* Y, float* Yf, const __bf16* xp)
 {
+    if (EPI == EPI_TANH) {
+        __attribute__((aligned(8))) __bf16 o[4];
 #pragma unroll
-    for (int t = 0; t < U + 2 * SG_HALO; ++t) {
-        const int row = r0 - SG_HALO + t;  // wave-uniform
-        const int off = row < 0 ? olo : row >= R ? ohi : omid;
-        const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(buf + row * 128 + off);
-        const bf16x8 b1 = *reinterpret_cast<const bf16x8*>(buf + row * 128 + (off ^ 64));
+        for (int v = 0; v < 4; ++v) o[v] = (__bf16)sg_tanh(acc[v] + bias[cb + v]);
+        *reinterpret_cast<uint2*>(Y + site * COUT + cb) = *reinterpret_cast<const uint2*>(o);
+    } else if (EPI == EPI_LINEAR_OUT) {
+        if (cb == 0) Yf[site] = acc[0] + (bias ? bias[0] : 0.0f);
+    } else {
+        const uint2 raw = *reinterpret_cast<const uint2*>(xp + site * COUT + cb);
+        const __bf16* xq = reinterpret_cast<const __bf16*>(&raw);
+        __attribute__((aligned(8))) __bf16 o[4];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int tap = t - u;
-            if (tap < 0 || tap >= SG_KW) continue;
-            o.acc[u] = mfma_bf16(a[tap][0], b0, o.acc[u]);
-            o.acc[u] = mfma_bf16(a[tap][1], b1, o.acc[u]);
+        for (int v = 0; v < 4; ++v) {
+            const float y = (float)xq[v];
+            o[v] = (__bf16)(acc[v] * (1.0f - y * y));
         }
+        *reinterpret_cast<uint2*>(Y + site * COUT + cb) = *reinterpret_cast<const uint2*>(o);
     }
 }
 
-// tanh (SG_FWD) or (1 - y^2) (y: this lane's four channels of xp) of one row,
-// rounded to BF16, zero outside the sample, into the other buffer
-template <int MODE>
-__device__ __forceinline__ void ch_store(const f4& acc, uint2 xp, bool inside, char* dst)
+template <int CIN, int COUT, int EPI>
+__global__ __launch_bounds__(COUT / 32 * 64) void sg_conv_kernel(int N, const __bf16* __restrict__ X,
+                                                                 const __bf16* __restrict__ W,
+                                                                 const float* __restrict__ bias,
+                                                                 __bf16* __restrict__ Y, float* __restrict__ Yf,
+                                                                 const __bf16* __restrict__ xp)
 {
-    const __bf16* y = reinterpret_cast<const __bf16*>(&xp);
-    f4 z;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        if (MODE == SG_FWD) {
-            z[v] = sg_tanh(acc[v]);
-        } else {
-            const float yv = (float)y[v];
-            z[v] = acc[v] * fmaf(-yv, yv, 1.0f);
-        }
-    }
-    uint2 r = __builtin_bit_cast(uint2, __builtin_convertvector(z, bf16x4));
-    if (!inside) r = make_uint2(0u, 0u);
-    *reinterpret_cast<uint2*>(dst) = r;
-}
-
-template <int MODE, bool STORE>
-__global__ __launch_bounds__(512) void sg_chain_kernel(SgChainArgs p)
-{
-    __shared__ __attribute__((aligned(16))) char buf[2][(CH_WMAX + 2 * SG_HALO) * 128];
-    __shared__ __bf16 plane[SG_IN][CH_WMAX + 4 * SG_HALO];  // inputs of sites -8 .. W + 7
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = lane & 15, g = lane >> 4;
-    const int cw = w & 3, rg = w >> 2;  // this wavefront's channels and rows
-    const int N = p.N, T = p.T, R = p.R, W = 16 * R;
+    constexpr int NT = COUT / 32 * 64;  // threads
+    constexpr int ROWS = SG_TILE + 2 * SG_HALO;
+    // LDS rows: 64 channels (eight 16-byte chunks) are stored with chunk c of
+    // row r at chunk c ^ (r & 7), so that the 16 rows of an operand fragment
+    // read 16 distinct bank groups; narrower rows are padded by 16 bytes
+    constexpr bool SW = CIN == 64;
+    constexpr int RS = SW ? CIN : CIN + 8;  // row stride (elements)
+    constexpr int V8 = CIN / 8;
+    constexpr int KC = CIN / 32;  // 32-channel k blocks
+    __shared__ __attribute__((aligned(16))) __bf16 xs[ROWS * RS];
     const int b = blockIdx.y;
-    const int n0 = blockIdx.x * T, nw = n0 - CH_HALO;  // first site of the tile and of the window
-    const size_t base = (size_t)b * N;
-    // ---- inputs
-    for (int k = tid; k < W + 4 * SG_HALO; k += 512) {
-        const int n = nw - 2 * SG_HALO + k;
-        const bool in = n >= 0 && n < N;
-        const int nc = min(max(n, 0), N - 1);
-        __bf16 v0 = (__bf16)0.0f, v1 = v0, v2 = v0;
-        if (MODE == SG_BWD) {
-            v0 = p.dq[base + nc];
-        } else {
-            v0 = (__bf16)(float)(p.in[base + nc] * 2.0);
-            if (MODE == SG_FWD) {
-                v1 = (__bf16)expf(-(float)min(nc, N - 1 - nc) * 0.0625f);
-                v2 = (__bf16)(float)(p.feat ? p.feat[b] : 0.0);
+    const int n0 = blockIdx.x * SG_TILE;
+    const int lane = threadIdx.x & 63;
+    const int w = threadIdx.x >> 6;
+    const int i = lane & 15, g = lane >> 4;
+    // stage rows n0 - 4 .. n0 + SG_TILE + 3 of the sample, eight loads in flight per thread
+    const __bf16* xb = X + (size_t)b * N * CIN;
+    constexpr int TOT = ROWS * V8, PER = (TOT + NT - 1) / NT, CH = 8;
+#pragma unroll
+    for (int q0 = 0; q0 < PER; q0 += CH) {
+        bf16x8 v[CH];
+#pragma unroll
+        for (int q = 0; q < CH; ++q) {
+            const int idx = threadIdx.x + (q0 + q) * NT;
+            const int r = idx / V8, c8 = idx - r * V8;
+            const int n = min(max(n0 - SG_HALO + r, 0), N - 1);  // clamped; rows outside the sample are zeroed below
+            v[q] = *reinterpret_cast<const bf16x8*>(xb + (size_t)n * CIN + c8 * 8);
+        }
+#pragma unroll
+        for (int q = 0; q < CH; ++q) {
+            const int idx = threadIdx.x + (q0 + q) * NT;
+            if (q0 + q < PER && idx < TOT) {
+                const int r = idx / V8, c8 = idx - r * V8;
+                const int n = n0 - SG_HALO + r;
+                if (n < 0 || n >= N) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[q][e] = (__bf16)0.0f;
+                }
+                *reinterpret_cast<bf16x8*>(xs + r * RS + (SW ? (c8 ^ (r & 7)) : c8) * 8) = v[q];
             }
         }
-        plane[0][k] = in ? v0 : (__bf16)0.0f;
-        plane[1][k] = in ? v1 : (__bf16)0.0f;
-        plane[2][k] = in ? v2 : (__bf16)0.0f;
     }
-    // first layer's weights: k = 8 g + e is tap e of input g (g < 3), and tap 8 of input e (g = 3)
-    bf16x8 a0;
-    {
-        const __bf16* w0 = p.w[0] + (size_t)(16 * cw + i) * SG_KW * SG_CP;
+    // this wavefront's weight fragments (after the staging, whose buffers are dead now)
+    bf16x8 a[2][SG_KW][KC];
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            a0[e] = g < 3 ? w0[e * SG_CP + g] : e < 3 ? w0[8 * SG_CP + e] : (__bf16)0.0f;
-    }
-    bf16x8 a[SG_KW][2], an[SG_KW][2];
-    auto load_w = [&](const __bf16* wl, bf16x8 (&d)[SG_KW][2]) {
-        const __bf16* wr = wl + (size_t)(16 * cw + i) * SG_KW * SG_C + 8 * g;
+    for (int h = 0; h < 2; ++h) {
+        const __bf16* wrow = W + (size_t)(w * 32 + h * 16 + i) * SG_KW * CIN + 8 * g;
 #pragma unroll
-        for (int t = 0; t < SG_KW; ++t)
+        for (int tap = 0; tap < SG_KW; ++tap)
 #pragma unroll
-            for (int k = 0; k < 2; ++k) d[t][k] = *reinterpret_cast<const bf16x8*>(wr + t * SG_C + 32 * k);
-    };
-    load_w(p.w[1], a);
-    // the four sites beyond each end of buffer 0 stay zero (buffer 1: below)
-    auto zero_ends = [&](char* bf) {
-        if (tid < 64) {
-            const int s = tid >> 3, c = tid & 7;  // sites -4 .. -1, W .. W + 3
-            *reinterpret_cast<uint4*>(bf + (s < 4 ? s : W + s) * 128 + c * 16) = make_uint4(0u, 0u, 0u, 0u);
-        }
-    };
-    zero_ends(buf[0]);
-    __syncthreads();
-    // im2col of the first layer in buffer 1: site s at 64 s bytes, chunk g at g ^ (s / R mod 4)
-    for (int s = tid; s < W; s += 512) {
-        __attribute__((aligned(16))) __bf16 col[32];
-#pragma unroll
-        for (int gg = 0; gg < 3; ++gg)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) col[8 * gg + e] = plane[gg][s + SG_HALO + e];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) col[24 + e] = e < 3 ? plane[e][s + SG_HALO + 8] : (__bf16)0.0f;
-        const int f = (s / R) & 3;
-#pragma unroll
-        for (int gg = 0; gg < 4; ++gg)
-            *reinterpret_cast<uint4*>(buf[1] + s * 64 + ((gg ^ f) << 4)) = reinterpret_cast<const uint4*>(col)[gg];
+            for (int kc = 0; kc < KC; ++kc) a[h][tap][kc] = *reinterpret_cast<const bf16x8*>(wrow + tap * CIN + kc * 32);
     }
     __syncthreads();
-    const int olo = (4 + R * i) * 128 + ((g ^ ((i - 1) & 7)) << 4);
-    const int omid = (4 + R * i) * 128 + ((g ^ (i & 7)) << 4);
-    const int ohi = (4 + R * i) * 128 + ((g ^ ((i + 1) & 7)) << 4);
-    const int half = (R + 1) >> 1;
-    const int rb = rg ? half : 0, re = rg ? R : half;  // this wavefront's rows
-    const int ch = 16 * cw + 4 * g;                    // this lane's first output channel
-    const int dst0 = (4 + R * i) * 128 + (((2 * cw + (g >> 1)) ^ (i & 7)) << 4) + (g & 1) * 8;
-    // step st makes layer output x_{st+1} (forward, tangent) or dz_{4-st}; the x it is scaled with:
-    auto scale_src = [&](int st) { return p.x[MODE == SG_BWD ? SG_LAYERS - 1 - st : st + 1]; };
-    auto load_xp = [&](const __bf16* xs, int r) {
-        if (MODE == SG_FWD) return make_uint2(0u, 0u);
-        const int n = min(max(nw + r + R * i, 0), N - 1);
-        return *reinterpret_cast<const uint2*>(xs + (base + n) * SG_C + ch);
-    };
-    f4 bias0 = f4{0.f, 0.f, 0.f, 0.f};
-    auto load_bias = [&](int st) {
-        if (MODE == SG_FWD) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) bias0[v] = p.bias[st][ch + v];
-        }
-    };
-    auto inside = [&](int r) { return (unsigned)(nw + r + R * i) < (unsigned)N; };
-    // ---- first layer
-    load_bias(0);
-    {
-        const __bf16* xs = MODE == SG_FWD ? nullptr : scale_src(0);
-        for (int r = rb; r < re; ++r) {
-            const uint2 xp = load_xp(xs, r);
-            const int s = r + R * i;
-            const bf16x8 bb = *reinterpret_cast<const bf16x8*>(buf[1] + s * 64 + ((g ^ (i & 3)) << 4));
-            const f4 acc = mfma_bf16(a0, bb, bias0);
-            ch_store<MODE>(acc, xp, inside(r), buf[0] + r * 128 + dst0);
-        }
-    }
-    __syncthreads();
-    zero_ends(buf[1]);
-    __syncthreads();
-    // the tile's sites of a buffer to memory, whole lines
-    auto write_out = [&](const char* src, __bf16* dst) {
-        const int nt = min(T, N - n0);
-        for (int k = tid; k < nt * 8; k += 512) {
-            const int t = k >> 3, c = k & 7, s = CH_HALO + t;
-            const uint4 v = *reinterpret_cast<const uint4*>(src + (s + 4) * 128 + ((c ^ ((s / R) & 7)) << 4));
-            *reinterpret_cast<uint4*>(dst + (base + n0 + t) * SG_C + c * 8) = v;
-        }
-    };
-    // ---- hidden layers
+    // two site tiles at a time: four independent accumulators per lane
 #pragma unroll 1
-    for (int st = 1; st < SG_LAYERS - 1; ++st) {
-        const char* src = buf[(st + 1) & 1];
-        char* dst = buf[st & 1];
-        if (st + 1 < SG_LAYERS - 1) load_w(p.w[st + 1], an);
-        if (STORE) write_out(src, MODE == SG_BWD ? p.dz[SG_LAYERS - 1 - st] : p.x[st]);
-        load_bias(st);
-        const __bf16* xs = MODE == SG_FWD ? nullptr : scale_src(st);
-        auto pass = [&](auto u_c, int r0) {
-            constexpr int U = decltype(u_c)::value;
-            ChOut<U> o;
-            uint2 xp[U];
+    for (int t0 = 0; t0 < SG_TILE / 16; t0 += 2) {
+        f4 acc[2][2];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                o.acc[u] = bias0;
-                xp[u] = load_xp(xs, r0 + u);
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) acc[h][u] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int tap = 0; tap < SG_KW; ++tap) {
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    // site n0 + 16 (t0 + u) + i + tap - 4 is staged row 16 (t0 + u) + i + tap
+                    const int row = 16 * (t0 + u) + i + tap, c8 = kc * 4 + g;
+                    const bf16x8 bb =
+                        *reinterpret_cast<const bf16x8*>(xs + row * RS + (SW ? (c8 ^ (row & 7)) : c8) * 8);
+                    acc[0][u] = mfma_bf16(a[0][tap][kc], bb, acc[0][u]);
+                    acc[1][u] = mfma_bf16(a[1][tap][kc], bb, acc[1][u]);
+                }
             }
-            ch_rows<U>(src, olo, omid, ohi, r0, R, a, o);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                ch_store<MODE>(o.acc[u], xp[u], inside(r0 + u), dst + (r0 + u) * 128 + dst0);
-        };
-        int r = rb;
-#pragma unroll 1
-        for (; r + 8 <= re; r += 8) pass(std::integral_constant<int, 8>(), r);
-        if (r + 4 <= re) {
-            pass(std::integral_constant<int, 4>(), r);
-            r += 4;
         }
-        if (r + 2 <= re) {
-            pass(std::integral_constant<int, 2>(), r);
-            r += 2;
-        }
-        if (r < re) pass(std::integral_constant<int, 1>(), r);
 #pragma unroll
-        for (int t = 0; t < SG_KW; ++t)
+        for (int u = 0; u < 2; ++u) {
+            const int n = n0 + 16 * (t0 + u) + i;
+            if (n >= N) continue;
+            const size_t site = (size_t)b * N + n;
 #pragma unroll
-            for (int k = 0; k < 2; ++k) a[t][k] = an[t][k];
-        __syncthreads();
-    }
-    const char* last = buf[0];
-    if (STORE) write_out(last, MODE == SG_BWD ? p.dz[0] : p.x[SG_LAYERS - 1]);
-    if (MODE == SG_BWD) return;
-    // ---- last layer: z[tap][s] into buffer 1, then the nine shifted sums
-    float* z = reinterpret_cast<float*>(buf[1]);
-    bf16x8 a5[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(p.w[SG_LAYERS - 1] + (size_t)min(i, SG_KW - 1) * SG_C + 32 * k + 8 * g);
-        bf16x8 zero;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) zero[e] = (__bf16)0.0f;
-        a5[k] = i < SG_KW ? v : zero;
-    }
-    for (int r = w; r < R; r += 8) {
-        const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(last + r * 128 + omid);
-        const bf16x8 b1 = *reinterpret_cast<const bf16x8*>(last + r * 128 + (omid ^ 64));
-        f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-        acc = mfma_bf16(a5[0], b0, acc);
-        acc = mfma_bf16(a5[1], b1, acc);
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            if (4 * g + v < SG_KW) z[(4 * g + v) * CH_WMAX + r + R * i] = acc[v];
-    }
-    __syncthreads();
-    const float b5 = MODE == SG_FWD ? p.bias[SG_LAYERS - 1][0] : 0.0f;
-    for (int t = tid; t < min(T, N - n0); t += 512) {
-        float qv = b5;
-#pragma unroll
-        for (int tap = 0; tap < SG_KW; ++tap) qv += z[tap * CH_WMAX + CH_HALO + t + tap - SG_HALO];
-        const size_t o = base + n0 + t;
-        if (p.q) p.q[o] = qv;
-        if (p.Q) p.Q[o] = p.mean + p.scale * (double)qv;
-    }
-}
-
-// Tile length: the one that keeps the CUs (one workgroup each) busy with the
-// fewest rows in all, rounds of workgroups x rows per wavefront.
-static void chain_tile(int N, int B, int* T, int* R)
-{
-    const int cus = 256;
-    long long best = -1;
-    for (int tiles = 1; tiles <= (N + 15) / 16; ++tiles) {
-        // (a shift of four sites must stay within one row of the next lane: r >= 4)
-        const int t = (N + tiles - 1) / tiles, r = std::max(4, (t + 2 * CH_HALO + 15) / 16);
-        if (r > CH_RMAX) continue;
-        const long long rounds = ((long long)tiles * B + cus - 1) / cus;
-        const long long cost = rounds * ((r + 1) / 2 + 3);  // 3: the fixed part of a workgroup, in rows
-        if (best < 0 || cost < best) {
-            best = cost;
-            *T = t;
-            *R = r;
+            for (int h = 0; h < 2; ++h) sg_epilogue<EPI>(acc[h][u], w * 32 + h * 16 + 4 * g, site, COUT, bias, Y, Yf, xp);
         }
     }
 }
@@ -390,7 +205,7 @@ static void chain_tile(int N, int B, int* T, int* R)
 // inputs x 9 taps as the 27 columns of two tiles) and the last (9 taps as the
 // rows, one output channel).  Each workgroup walks a run of chunks and writes
 // one partial copy; sg_wreduce_kernel sums the copies in order.
-// At 32 x 2048 sites all six layers take 37 us (MFMA time 9 us; the rest is
+// At 32 x 2048 sites all six layers take 50 us (MFMA time 9 us; the rest is
 // the global loads and transposes of each chunk, three workgroups per CU
 // covering for each other) and the sum of the copies 7 us.  One launch per
 // layer with 2-byte transposing loads and a serial bias sum took 4.7 ms.
@@ -403,11 +218,8 @@ constexpr int WG_GROUPS = 42;            // partial copies at most: 18 jobs x 42
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 
 struct SgWgradArgs {
-    const __bf16* dz[SG_LAYERS];  // gradient at layer l's output [site][64], l < 5
-    const __bf16* x[SG_LAYERS];   // hidden layer l's input [site][64]
-    const __bf16* dq;             // gradient at the output [site]
-    const double* U;              // the potentials and features of the first layer's inputs
-    const double* feat;
+    const __bf16* dz[SG_LAYERS];  // gradient at layer l's output [site][cout]
+    const __bf16* x[SG_LAYERS];   // layer l's input [site][cin]
     int woff[SG_LAYERS], boff[SG_LAYERS];
     int N, cps, nchunks, per;     // sites and chunks per sample, chunks, chunks per workgroup
     int nparam;
@@ -450,7 +262,6 @@ __global__ __launch_bounds__(256, 3) void sg_wgrad_kernel(SgWgradArgs a)
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i = lane & 15, g = lane >> 4;
     const int c0 = blockIdx.x * a.per, c1 = min(a.nchunks, c0 + a.per);
-    if (c0 >= c1) return;  // (the grid is rounded up: see the launch)
     const int N = a.N;
     float* P = a.P + (size_t)blockIdx.x * a.nparam;
     // wide tile: thread = (row tid / 8, channel octet tid % 8); the octet's number
@@ -526,6 +337,7 @@ __global__ __launch_bounds__(256, 3) void sg_wgrad_kernel(SgWgradArgs a)
     const bool first = job == WG_JOBS - 2;
     const int l = first ? 0 : SG_LAYERS - 1;
     const __bf16* wsr = first ? a.dz[0] : a.x[SG_LAYERS - 1];
+    const __bf16* psr = first ? a.x[0] : a.dz[SG_LAYERS - 1];
     const int np = first ? SG_IN : 1;
     u32x4 vw[8];
     f4 acc[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}}, accb = acc[0];
@@ -543,16 +355,7 @@ __global__ __launch_bounds__(256, 3) void sg_wgrad_kernel(SgWgradArgs a)
         for (int q = tid; q < np * WG_XR * 8; q += 256) {
             const int p = q / (WG_XR * 8), r = q - p * WG_XR * 8, row = r >> 3, e = r & 7;
             const int n = n0 + row - SG_HALO + WG_R * e;
-            const int nc = min(max(n, 0), N - 1);
-            __bf16 v;
-            if (!first)
-                v = a.dq[(size_t)b * N + nc];
-            else if (p == 0)
-                v = (__bf16)(float)(a.U[(size_t)b * N + nc] * 2.0);
-            else if (p == 1)
-                v = (__bf16)expf(-(float)min(nc, N - 1 - nc) * 0.0625f);
-            else
-                v = (__bf16)(float)(a.feat ? a.feat[b] : 0.0);
+            const __bf16 v = psr[((size_t)b * N + min(max(n, 0), N - 1)) * SG_CP + p];
             halo[q] = n >= 0 && n < N ? v : (__bf16)0.0f;
         }
         __syncthreads();
@@ -605,6 +408,39 @@ __global__ __launch_bounds__(256) void sg_wreduce_kernel(int ncopies, SgWgradArg
     out[j] = s;
 }
 
+__global__ void sg_input_kernel(int N, long long total, const double* __restrict__ U,
+                                const double* __restrict__ feat, __bf16* __restrict__ X0)
+{
+    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= total) return;
+    const long long b = q / N;
+    const int n = (int)(q - b * N);
+    __attribute__((aligned(16))) __bf16 x[SG_CP];
+#pragma unroll
+    for (int c = 0; c < SG_CP; ++c) x[c] = (__bf16)0.0f;
+    x[0] = (__bf16)(float)(U[q] * 2.0);
+    const int d = min(n, N - 1 - n);
+    x[1] = (__bf16)expf(-(float)d * 0.0625f);
+    x[2] = (__bf16)(float)(feat ? feat[b] : 0.0);
+    bf16x8* dst = reinterpret_cast<bf16x8*>(X0 + q * SG_CP);
+#pragma unroll
+    for (int c8 = 0; c8 < SG_CP / 8; ++c8) dst[c8] = reinterpret_cast<const bf16x8*>(x)[c8];
+}
+
+// tangent of the input: channel 0 = 2 V (per eV), other channels 0
+__global__ void sg_tangent_input_kernel(long long total, const double* __restrict__ V, __bf16* __restrict__ T0)
+{
+    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= total) return;
+    __attribute__((aligned(16))) __bf16 x[SG_CP];
+#pragma unroll
+    for (int c = 0; c < SG_CP; ++c) x[c] = (__bf16)0.0f;
+    x[0] = (__bf16)(float)(V[q] * 2.0);
+    bf16x8* dst = reinterpret_cast<bf16x8*>(T0 + q * SG_CP);
+#pragma unroll
+    for (int c8 = 0; c8 < SG_CP / 8; ++c8) dst[c8] = reinterpret_cast<const bf16x8*>(x)[c8];
+}
+
 __global__ void sg_output_kernel(long long n, const float* __restrict__ q, double mean, double scale,
                                  double* __restrict__ Q)
 {
@@ -612,8 +448,8 @@ __global__ void sg_output_kernel(long long n, const float* __restrict__ q, doubl
     if (i < n) Q[i] = mean + scale * (double)q[i];
 }
 
-// Mean squared error of the normalised output; dq = 2 (q - t) / n; one partial
-// sum per block.
+// Mean squared error of the normalised output; dq = 2 (q - t) / n in
+// channel 0 of the padded gradient buffer; one partial sum per block.
 __global__ __launch_bounds__(256) void sg_loss_kernel(long long n, const float* __restrict__ q,
                                                       const double* __restrict__ Qt, double mean, double inv_scale,
                                                       __bf16* __restrict__ dq, float* __restrict__ part)
@@ -625,7 +461,13 @@ __global__ __launch_bounds__(256) void sg_loss_kernel(long long n, const float* 
         const float t = (float)((Qt[i] - mean) * inv_scale);
         const float d = q[i] - t;
         l = d * d;
-        dq[i] = (__bf16)(2.0f * d / (float)n);
+        __attribute__((aligned(16))) __bf16 x[SG_CP];
+#pragma unroll
+        for (int c = 0; c < SG_CP; ++c) x[c] = (__bf16)0.0f;
+        x[0] = (__bf16)(2.0f * d / (float)n);
+        bf16x8* dst = reinterpret_cast<bf16x8*>(dq + i * SG_CP);
+#pragma unroll
+        for (int c8 = 0; c8 < SG_CP / 8; ++c8) dst[c8] = reinterpret_cast<const bf16x8*>(x)[c8];
     }
     red[threadIdx.x] = l;
     __syncthreads();
@@ -744,93 +586,50 @@ int Surrogate::ensure_batch(int B)
     if (B <= capB) return NEGF_OK;
     int rc;
     const size_t sites = (size_t)B * N;
-    for (int l = 1; l < SG_LAYERS; ++l)
-        if ((rc = d_act[l].ensure(2 * sites * SG_C))) return rc;
+    for (int l = 0; l < SG_LAYERS; ++l)
+        if ((rc = d_act[l].ensure(2 * sites * sg_cin(l)))) return rc;
     if ((rc = d_act[SG_LAYERS].ensure(sizeof(float) * sites))) return rc;
+    for (int l = 0; l < 2; ++l)
+        if ((rc = d_dz[l].ensure(2 * sites * SG_C))) return rc;
     capB = B;
     return NEGF_OK;
 }
 
-template <int MODE, bool STORE>
-static int chain(SgChainArgs& p, int N, int B, hipStream_t s)
+template <int CIN, int COUT, int EPI>
+static void conv(int N, int B, const __bf16* X, const __bf16* W, const float* bias, __bf16* Y, float* Yf,
+                 const __bf16* xp, hipStream_t s)
 {
-    p.N = N;
-    chain_tile(N, B, &p.T, &p.R);
-    // samples along y, at most 65535 at a time
-    for (int b0 = 0; b0 < B; b0 += 65535) {
-        SgChainArgs q = p;
-        const size_t o = (size_t)b0 * N;
-        if (q.in) q.in += o;
-        if (q.feat) q.feat += b0;
-        if (q.dq) q.dq += o;
-        if (q.q) q.q += o;
-        if (q.Q) q.Q += o;
-        for (int l = 0; l < SG_LAYERS; ++l) {
-            if (q.x[l]) q.x[l] += o * SG_C;
-            if (q.dz[l]) q.dz[l] += o * SG_C;
-        }
-        hipLaunchKernelGGL((sg_chain_kernel<MODE, STORE>), dim3((N + p.T - 1) / p.T, std::min(B - b0, 65535)), dim3(512),
-                           0, s, q);
-    }
-    NEGF_HIP_TRY(hipGetLastError());
-    return NEGF_OK;
-}
-
-// arguments common to the passes: weights of the layers in the order of the steps
-static SgChainArgs chain_args(Surrogate& g, bool backward)
-{
-    SgChainArgs p;
-    std::memset(&p, 0, sizeof(p));
-    for (int st = 0; st < SG_LAYERS; ++st) {
-        const int l = backward ? SG_LAYERS - 1 - st : st;
-        p.w[st] = (backward ? g.d_wt : g.d_wb).as<__bf16>() + g.woff[l];
-        p.bias[st] = g.d_w.as<float>() + g.boff[l];
-    }
-    return p;
+    dim3 g((N + SG_TILE - 1) / SG_TILE, B);
+    hipLaunchKernelGGL((sg_conv_kernel<CIN, COUT, EPI>), g, dim3(COUT / 32 * 64), 0, s, N, X, W, bias, Y, Yf, xp);
 }
 
 int Surrogate::forward(int B, const double* dU, const double* dfeat, hipStream_t s)
 {
     int rc;
     if ((rc = ensure_batch(B))) return rc;
-    SgChainArgs p = chain_args(*this, false);
-    p.in = dU;
-    p.feat = dfeat;
-    for (int l = 1; l < SG_LAYERS; ++l) p.x[l] = d_act[l].as<__bf16>();
-    p.q = d_act[SG_LAYERS].as<float>();
-    return chain<SG_FWD, true>(p, N, B, s);
-}
-
-// The pass's output as doubles.  A tile reads its neighbours' inputs, so an
-// output that overlaps the inputs goes through the float buffer.
-template <int MODE>
-int Surrogate::chain_to(SgChainArgs& p, int B, double mean, double* dQ, hipStream_t s)
-{
-    const long long n = (long long)B * N;
-    const double* lo = dQ;
-    const double* hi = dQ + n;
-    const bool overlap = (p.in < hi && lo < p.in + n) || (p.feat && p.feat < hi && lo < p.feat + B);
-    p.mean = mean;
-    p.scale = scale_Q;
-    if (!overlap) {
-        p.Q = dQ;
-        return chain<MODE, false>(p, N, B, s);
-    }
-    int rc;
-    if ((rc = d_act[SG_LAYERS].ensure(sizeof(float) * (size_t)n))) return rc;
-    p.q = d_act[SG_LAYERS].as<float>();
-    if ((rc = chain<MODE, false>(p, N, B, s))) return rc;
-    hipLaunchKernelGGL(sg_output_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, p.q, mean, scale_Q, dQ);
+    const long long sites = (long long)B * N;
+    hipLaunchKernelGGL(sg_input_kernel, dim3((unsigned)((sites + 255) / 256)), dim3(256), 0, s, N, sites, dU, dfeat,
+                       d_act[0].as<__bf16>());
+    const __bf16* wb = d_wb.as<__bf16>();
+    const float* w = d_w.as<float>();
+    conv<SG_CP, SG_C, EPI_TANH>(N, B, d_act[0].as<__bf16>(), wb + woff[0], w + boff[0], d_act[1].as<__bf16>(),
+                                nullptr, nullptr, s);
+    for (int l = 1; l < SG_LAYERS - 1; ++l)
+        conv<SG_C, SG_C, EPI_TANH>(N, B, d_act[l].as<__bf16>(), wb + woff[l], w + boff[l],
+                                   d_act[l + 1].as<__bf16>(), nullptr, nullptr, s);
+    conv<SG_C, SG_CP, EPI_LINEAR_OUT>(N, B, d_act[SG_LAYERS - 1].as<__bf16>(), wb + woff[SG_LAYERS - 1],
+                                      w + boff[SG_LAYERS - 1], nullptr, d_act[SG_LAYERS].as<float>(), nullptr, s);
     NEGF_HIP_TRY(hipGetLastError());
     return NEGF_OK;
 }
 
-int Surrogate::evaluate(int B, const double* dU, const double* dfeat, double* dQ, hipStream_t s)
+int Surrogate::output(int B, double* dQ, hipStream_t s)
 {
-    SgChainArgs p = chain_args(*this, false);
-    p.in = dU;
-    p.feat = dfeat;
-    return chain_to<SG_FWD>(p, B, mean_Q, dQ, s);
+    const long long n = (long long)B * N;
+    hipLaunchKernelGGL(sg_output_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n,
+                       d_act[SG_LAYERS].as<float>(), mean_Q, scale_Q, dQ);
+    NEGF_HIP_TRY(hipGetLastError());
+    return NEGF_OK;
 }
 
 // forward-mode tangent: t_{l+1} = conv(W_l, t_l) (1 - x_{l+1}^2), dq = conv(W_5, t_5)
@@ -840,39 +639,53 @@ int Surrogate::jvp(int B, const double* dV, double* dout, hipStream_t s)
         set_error("surrogate tangent needs a forward of at least %d samples first", B);
         return NEGF_EARG;
     }
-    SgChainArgs p = chain_args(*this, false);
-    p.in = dV;
-    for (int l = 1; l < SG_LAYERS; ++l) p.x[l] = d_act[l].as<__bf16>();
-    return chain_to<SG_TAN>(p, B, 0.0, dout, s);
+    const long long sites = (long long)B * N;
+    __bf16* t0 = d_dz[0].as<__bf16>();
+    __bf16* t1 = d_dz[1].as<__bf16>();
+    hipLaunchKernelGGL(sg_tangent_input_kernel, dim3((unsigned)((sites + 255) / 256)), dim3(256), 0, s, sites, dV,
+                       t0);
+    const __bf16* wb = d_wb.as<__bf16>();
+    conv<SG_CP, SG_C, EPI_DTANH>(N, B, t0, wb + woff[0], nullptr, t1, nullptr, d_act[1].as<__bf16>(), s);
+    for (int l = 1; l < SG_LAYERS - 1; ++l) {
+        conv<SG_C, SG_C, EPI_DTANH>(N, B, t1, wb + woff[l], nullptr, t0, nullptr, d_act[l + 1].as<__bf16>(), s);
+        std::swap(t0, t1);
+    }
+    float* q = d_act[SG_LAYERS].as<float>();  // the forward output is consumed; the tangent reuses it
+    conv<SG_C, SG_CP, EPI_LINEAR_OUT>(N, B, t1, wb + woff[SG_LAYERS - 1], nullptr, nullptr, q, nullptr, s);
+    hipLaunchKernelGGL(sg_output_kernel, dim3((unsigned)((sites + 255) / 256)), dim3(256), 0, s, sites, q, 0.0,
+                       scale_Q, dout);
+    NEGF_HIP_TRY(hipGetLastError());
+    return NEGF_OK;
 }
 
-int Surrogate::backward(int B, const double* dU, const double* dfeat, const double* dQt, double* loss, hipStream_t s)
+int Surrogate::backward(int B, const double* dQt, double* loss, hipStream_t s)
 {
     int rc;
     const long long sites = (long long)B * N;
     const int lblocks = (int)((sites + 255) / 256);
     if ((rc = d_loss.ensure(sizeof(float) * lblocks))) return rc;
     for (int l = 0; l < SG_LAYERS; ++l)
-        if ((rc = d_dz[l].ensure(2 * (size_t)sites * (l == SG_LAYERS - 1 ? 1 : SG_C)))) return rc;
-    __bf16* dq = d_dz[SG_LAYERS - 1].as<__bf16>();
+        if ((rc = d_dz[l].ensure(2 * (size_t)sites * sg_cout(l)))) return rc;
     hipLaunchKernelGGL(sg_loss_kernel, dim3(lblocks), dim3(256), 0, s, sites, d_act[SG_LAYERS].as<float>(), dQt,
-                       mean_Q, 1.0 / scale_Q, dq, d_loss.as<float>());
-    // data gradients of layers 5..1, kept for the one launch that forms all weight gradients
-    SgChainArgs p = chain_args(*this, true);
-    p.dq = dq;
-    for (int l = 1; l < SG_LAYERS; ++l) p.x[l] = d_act[l].as<__bf16>();
-    for (int l = 0; l < SG_LAYERS - 1; ++l) p.dz[l] = d_dz[l].as<__bf16>();
-    if ((rc = chain<SG_BWD, true>(p, N, B, s))) return rc;
+                       mean_Q, 1.0 / scale_Q, d_dz[SG_LAYERS - 1].as<__bf16>(), d_loss.as<float>());
+    // every layer's gradient stays until the one launch that forms all weight gradients
+    for (int l = SG_LAYERS - 1; l > 0; --l) {
+        // data gradient into layer l's input, through the tanh that made it
+        const __bf16* wt = d_wt.as<__bf16>() + woff[l];
+        if (l == SG_LAYERS - 1)
+            conv<SG_CP, SG_C, EPI_DTANH>(N, B, d_dz[l].as<__bf16>(), wt, nullptr, d_dz[l - 1].as<__bf16>(), nullptr,
+                                         d_act[l].as<__bf16>(), s);
+        else
+            conv<SG_C, SG_C, EPI_DTANH>(N, B, d_dz[l].as<__bf16>(), wt, nullptr, d_dz[l - 1].as<__bf16>(), nullptr,
+                                        d_act[l].as<__bf16>(), s);
+    }
     SgWgradArgs a;
     for (int l = 0; l < SG_LAYERS; ++l) {
-        a.dz[l] = l < SG_LAYERS - 1 ? d_dz[l].as<__bf16>() : nullptr;
-        a.x[l] = l > 0 ? d_act[l].as<__bf16>() : nullptr;
+        a.dz[l] = d_dz[l].as<__bf16>();
+        a.x[l] = d_act[l].as<__bf16>();
         a.woff[l] = woff[l];
         a.boff[l] = boff[l];
     }
-    a.dq = dq;
-    a.U = dU;
-    a.feat = dfeat;
     a.N = N;
     a.cps = (N + WG_SITES - 1) / WG_SITES;
     a.nchunks = B * a.cps;
@@ -881,10 +694,7 @@ int Surrogate::backward(int B, const double* dU, const double* dfeat, const doub
     const int copies = (a.nchunks + a.per - 1) / a.per;
     if ((rc = d_part.ensure(sizeof(float) * (size_t)copies * nparam))) return rc;
     a.P = d_part.as<float>();
-    // Workgroups go to the eight XCDs in turn: with a multiple of eight runs, the
-    // jobs of one run share an XCD and find each other's chunks in its L2
-    // (37 against 48 us at 32 x 2048 sites).
-    hipLaunchKernelGGL(sg_wgrad_kernel, dim3((copies + 7) / 8 * 8, WG_JOBS), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(sg_wgrad_kernel, dim3(copies, WG_JOBS), dim3(256), 0, s, a);
     hipLaunchKernelGGL(sg_wreduce_kernel, dim3((nparam + 255) / 256), dim3(256), 0, s, copies, a, d_g.as<float>());
     NEGF_HIP_TRY(hipGetLastError());
     if (loss) {
@@ -991,7 +801,9 @@ int negf_surrogate_forward(negf_surrogate* s, int B, const double* d_U, const do
         return NEGF_EARG;
     }
     hipStream_t st = stream ? (hipStream_t)stream : s->s.st;
-    return s->s.evaluate(B, d_U, d_feat, d_Q, st);
+    int rc = s->s.forward(B, d_U, d_feat, st);
+    if (!rc) rc = s->s.output(B, d_Q, st);
+    return rc;
 }
 
 int negf_surrogate_jvp(negf_surrogate* s, int B, const double* d_U, const double* d_feat, const double* d_V,
@@ -1017,7 +829,7 @@ int negf_surrogate_gradient(negf_surrogate* s, int B, const double* d_U, const d
         return NEGF_EARG;
     }
     int rc = s->s.forward(B, d_U, d_feat, s->s.st);
-    if (!rc) rc = s->s.backward(B, d_U, d_feat, d_Q, loss, s->s.st);
+    if (!rc) rc = s->s.backward(B, d_Q, loss, s->s.st);
     if (rc) return rc;
     NEGF_HIP_TRY(hipStreamSynchronize(s->s.st));
     if (grad) NEGF_HIP_TRY(hipMemcpy(grad, s->s.d_g.p, sizeof(float) * s->s.nparam, hipMemcpyDeviceToHost));
@@ -1079,11 +891,9 @@ int negf_surrogate_train(negf_surrogate* s, int nsamples, const double* d_U, con
                                m.d_idx.as<int>() + (size_t)k * batch, d_U, d_Q, d_feat, m.d_bU.as<double>(),
                                m.d_bQ.as<double>(), m.d_bF.as<double>());
             NEGF_HIP_TRY(hipGetLastError());
-            const double* bF = d_feat ? m.d_bF.as<double>() : nullptr;
-            if ((rc = m.forward(batch, m.d_bU.as<double>(), bF, m.st))) return rc;
+            if ((rc = m.forward(batch, m.d_bU.as<double>(), d_feat ? m.d_bF.as<double>() : nullptr, m.st))) return rc;
             const bool want = (k == steps_per_epoch - 1) && last_loss;
-            if ((rc = m.backward(batch, m.d_bU.as<double>(), bF, m.d_bQ.as<double>(), want ? &l : nullptr, m.st)))
-                return rc;
+            if ((rc = m.backward(batch, m.d_bQ.as<double>(), want ? &l : nullptr, m.st))) return rc;
             const double frac = total_steps > 1 ? (double)step / (double)(total_steps - 1) : 1.0;
             if ((rc = m.adam((float)(lr + (lr_end - lr) * frac), m.st))) return rc;
             ++step;

@@ -114,46 +114,6 @@ def test_jvp_matches_cpu_model_and_differences(dev):
     sg.close()
 
 
-@pytest.mark.parametrize("N", [16, 17, 33, 200, 536, 537, 1100])
-def test_passes_do_not_depend_on_the_tiling(dev, N):
-    """One sample alone and the same among many get other tile lengths; a site's
-    sums run in the same order in every tile, so the results agree bit by bit.
-    Against the CPU model as above."""
-    sg = Surrogate(N, seed=5)
-    p = S.init_params(seed=N)
-    norm = np.array([0.02, 0.3])
-    sg.set_params(p, norm)
-    U, V = smooth_U(1, N, seed=N), smooth_U(1, N, seed=N + 1)
-    f1 = sg.forward(U, np.array([0.2])).cpu().numpy()
-    j1 = sg.jvp(U, V, np.array([0.2])).cpu().numpy()
-    for B in (5, 300):
-        Ub, Vb, fb = np.repeat(U, B, 0), np.repeat(V, B, 0), np.full(B, 0.2)
-        assert np.array_equal(sg.forward(Ub, fb).cpu().numpy(), np.repeat(f1, B, 0))
-        assert np.array_equal(sg.jvp(Ub, Vb, fb).cpu().numpy(), np.repeat(j1, B, 0))
-    Qc = norm[0] + norm[1] * S.forward(p, U, np.array([0.2]), bf=True)[0]
-    assert np.abs(f1 - Qc).max() / np.abs(Qc - norm[0]).max() < 2e-2
-    jc = S.jvp(p, U, V, norm[1], np.array([0.2]), bf=True)
-    assert np.abs(j1 - jc).max() / np.abs(jc).max() < 2e-2
-    sg.close()
-
-
-def test_forward_and_tangent_in_place(dev):
-    """The output may be the input's own array."""
-    from electrostatic_amd import _lib
-    from tests.gpu_util import ptr
-    N, B = 700, 3
-    sg = Surrogate(N, seed=6)
-    U = torch.as_tensor(smooth_U(B, N, seed=1), device="cuda")
-    V = torch.as_tensor(smooth_U(B, N, seed=2), device="cuda")
-    Q, J = sg.forward(U), sg.jvp(U, V)
-    Ui, Vi = U.clone(), V.clone()
-    _lib.check(sg.lib.negf_surrogate_jvp(sg.h, B, ptr(U), None, ptr(Vi), ptr(Vi), None))
-    _lib.check(sg.lib.negf_surrogate_forward(sg.h, B, ptr(Ui), None, ptr(Ui), None))
-    torch.cuda.synchronize()
-    assert torch.equal(Ui, Q) and torch.equal(Vi, J)
-    sg.close()
-
-
 def test_training_reduces_loss(dev):
     # a local, smooth target: Q = -0.2 tanh(3 (G * U)) + 0.05 f, G a Gaussian window
     N, Sn = 256, 256
