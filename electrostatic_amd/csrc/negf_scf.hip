@@ -699,8 +699,8 @@ struct TrackOut {
 // at most 16 rows, into eq; Q = (eq + noneq) - rho0), one Broyden update, and the
 // tube's record.  A tube whose max norm reached max_norm keeps its U and Q (Uo, Qo) and
 // leaves the active set, as does one at its step limit; the host applies the same
-// tests to the same values, so its bookkeeping follows without copies.  A norm that is
-// not finite stops every tube from the next iteration on (the host reports it).  The
+// tests to the same values, so its bookkeeping follows without copies.  A residual that
+// is not finite stops every tube from the next iteration on (the host reports it).  The
 // counters live on the device so that the launch is identical every iteration: steps[t]
 // the Broyden step, steps[T + t] the iteration, steps[2T] the first iteration that is not
 // to run (0: none), steps[2T + 1] the tubes still active (0 or less: the loop has
@@ -777,14 +777,16 @@ __global__ __launch_bounds__(kBroydenThreads) void broyden_batch_kernel(int S, i
     if (tid == 0) {  // b.out[0..2] were written by this thread
         if (!limit) steps[t] = m + 2;
         const double nrm = b.out[0];
+        // the max norm drops a NaN (it is a chain of fmax), |dF|^2 keeps it
+        const bool finite = isfinite(nrm) && isfinite(b.out[2]);
         b.out[3] = limit ? 1.0 : 0.0;  // step limit reached
         for (int k = 0; k < 3; ++k) rec[4 * t + k] = b.out[k];
         rec[4 * t + 3] = limit ? 1.0 : 0.0;
-        keep = !limit && nrm <= tr.max_norm;
+        keep = !limit && finite && nrm <= tr.max_norm;
         if (limit || keep) {
             active[t] = 0;
             atomicSub(&steps[2 * T + 1], 1);
-        } else if (!isfinite(nrm)) {
+        } else if (!finite) {
             steps[2 * T] = it + 1;
             atomicSub(&steps[2 * T + 1], T + 1);
         }
@@ -1062,7 +1064,7 @@ class BatchScf {
                 continue;
             }
             const double nrm = o[4 * t];
-            if (!std::isfinite(nrm)) {
+            if (!std::isfinite(nrm) || !std::isfinite(o[4 * t + 2])) {
                 set_error("batched SCF: non-finite Broyden norm for tube %d at iteration %d", t, it + 1);
                 return NEGF_ENAN;
             }
