@@ -199,14 +199,15 @@ __global__ __launch_bounds__(kMsThreads) void big_broyden_pass3(BigBroyden b, do
 
 __global__ void big_broyden_first_step(int* step) { *step = 1; }
 
-// The iteration's norms (coef[0..1]) and the batch plans' status words into
-// the host's mapped, coherent read-back record: no copy in the iteration.
+// The iteration's max norm and |dF|^2 (which keeps a NaN; the max norm, a chain of
+// fmax, drops it) and the batch plans' status words into the host's mapped,
+// coherent read-back record: no copy in the iteration.
 __global__ void multi_readback_kernel(const double* __restrict__ coef, const int* __restrict__ st_eq,
                                       const int* __restrict__ st_neq, double* __restrict__ back)
 {
     if (threadIdx.x == 0) {
         back[0] = coef[0];
-        back[1] = coef[1];
+        back[1] = coef[2];
         int* bs = reinterpret_cast<int*>(back + 2);
         bs[0] = *st_eq;
         bs[1] = st_neq ? *st_neq : 0;
@@ -400,7 +401,7 @@ class MultiScf {
         if ((rc = d_coef.ensure(sizeof(double) * (6 + 2 * (size_t)M)))) return rc;
         if ((rc = d_step.ensure(sizeof(int)))) return rc;
         {
-            // read-back record: 2 doubles (norms), then 2 status ints
+            // read-back record: 2 doubles (max norm, |dF|^2), then 2 status ints
             hipError_t eh = hipHostMalloc(&h_back, 2 * sizeof(double) + 2 * sizeof(int),
                                           hipHostMallocMapped | hipHostMallocCoherent);
             if (eh == hipSuccess) eh = hipHostGetDevicePointer(&d_back, h_back, 0);
@@ -476,7 +477,7 @@ class MultiScf {
         hipLaunchKernelGGL(big_broyden_pass2, dim3(1), dim3(kMsThreads), 0, st, bro(), nb);
         hipLaunchKernelGGL(big_broyden_pass3, dim3(nb), dim3(kMsThreads), 0, st, bro(), p.Broyden_fraction);
         NEGF_HIP_TRY(hipGetLastError());
-        // Broyden_Norm, the l2 norm and the plans' status words to the host
+        // Broyden_Norm, |dF|^2 and the plans' status words to the host
         const int* st_eq = nullptr;
         const int* st_neq = nullptr;
         batch_status_words(batch, &st_eq, &st_neq);
@@ -569,7 +570,7 @@ class MultiScf {
             if ((bs[0] | bs[1]) && (rc = batch_poll_status(batch))) break;
             norm = back[0];
             ++it;
-            if (!std::isfinite(norm)) {
+            if (!std::isfinite(norm) || !std::isfinite(back[1])) {
                 set_error("multi-tube SCF: non-finite Broyden norm at iteration %d", it);
                 rc = NEGF_ENAN;
                 break;

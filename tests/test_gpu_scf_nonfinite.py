@@ -1,4 +1,4 @@
-"""A gate voltage or charge that is not a number ends a batched self-consistent run with
+"""A gate voltage or charge that is not a number ends a self-consistent run of many tubes with
 the non-finite error, at the first iteration that meets it, and is never reported as
 converged (a maximum norm formed with fmax reads 0 there)."""
 import numpy as np
@@ -81,3 +81,16 @@ def test_preconditioned_run(dev, ahead):
             s.scf.run_surrogate(np.array([0.1, np.nan]), seed_iters=0, refresh_iter=0)
         assert e.value.code == ENAN
         sg.close()
+
+
+@pytest.mark.parametrize("graph", [True, False])
+@pytest.mark.parametrize("max_iters", [0, 3])
+def test_one_system_of_all_tubes(dev, graph, max_iters):
+    with Setup(3, 13) as s:
+        scf = negf.MultiScf(s.batch, Broyden_fraction=0.1, Broyden_max_norm=1e-6, Broyden_threshold_maxstep=200,
+                            eps_r=3.9, R_ring_nm=0.665, R_image_nm=10.0)
+        scf.use_graph(graph)
+        with pytest.raises(_lib.NegfError) as e:
+            scf.bias_point(np.array([0.1, np.nan, 0.2]), max_iters)
+        assert e.value.code == ENAN and "iteration 1" in str(e.value)
+        scf.close()
