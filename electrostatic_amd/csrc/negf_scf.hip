@@ -1132,28 +1132,45 @@ class BatchScf {
     // limit); per-tube iteration counts and final norms.
     int run(const double* V, double* U_out, double* Q_out, int* iters, double* norms, int* total_iters)
     {
-        int rc;
+        int rc, it = 0;
         LoopState ls;
         if ((rc = start_run(V, ls))) return rc;
-        int it = 0, launched = 0;
+        auto next = [&] { return enqueue_iteration(); };
+        if ((rc = iterate(ls, &it, [](int) { return NEGF_OK; }, next, -1))) return drain(rc);
+        return finish_run(it, ls, U_out, Q_out, iters, norms, total_iters);
+    }
+    // The loop of a run: before(it) on the host, then iteration it, and the next one ahead
+    // of it unless that is number hold.  *it counts the iterations.
+    template <class B, class F>
+    int iterate(LoopState& ls, int* count, B before, F enqueue, int hold)
+    {
+        int rc, launched = 0;
+        int& it = *count;
         while (ls.remaining > 0) {
             if (it > M + 1) {
                 ls.overflow = true;
                 break;
             }
+            if ((rc = before(it))) return rc;
             if (launched == it) {
-                if ((rc = launch_iteration(it, [&] { return enqueue_iteration(); }))) return rc;
+                if ((rc = launch_iteration(it, enqueue))) return rc;
                 ++launched;
             }
-            if (runs_ahead(it + 1)) {
-                if ((rc = launch_iteration(it + 1, [&] { return enqueue_iteration(); })))
-                    return rc;
+            if (it + 1 != hold && runs_ahead(it + 1)) {
+                if ((rc = launch_iteration(it + 1, enqueue))) return rc;
                 ++launched;
             }
             if ((rc = after_iteration(it, ls))) return rc;
             ++it;
         }
-        return finish_run(it, ls, U_out, Q_out, iters, norms, total_iters);
+        return NEGF_OK;
+    }
+    // A run that ends by an error: the iteration launched ahead still writes the batch's
+    // rows, the status words and the record, so it is waited for before the caller goes on.
+    int drain(int rc)
+    {
+        (void)hipStreamSynchronize(st);
+        return rc;
     }
 
     // ---- surrogate-seeded, preconditioned iteration
@@ -1291,32 +1308,18 @@ class BatchScf {
         }
         if (seed_iters > 0 && (rc = enqueue_capacitance())) return rc;
         NEGF_HIP_TRY(hipStreamSynchronize(st));
-        int it = 0, launched = 0;
-        while (ls.remaining > 0) {
-            if (it > M + 1) {
-                ls.overflow = true;
-                break;
-            }
-            if (it > 0 && it == refresh_iter) {
-                // new capacitances at the present potential; fresh history, n_in kept
-                if ((rc = enqueue_capacitance())) return rc;
-                std::vector<int> steps(T, 1);
-                NEGF_HIP_TRY(hipMemcpyAsync(d_steps.p, steps.data(), sizeof(int) * T, hipMemcpyHostToDevice, st));
-                NEGF_HIP_TRY(hipStreamSynchronize(st));
-            }
-            if (launched == it) {
-                if ((rc = launch_iteration(it, [&] { return enqueue_iteration_pc(); })))
-                    return rc;
-                ++launched;
-            }
-            if (it + 1 != refresh_iter && runs_ahead(it + 1)) {
-                if ((rc = launch_iteration(it + 1, [&] { return enqueue_iteration_pc(); })))
-                    return rc;
-                ++launched;
-            }
-            if ((rc = after_iteration(it, ls))) return rc;
-            ++it;
-        }
+        auto refresh = [&](int it) {
+            if (it == 0 || it != refresh_iter) return (int)NEGF_OK;
+            // new capacitances at the present potential; fresh history, n_in kept
+            if (int e = enqueue_capacitance()) return e;
+            std::vector<int> steps(T, 1);
+            NEGF_HIP_TRY(hipMemcpyAsync(d_steps.p, steps.data(), sizeof(int) * T, hipMemcpyHostToDevice, st));
+            NEGF_HIP_TRY(hipStreamSynchronize(st));
+            return (int)NEGF_OK;
+        };
+        auto next = [&] { return enqueue_iteration_pc(); };
+        int it = 0;
+        if ((rc = iterate(ls, &it, refresh, next, refresh_iter))) return drain(rc);
         rc = finish_run(it, ls, U_out, Q_out, iters, norms, total_iters);
         if (cap) NEGF_HIP_TRY(hipMemcpy(cap, d_c.p, sizeof(double) * T, hipMemcpyDeviceToHost));
         return rc;

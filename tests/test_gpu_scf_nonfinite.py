@@ -94,3 +94,33 @@ def test_one_system_of_all_tubes(dev, graph, max_iters):
             scf.bias_point(np.array([0.1, np.nan, 0.2]), max_iters)
         assert e.value.code == ENAN and "iteration 1" in str(e.value)
         scf.close()
+
+
+@pytest.mark.parametrize("ahead", [True, False])
+@pytest.mark.parametrize("surrogate", [False, True])
+def test_calls_after_an_error(dev, ahead, surrogate):
+    """The iteration launched ahead of the error has ended when the call returns: solves
+    on the same tubes and the next run give what they give on their own."""
+    with Setup(3, 64) as s:
+        s.scf.use_graph(ahead)
+        sg = Surrogate(s.N, seed=1)
+        s.scf.set_surrogate(sg)
+
+        def run(V):
+            s.scf.set_input_charge(np.zeros((3, s.N)))
+            return s.scf.run_surrogate(V, seed_iters=0, refresh_iter=2) if surrogate else s.scf.run(V)
+
+        want = run(s.V)
+        for t, u in zip(s.tubes, s.U_ext):
+            t.set_potential(u)
+        alone = [t.solve(1)[0] for t in s.tubes]
+        for _ in range(3):
+            with pytest.raises(_lib.NegfError) as e:
+                run(np.array([0.1, np.nan, 0.2]))
+            assert e.value.code == ENAN
+            for t, u, q in zip(s.tubes, s.U_ext, alone):
+                t.set_potential(u)
+                assert np.array_equal(t.solve(1)[0], q)
+            for a, b in zip(run(s.V), want):
+                assert np.array_equal(a, b)
+        sg.close()
