@@ -158,10 +158,16 @@ static void launch_sweep_pair(int ns, const WLaunch2& a, hipStream_t st)
 // ---------------------------------------------------------------- plan
 RgfPlan::~RgfPlan()
 {
-    DevBuf* bufs[] = {&d_tab_, &d_Tm_, &d_St_, &d_Dd_, &d_part_, &d_dos_part_};
-    for (DevBuf* b : bufs) b->release();
+    release();
     for (hipEvent_t e : ev_start_) (void)hipEventDestroy(e);
     for (hipEvent_t e : ev_stop_) (void)hipEventDestroy(e);
+}
+
+void RgfPlan::release()
+{
+    DevBuf* bufs[] = {&d_tab_, &d_Tm_, &d_St_, &d_Dd_, &d_part_, &d_dos_part_};
+    for (DevBuf* b : bufs) b->release();
+    nitems_ = 0;
 }
 
 int RgfPlan::kernel_time(double* total_ms, int* launches)

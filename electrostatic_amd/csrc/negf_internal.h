@@ -121,6 +121,13 @@ class RgfPlan {
     // The device status word itself (an int), for a copy enqueued by the caller.
     const int* status_ptr() const { return d_status_; }
     int num_items() const { return nitems_; }
+    // Device memory that the plan holds, and giving it back (enqueue() needs another
+    // build() then).
+    size_t held_bytes() const
+    {
+        return d_tab_.cap + d_Tm_.cap + d_St_.cap + d_Dd_.cap + d_part_.cap + d_dos_part_.cap;
+    }
+    void release();
     // hipEvent timing of the RGF kernels (transfer + scan + sweep)
     void enable_timing(bool on) { timing_ = on; }
     int kernel_time(double* total_ms, int* launches);

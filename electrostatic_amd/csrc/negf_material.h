@@ -110,6 +110,8 @@ class Tube {
     DecParams dec() const;
 
    private:
+    // Keeps the workspace of a DOS or current call for the next one up to a bound.
+    struct DosWorkspace;
     int take_charge(double* Q, const double* dQ);
     int upload_chains(DevBuf& buf, const std::vector<ChainDesc>& ch);
     void eq_chains_of(const Path& path, double cm, bool with_fermi, std::vector<ChainDesc>& out) const;
