@@ -204,11 +204,20 @@ static int fused_for(int P, bool few)
 // the default length would give fewer than it takes.  0 (the default) otherwise.
 // Measured, equilibrium charge with host part, short against default length: 64 to 4096
 // energies (1 to 64 groups) 46 .. 76 us against 49 .. 80 us at 40 to 1501 sites, diag G
-// of 1501 x 777 69 against 84 us; 128 groups (8192 energies) 88 against 81 us at 1000
-// sites, 95 against 87 us at 1501.  Above FUSED_FEW_GROUPS, where workgroups share the
+// of 1501 x 777 69 against 84 us.  Above FUSED_FEW_GROUPS, where workgroups share the
 // CUs, half the segments: 96 groups, 1024 / 600 / 256 sites, in us an SCF iteration: 16
 // segments 52.2 / 44.8 / 37.3, 32 segments 54.9 / 47.6 / - , the default length's
 // 59.0 / 54.6 / 48.9.
+//
+// The line lies where the fused launch's workgroups, two of 32 chains per group, take
+// every CU once.  16 segments against the default length, device time of one charge in
+// us at 128 groups: 100 / 256 / 600 / 1024 / 1501 / 2048 sites 15 / 18 / 22 / 26 / 32 / 34
+// against 31 / 27 / 34 / 31 / 44 / 43; with diag G written 19 / 30 / 37 / 44 / 71 / 69 against 41 / 49 /
+// 52 / 52 / 83 / 78; an SCF iteration at 114 groups 36 / 39 / 47 / 57 / - / 98 against 52 / 48 /
+// 59 / 60 / - / 106.  Beyond it the gain shrinks (192 groups: 22 / 27 / 41 / 41 / 52 / 54 against 35 / 31 / 40 /
+// 46 / 57 / 58) and turns for biased batches, whose two plans share the CUs (172 + 129
+// groups: 85 / 96 / 111 / 120 / - / 142 against 102 / 90 / 107 / 121 / - / 139; 128 + 96
+// groups: 81 / 88 / 96 / 104 / - / 123 against 101 / 87 / 99 / 107 / - / 131).
 static int segment_length_for(int N, int groups)
 {
     if (groups > RGF_FEW_GROUPS) return 0;

@@ -818,7 +818,7 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void scan_kernel(WLaunch lp, int n
 #define FUSED_CHAINS_MANY 32
 #define FUSED_FEW_GROUPS 32  // chain groups up to which FUSED_CHAINS_FEW is taken (one workgroup per CU)
 #define FUSED_MIN_SEGS 17
-#define RGF_FEW_GROUPS 96  // chain groups of a launch that counts as short of wavefronts
+#define RGF_FEW_GROUPS 128  // chain groups of a launch that counts as short of wavefronts: two workgroups each on 256 CUs
 #define FUSED_CHUNK 4
 
 // One walk over the segment matrices in LDS (V: the v walk), by CW lanes of one

@@ -15,12 +15,14 @@ def rel_err(a, ref):
     return np.abs(a - ref).max() / np.abs(ref).max()
 
 
-# 1, 2, 3, 16, 17 and 32 segments of 16, then of 32, 64 and 80 sites, last ones partial;
-# 2176 sites: the first length that keeps the default
+# 1, 2, 3, 16, 17 and 32 segments of 16, then of 32 and 48, then 64 sites, last ones
+# partial; 2049 sites: the first length that keeps the default (17 segments of 128)
 SIZES = [(2, 1), (16, 33), (17, 64), (40, 65), (256, 3), (257, 64), (500, 1), (512, 65), (513, 40), (1024, 64),
-         (1030, 65), (2175, 64), (2176, 5),
+         (1030, 65), (2048, 64), (2049, 64), (2175, 64), (2176, 5),
          # above 32 chain groups: at most 16 segments, 32 chains per workgroup
-         (40, 2049), (600, 2112), (1024, 2305)]
+         (40, 2048), (40, 2049), (600, 2112), (1024, 2305), (2048, 2049), (2049, 2049),
+         # 128 chain groups and one more
+         (40, 8192), (40, 8193), (300, 8192), (300, 8193)]
 
 
 @pytest.mark.parametrize("N,nE", SIZES)
