@@ -343,6 +343,26 @@ __device__ __forceinline__ void store_quad4_sym(double* Mre, double* Mim, const 
     }
 }
 
+// M <- (M + M^T) / 2 in LDS, by one wavefront: lane (h, i) takes the pairs of row i and
+// column i + k (mod 32), k = 1 + h, 3 + h, ..., 15 + h (of k = 16 every pair once).
+__device__ __forceinline__ void symmetrize_wave(double* Mre, double* Mim, int lane)
+{
+    wave_sync();
+    const int i = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int k = 1 + 2 * q + h, j = (i + k) & 31;
+        if (k == 16 && i >= 16) continue;
+        const int a = i * BLD + j, b = j * BLD + i;
+        const double re = 0.5 * (Mre[a] + Mre[b]), im = 0.5 * (Mim[a] + Mim[b]);
+        Mre[a] = re;
+        Mre[b] = re;
+        Mim[a] = im;
+        Mim[b] = im;
+    }
+    wave_sync();
+}
+
 // Sancho-Rubio decimation for one energy (blockIdx.x) and one lead
 // (blockIdx.y: 0 = left lead, surface = its last block, alpha = T^T;
 // 1 = right lead, surface = its first block, alpha = T), on-site H0 + Uc.
@@ -477,6 +497,12 @@ __global__ __launch_bounds__(BTHREADS) void sancho_rubio_kernel(int nE, const do
 // workgroup's wavefronts; H0 and the stored g_b are read through the caches.
 // KEEP_X: the forward product g_b T (computed for S) is stored beside g_b and
 // read back as the backward's X instead of being computed again.
+//
+// The products skip a quadrant because their results are symmetric; g_b and G_bb are
+// made so exactly, or the antisymmetric part that rounding leaves in the other quadrants
+// grows from block to block by |g T|^2 (dense T of 32 orbitals: 7e-10 of G after 7 blocks,
+// nothing left of it after 20).  Off by 1e-14 .. 1e-13 of G with it, as the recursion
+// with all quadrants.
 template <bool KEEP_X>
 __global__ __launch_bounds__(64 * WPB, 1) void block_rgf_kernel(int e0, int n, int nb, const double2* __restrict__ E,
                                                              const double2* __restrict__ coef,
@@ -563,6 +589,7 @@ __global__ __launch_bounds__(64 * WPB, 1) void block_rgf_kernel(int e0, int n, i
         }
         wave_sync();
         gj_inverse_wave(Cre, Cim, perm_s[w], lane);
+        symmetrize_wave(Cre, Cim, lane);
         if (b < nb - 1) {
             double* dst = gs + (size_t)b * 2 * BGL;
             for (int x = lane; x < BGL; x += 64) {
@@ -620,7 +647,7 @@ __global__ __launch_bounds__(64 * WPB, 1) void block_rgf_kernel(int e0, int n, i
         wmm<true, true, false, true, BLD, BLD, true>(G, Cre, Cim, Pre, Pim, lane);  // G_b = g_b + Y X^T
         wave_sync();
         store_quad4_sym(Cre, Cim, G, lane);
-        wave_sync();
+        symmetrize_wave(Cre, Cim, lane);
         emit(b);
     }
 }

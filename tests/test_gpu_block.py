@@ -44,8 +44,8 @@ def test_sancho_rubio_self_energies_match_oracle(dev):
 @pytest.mark.parametrize("keep_x", [True, False])
 @pytest.mark.parametrize("nb", [1, 2, 7])
 def test_block_rgf_diag_matches_oracle(dev, nb, keep_x):
-    # keep_x False: a scratch bound of one g_b set per energy makes the
-    # backward sweep recompute g_b T instead of reading it back
+    # ring blocks, which the two-part sweep takes: keep_x False bounds its
+    # scratch (the 32-wide sweep that recomputes g_b T: test_gpu_block_wide.py)
     H0, T, v, Uc = chain(nb, seed=nb)
     E = np.array([0.37 + 1e-5j, -0.8 + 1e-5j, 1.9 + 1e-3j, -2.6 + 0.05j, 0.02 + 1e-5j])
     c = negf.BlockChain(nb, H0, T)
@@ -100,10 +100,11 @@ def test_block_rgf_ring_traces_match_mode_space(dev):
 
 
 def test_block_rgf_energy_chunks_are_bit_identical(dev):
-    # a scratch limit of two energies' g_b splits 7 energies into sweeps of
-    # 2, 2, 2, 1 (the last workgroup partly empty); every energy is computed
-    # independently and the charge is summed in energy order, so the result
-    # equals the single sweep bit for bit
+    # a scratch limit below what 7 energies of the two-part sweep take splits
+    # them into several launches (sizes of either sweep:
+    # test_gpu_block_wide.py); every energy is computed independently and the
+    # charge is summed in a fixed order, so the result equals the single sweep
+    # bit for bit
     nb = 9
     H0, T, v, Uc = chain(nb, 5)
     E = np.array([0.37 + 1e-5j, -0.8 + 1e-5j, 1.9 + 1e-3j, -2.6 + 0.05j, 0.02 + 1e-5j, 0.9 + 1e-2j,
