@@ -82,8 +82,8 @@ def test_zero_coupling(dev):
 
 def test_singular_parts_take_the_pivoted_elimination(dev):
     """H_00 = H_11 = 0 with energies at the bare level: the first pivots of the
-    leads' elimination are Im E, far below the couplings (limit 8), and one
-    orbital of the chain is tuned to a multiplier above its limit (256)."""
+    leads' elimination are Im E, far below the couplings (limit 8).  The chain's own
+    pivoted elimination is reached by test_gpu_block_pivot.py."""
     m, h, nb = 12, 6, 3
     rng = np.random.default_rng(7)
     H0 = np.zeros((m, m))
