@@ -706,7 +706,10 @@ struct TrackOut {
 // to run (0: none), steps[2T + 1] the tubes still active (0 or less: the loop has
 // ended, and the potential stays too).  Row sum, charge, update and record in one launch instead of four: 32
 // tubes x 1024 sites, 16.6 us against 3.9 + 2.9 + 14.8 + 3.9.
-template <bool PC>
+// SMALL (at most kBroydenThreads sites) and the general update are kernels of their own: as
+// one with a branch the general one runs at half the speed (104 registers instead of
+// 53); 3 tubes x 6000 / 2048 / 1200 sites 265 / 81 / 54 us an iteration, now 204 / 68 / 52.
+template <bool PC, bool SMALL>
 __global__ __launch_bounds__(kBroydenThreads) void broyden_batch_kernel(int S, int T, int max_step, double fraction,
                                                                           int norm_type, ChargeRows cr, double* n_out_all,
                                                                           const double* __restrict__ PF,
@@ -767,12 +770,11 @@ __global__ __launch_bounds__(kBroydenThreads) void broyden_batch_kernel(int S, i
     b.out = base.out + (size_t)t * 4;
     b.PFp = PC ? base.PFp + t * state_stride : nullptr;
     const bool limit = m > max_step;
-    if (limit) {
-        // nothing more
-    } else if (S <= kBroydenThreads) {
-        broyden_update_small<PC>(S, m, fraction, norm_type, q, PC ? PF + o : nullptr, b);
-    } else {
-        broyden_update<PC>(S, m, fraction, norm_type, n_out, PC ? PF + o : nullptr, b);
+    if (!limit) {  // uniform
+        if constexpr (SMALL)
+            broyden_update_small<PC>(S, m, fraction, norm_type, q, PC ? PF + o : nullptr, b);
+        else
+            broyden_update<PC>(S, m, fraction, norm_type, n_out, PC ? PF + o : nullptr, b);
     }
     if (tid == 0) {  // b.out[0..2] were written by this thread
         if (!limit) steps[t] = m + 2;
@@ -992,9 +994,20 @@ class BatchScf {
         rc = batch_enqueue(batch, d_Q.as<double>(), st, d_active.as<int>(), !fuse);
         if (rc) return rc;
         if (fuse) cr = ChargeRows{br.part, br.off, br.nrows, br.eq, br.neq, br.rho0};
-        hipLaunchKernelGGL(broyden_batch_kernel<false>, dim3(T), dim3(kBroydenThreads), 0, st, N, T, M,
-                           p.Broyden_fraction, p.Broyden_norm_type, cr, d_Q.as<double>(), nullptr, base(),
-                           state_stride, hist_stride, d_steps.as<int>(), d_active.as<int>(), track_out());
+        return enqueue_broyden<false>(cr, nullptr);
+    }
+    template <bool PC>
+    int enqueue_broyden(const ChargeRows& cr, const double* PF)
+    {
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(T), dim3(kBroydenThreads), 0, st, N, T, M, p.Broyden_fraction,
+                               p.Broyden_norm_type, cr, d_Q.as<double>(), PF, base(), state_stride, hist_stride,
+                               d_steps.as<int>(), d_active.as<int>(), track_out());
+        };
+        if (N <= kBroydenThreads)
+            launch(broyden_batch_kernel<PC, true>);
+        else
+            launch(broyden_batch_kernel<PC, false>);
         NEGF_HIP_TRY(hipGetLastError());
         return NEGF_OK;
     }
@@ -1268,12 +1281,7 @@ class BatchScf {
         if (!rc) rc = batch_enqueue(batch, d_Q.as<double>(), st, d_active.as<int>());
         if (!rc) rc = enqueue_precondition(d_Q.as<double>());
         if (rc) return rc;
-        hipLaunchKernelGGL(broyden_batch_kernel<true>, dim3(T), dim3(kBroydenThreads), 0, st, N, T, M,
-                           p.Broyden_fraction, p.Broyden_norm_type, ChargeRows(), d_Q.as<double>(),
-                           d_PF.as<double>(), base(), state_stride, hist_stride, d_steps.as<int>(),
-                           d_active.as<int>(), track_out());
-        NEGF_HIP_TRY(hipGetLastError());
-        return NEGF_OK;
+        return enqueue_broyden<true>(ChargeRows(), d_PF.as<const double>());
     }
     // Seed steps are half steps: with full steps the scalar capacitance
     // overshoots on the high-gate tubes, whose seed then oscillates (128

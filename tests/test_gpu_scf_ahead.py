@@ -90,3 +90,26 @@ def test_input_charge_round_trip(T, cells):
         assert np.array_equal(scf.get_input_charge(), k * n)
     scf.close()
     batch.close()
+
+
+@pytest.mark.parametrize("cells", [256, 257])
+def test_batch_against_single(cells):
+    """The last size of the small Broyden update and the first of the general one: both
+    loops stop at a residual of 1e-8 e, so their potentials agree to 1e-6 V."""
+    V = np.array([0.2, 0.6])
+    tubes = tubes_of(2, cells)
+    batch = negf.Batch(tubes)
+    sp = dict(SP, Broyden_max_norm=1e-8, Broyden_threshold_maxstep=200)
+    U_ext = np.stack([gaussian_bumps(tubes[0].N, seed=t, amp=0.2) for t in range(2)])
+    scf = negf.BatchScf(batch, **sp)
+    scf.set_external_potential(U_ext)
+    scf.set_input_charge(np.zeros(U_ext.shape))
+    U, Q, it, norms, _ = scf.run(V)
+    scf.close()
+    batch.close()
+    for t in range(2):
+        one = negf.Scf(tubes[t], **sp)
+        one.set_external_potential(U_ext[t])
+        U1, Q1 = one.bias_point(V[t])[:2]
+        one.close()
+        assert np.abs(U[t] - U1).max() < 1e-6 and np.abs(Q[t] - Q1).max() < 1e-6
