@@ -94,7 +94,7 @@ def scf_sweep(with_cpu=True):
     potential = 4 seeded Gaussians (amplitude <= 0.3 eV), metal voltage 0..1 V
     in 0.1 V steps, Broyden fraction 0.1, absolute norm <= 1e-6, warm start.
     Reports bias points per second on the GPU (whole SCF loop per bias point,
-    device-resident, each iteration replayed from one captured graph) and for
+    device-resident, iterations launched ahead of the convergence test) and for
     the oracle's serial SCF on one host thread."""
     from electrostatic_amd import negf
     from electrostatic_amd.workloads import gaussian_bumps
@@ -290,7 +290,7 @@ def surrogate_leg(dev, n_pairs=20000, epochs=5, with_cpu=True):
                 ("surrogate_seeded", lambda: scf.run_surrogate(V, seed_iters=6, refresh_iter=0)))
     for key, fn in variants:
         scf.set_input_charge(np.zeros((T, N)))
-        fn()                      # warm-up: graph capture, path set-up
+        fn()                      # warm-up: path set-up
         scf.set_input_charge(np.zeros((T, N)))
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -353,10 +353,12 @@ def block_leg(steps=3, with_cpu=True):
     orbitals), 2000 blocks, 1024 energies (512 on a contour arc, 512 on the
     real axis [-3, 3] eV with eta = 1e-5 eV), on-site disorder N(0, 0.05 eV)
     per orbital (seed 4) plus a smooth potential; Sancho-Rubio leads to
-    1e-12.  Algorithmic flops per energy-block: 36 m^3 (forward: g T, T^T (gT),
-    inverse; backward: g T, X G, Y X^T; real H0 and T).  The general-block
-    count of the same sweep (complex T, a second inverse for G: 56 m^3) is
-    reported beside it."""
+    1e-12.  The coupling joins half blocks, so the two-part sweep takes it:
+    10 m^3 flops per energy-block (six complex inverses of m / 2 orbitals, g
+    from either side and G of both parts, and two real-by-complex products for
+    each of the four coupling steps; real H0 and T).  The 32-wide sweep of a general coupling
+    (36 m^3: forward g T, T^T (gT), inverse; backward g T, X G, Y X^T) is
+    named beside it."""
     from electrostatic_amd import negf
     from electrostatic_amd.workloads import zigzag_ring_blocks
     nb, nE, m = 2000, 1024, 32
@@ -380,18 +382,18 @@ def block_leg(steps=3, with_cpu=True):
     c.close()
     if not np.all(np.isfinite(acc)):
         raise RuntimeError("non-finite block charge")
-    flops = 36 * m ** 3 * nb * nE
+    flops = 10 * m ** 3 * nb * nE
     rg = float(np.median(rgf_ms))
     out = {"workload": "(16,0) tube, 2000 blocks of 32 orbitals, 1024 energies, disorder N(0, 0.05 eV) "
                        "+ smooth U, Sancho-Rubio to 1e-12",
            "ms_per_evaluation": wall, "ms_sancho_rubio": float(np.median(sr_ms)), "ms_block_rgf": rg,
            "sancho_rubio_iterations_max": int(it.max()),
            "energy_blocks_per_s": nb * nE / (wall * 1e-3),
-           "flop_per_energy_block": 36 * m ** 3,
+           "flop_per_energy_block": 10 * m ** 3,
            "rgf_tflops": flops / (rg * 1e-3) / 1e12,
            "rgf_frac_fp64_peak": flops / (rg * 1e-3) / 1e12 / FP64_PEAK_TFLOPS,
-           "note": "fraction at the general sweep's 36 m^3 flops per energy-block (real H0 and T); "
-                   "a general complex block would need 56 m^3"}
+           "note": "fraction at the two-part sweep's 10 m^3 flops per energy-block (real H0 and T, half-block "
+                   "coupling); the sweep of a general real coupling takes 36 m^3"}
     if with_cpu:
         from oracle import block_oracle as B
         # numpy oracle on 4 energies of the same chain

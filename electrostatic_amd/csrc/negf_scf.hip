@@ -1358,8 +1358,8 @@ class BatchScf {
 // The potential of one SCF iteration written where the loop and the tube
 // read it: U_i = U_ext_i - V - sum_j K_ij n_j (the sum as in
 // coulomb_potential_kernel) into U and tU, the contact potentials U_0 and
-// U_{N-1} into tUc.  V is read from the device so that one captured
-// iteration serves every bias point.
+// U_{N-1} into tUc.  V is read from the device, with the flag that says whether the
+// loop still runs: an iteration launched ahead needs nothing from the host.
 __global__ __launch_bounds__(256) void scf_potential_kernel(int N, const double* __restrict__ K,
                                                             const double* __restrict__ n,
                                                             const double* __restrict__ U_ext,
@@ -1830,8 +1830,7 @@ int negf_batch_scf_set_external_potential(negf_batch_scf* s, const double* U_ext
         set_error("null argument");
         return NEGF_EARG;
     }
-    // The captured iteration reads d_Uext by address, so setting or clearing
-    // U_ext only rewrites that buffer (zeros when cleared): no graph goes stale.
+    // The iterations read d_Uext by address: cleared means zeros.
     BatchScf& b = s->s;
     const long long NT = (long long)b.N * b.T;
     NEGF_HIP_TRY(hipStreamSynchronize(b.st));
