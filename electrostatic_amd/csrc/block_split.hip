@@ -50,9 +50,9 @@
 // written out twice, at the same time.  Measured, 500 blocks of 32 orbitals, 1024
 // energies: sweep 8.6 ms against 20.5 ms for the 32-orbital sweep (one wavefront
 // per energy, pivoted inverse of 1600 cycles per step) and 9.0 ms with 32-bit DPP
-// moves and two Newton steps; leads 0.90 ms against 4.5 ms (four wavefronts and a
+// moves and two Newton steps; leads 1.08 ms against 4.5 ms (four wavefronts and a
 // barrier per pivot step); 40 blocks of 20 orbitals, 143 energies: 0.31 against
-// 1.6 ms and 0.21 against 0.53 ms.
+// 1.6 ms and 0.27 against 0.53 ms.
 #include "block_split.h"
 
 #include <algorithm>
@@ -266,47 +266,85 @@ __device__ __forceinline__ double row_lane(double x)
 }
 
 // A multiplier of a later row above the limit (squared here) sends the matrix to
-// the pivoted inverse16s: up to 6% of the blocks at energies within the edge states
-// of a disordered (16,0) tube, under 1% elsewhere; the bits lost below it are fewer
-// than the condition of those blocks costs (diag G within 1e-10 of the dense inverse
-// given Sigma, as with a limit of 8, which took 16 instead of 9 ms for 500 x 1024 as
-// half of those blocks are inverted twice).
-constexpr double CHAIN_GROW2 = 256.0 * 256.0;
+// the pivoted inverse16s.  The sweep of the chain (256): up to 6% of the blocks at
+// energies within the edge states of a disordered (16,0) tube, under 1%
+// elsewhere; the bits lost there are fewer than the condition of those blocks
+// costs (diag G within 1e-10 of the dense inverse given Sigma, as with a limit
+// of 8, which took 16 instead of 9 ms for 500 x 1024 as half of those blocks
+// are inverted twice).
+// The leads (4): the doublings amplify every error.  Mean of log10(error of Sigma,
+// 80-bit references) less that of the 32-orbital kernel, ring tubes and random chains of 8 to 32
+// orbitals, Im E 1e-5 .. 0.1 / on the contour (largest of a chain and Im E), and the time
+// of a solve of 40 blocks of 20 orbitals: limit 8 0.16 / -0.08 (0.58), 652 us; 5 0.08 /
+// -0.08 (0.28), 688; 4 0.05 / -0.08 (0.14), 730; 3 0.02 / -0.08 (0.12), 883; pivoted always
+// 0.01 / 0.01 (0.12), 857.  256 costs up to four digits.
+constexpr double CHAIN_GROW2 = 256.0 * 256.0, LEAD_GROW2 = 4.0 * 4.0;
 
 // Elimination step on column 4 T + K of a panel x (columns 4 T .. 4 T + 3; lane
-// (i, q): row i, column 4 T + q), pivot in row 4 T + K.  Ends with -A_iJ P^-1 in
-// the other rows and P^-1 in rows J.
-template <int T, int K>
-__device__ __forceinline__ void panel_step(double2& x, int lane, bool& grow)
+// (i, q): row i, column 4 T + q), pivot in row 4 T + K of the panel's own part.
+// x[1] (if NR = 2): the panel's rows in the other part, check: not yet pivots.
+// Ends with -A_iJ P^-1 in the other rows and P^-1 in rows J.  In the leads (NR = 2) the
+// products are formed before they are added, as in inverse16s.
+template <int T, int K, int NR>
+__device__ __forceinline__ void panel_step(double2 (&x)[NR], int lane, bool& grow, bool check = false)
 {
     constexpr int row = 4 * T + K;
     asm volatile("" : "+v"(lane));  // the lane masks are made here: kept over all steps they spill
     const int i = lane & 15;
     const int addr = (K * 16 + i) * 4;
     const bool col = (lane >> 4) == K, prow = i == row;
-    const double2 c = make_double2(bperm64(addr, x.x), bperm64(addr, x.y));
-    const double pr = row_lane<row>(c.x), pi = row_lane<row>(c.y);
+    double2 c[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) c[r] = make_double2(bperm64(addr, x[r].x), bperm64(addr, x[r].y));
+    const double pr = row_lane<row>(c[0].x), pi = row_lane<row>(c[0].y);
     // 1 / |pivot|^2: estimate and one third-order step y (1 + e + e^2), e = 1 - d y
     const double d = fma(pr, pr, pi * pi), y = __builtin_amdgcn_rcp(d), ee = fma(-d, y, 1.0);
     const double iv = fma(y, fma(ee, ee, ee), y);
     const double ir = pr * iv, ni = pi * iv;  // 1 / pivot = ir - i ni
-    double rr = row_lane<row>(x.x), ri = row_lane<row>(x.y);
+    double rr = row_lane<row>(x[0].x), ri = row_lane<row>(x[0].y);
     rr = col ? 1.0 : rr;
     ri = col ? 0.0 : ri;
-    // -c / pivot
-    double fr = -fma(c.x, ir, c.y * ni), fi = fma(c.x, ni, -c.y * ir);
-    grow |= !(fma(fr, fr, fi * fi) <= CHAIN_GROW2) && i > row;
-    fr = prow ? ir : fr;
-    fi = prow ? -ni : fi;
-    const bool z = prow || col;
-    const double br = z ? 0.0 : x.x, bi = z ? 0.0 : x.y;
-    x.x = fma(fr, rr, fma(-fi, ri, br));
-    x.y = fma(fr, ri, fma(fi, rr, bi));
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+        // -c / pivot
+        double fr = -fma(c[r].x, ir, c[r].y * ni), fi = fma(c[r].x, ni, -c[r].y * ir);
+        const bool big = !(fma(fr, fr, fi * fi) <= (NR == 1 ? CHAIN_GROW2 : LEAD_GROW2));
+        grow |= r == 0 ? big && i > row : check && big;
+        const bool p = r == 0 && prow;
+        fr = p ? ir : fr;
+        fi = p ? -ni : fi;
+        const bool z = p || col;
+        const double br = z ? 0.0 : x[r].x, bi = z ? 0.0 : x[r].y;
+        if (NR == 1) {
+            x[r].x = fma(fr, rr, fma(-fi, ri, br));
+            x[r].y = fma(fr, ri, fma(fi, rr, bi));
+        } else {
+            x[r].x = br + fma(fr, rr, -fi * ri);
+            x[r].y = bi + fma(fr, ri, fi * rr);
+        }
+    }
 }
 
-// a(i, j) += sum_k o[j][k] b[i][k] for panels o and b
+template <int T>
+__device__ __forceinline__ void panel_steps(double2 (&x)[2], int lane, bool& grow, bool check)
+{
+    panel_step<T, 0, 2>(x, lane, grow, check);
+    panel_step<T, 1, 2>(x, lane, grow, check);
+    panel_step<T, 2, 2>(x, lane, grow, check);
+    panel_step<T, 3, 2>(x, lane, grow, check);
+}
+
+// a(i, j) += sum_k o[j][k] b[i][k] for panels o and b (SUM: the sum formed first)
+template <bool SUM = false>
 __device__ __forceinline__ void rank4(M16& a, const double2& o, const double2& b)
 {
+    if constexpr (SUM) {
+        M16 c = zero16();
+        rank4(c, o, b);
+        a.re += c.re;
+        a.im += c.im;
+        return;
+    }
     a.re = mfma64(o.x, b.x, a.re);
     a.im = mfma64(o.x, b.y, a.im);
     a.re = mfma64(-o.y, b.y, a.re);
@@ -331,23 +369,23 @@ __device__ __forceinline__ void clear_rows(M16& a, int lane)
 template <int NS, int NB, int T = 0>
 __device__ __forceinline__ void sweep16(M16 (&a)[NB], int lane, bool (&grow)[NB])
 {
-    double2 x[NB], o[NB];
+    double2 x[NB][1], o[NB];
 #pragma unroll
-    for (int n = 0; n < NB; ++n) x[n] = o[n] = make_double2(a[n].re[T], a[n].im[T]);
+    for (int n = 0; n < NB; ++n) x[n][0] = o[n] = make_double2(a[n].re[T], a[n].im[T]);
 #pragma unroll
-    for (int n = 0; n < NB; ++n) panel_step<T, 0>(x[n], lane, grow[n]);
+    for (int n = 0; n < NB; ++n) panel_step<T, 0, 1>(x[n], lane, grow[n]);
 #pragma unroll
-    for (int n = 0; n < NB; ++n) panel_step<T, 1>(x[n], lane, grow[n]);
+    for (int n = 0; n < NB; ++n) panel_step<T, 1, 1>(x[n], lane, grow[n]);
 #pragma unroll
-    for (int n = 0; n < NB; ++n) panel_step<T, 2>(x[n], lane, grow[n]);
+    for (int n = 0; n < NB; ++n) panel_step<T, 2, 1>(x[n], lane, grow[n]);
 #pragma unroll
-    for (int n = 0; n < NB; ++n) panel_step<T, 3>(x[n], lane, grow[n]);
+    for (int n = 0; n < NB; ++n) panel_step<T, 3, 1>(x[n], lane, grow[n]);
 #pragma unroll
     for (int n = 0; n < NB; ++n) {
         clear_rows<T>(a[n], lane);
-        rank4(a[n], o[n], x[n]);
-        a[n].re[T] = -x[n].x;
-        a[n].im[T] = -x[n].y;
+        rank4(a[n], o[n], x[n][0]);
+        a[n].re[T] = -x[n][0].x;
+        a[n].im[T] = -x[n][0].y;
     }
     if constexpr (4 * T + 4 < NS) sweep16<NS, NB, T + 1>(a, lane, grow);
 }
@@ -414,6 +452,46 @@ __device__ __forceinline__ M16 symmetric16(const M16& m, double* lds, int lane)
 {
     const M16 t = transpose16(m, lds, lane);
     return M16{0.5 * (m.re + t.re), 0.5 * (m.im + t.im)};
+}
+
+// -A^-1 of the 32 x 32 complex symmetric matrix of the parts pp, rp (rows R,
+// columns P) and rr, by the sweep over the columns of P, then of R.  On return
+// rp holds the rows P, columns R.
+template <int NS, int T = 0>
+__device__ __forceinline__ void sweep32_part(M16& own, M16& cross, M16& other, int lane, bool& grow, bool check)
+{
+    double2 x[2] = {make_double2(own.re[T], own.im[T]), make_double2(cross.re[T], cross.im[T])};
+    const double2 o0 = x[0], o1 = x[1];
+    panel_steps<T>(x, lane, grow, check);
+    clear_rows<T>(own, lane);
+    rank4<true>(own, o0, x[0]);
+    rank4<true>(cross, o0, x[1]);
+    rank4<true>(other, o1, x[1]);
+    own.re[T] = -x[0].x;
+    own.im[T] = -x[0].y;
+    cross.re[T] = -x[1].x;
+    cross.im[T] = -x[1].y;
+    if constexpr (4 * T + 4 < NS) {
+        if (__any(grow)) return;  // the caller discards the matrix
+        sweep32_part<NS, T + 1>(own, cross, other, lane, grow, check);
+    }
+}
+
+template <int NS>
+__device__ __forceinline__ bool sweep32(M16& pp, M16& rp, M16& rr, double* lds, int lane)
+{
+    // the columns of P, then (parts exchanged, one copy of the code) those of R
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+        bool grow = false;
+        sweep32_part<NS>(pp, rp, rr, lane, grow, half == 0);
+        if (__any(grow)) return false;
+        if (half == 0) rp = transpose16(rp, lds, lane);
+        const M16 t = pp;
+        pp = rr;
+        rr = t;
+    }
+    return true;
 }
 
 // E - H - diag(v) - ... of one part: the diagonal of rows i < np gets (er, ei)
@@ -552,16 +630,12 @@ __global__ __launch_bounds__(128, 2) void split_rgf_kernel(SplitChain c, int e0,
 // alpha, and beta = alpha^T.  With G = (E - eps)^-1 (32 x 32, parts PP .. RR):
 //   eps_PP += a G_RR a^T (and the surface's),  eps_RR += a^T G_PP a,
 //   a <- a G_RP a,   Sigma = a0 g_RR a0^T on part P,  g = (E - eps_s)^-1.
-// The doublings amplify every error, and the bare parts (E - H_PP) can be singular
-// on the real axis, so G comes from the pivoted 32-column elimination, G_PR as the
-// mean of it and the transpose of G_RP, and the updates of eps are made exactly
-// symmetric: without that an antisymmetric rounding error doubles with every
-// iteration (1e-8 of Sigma after 22 at E = -0.9 + 1e-5i on the (16,0) tube; 7e-13
-// with it).  Against 80-bit references (ring tubes and random chains of 8 to 32 orbitals,
-// Im E 1e-5 .. 0.1 and the contour) the error of Sigma is that of the 32-orbital
-// kernel, 10^(0.0 +- 0.1) of it in the mean of the logarithms; the symmetric sweep with a
-// limit of 8 on the multipliers was 10^(0.1 .. 0.65) above it.  500 x 1024: 1.27 ms, the
-// sweep's 0.87, the 32-orbital kernel's 4.5.
+// The bare parts (E - H_PP) can be singular on the real axis, where the sweep
+// over P grows and the pivoted 32-column elimination takes over; G_PR is then the mean of
+// it and the transpose of G_RP (the sweep's are one matrix).  The updates
+// of eps are made exactly symmetric: without that an antisymmetric rounding
+// error doubles with every iteration (1e-8 of Sigma after 22 at E = -0.9 + 1e-5i
+// on the (16,0) tube; 7e-13 with it).
 template <int NS>
 __global__ __launch_bounds__(128, 1) void split_sr_kernel(SplitChain c, const double2* __restrict__ E, double Uc0,
                                                           double Uc1, double tol, int max_iter,
@@ -583,12 +657,18 @@ __global__ __launch_bounds__(128, 1) void split_sr_kernel(SplitChain c, const do
     M16 es = M16{HP, zr}, eP = es, eR = M16{HR, zr};
     // -G of the on-site matrices p, r: parts PP, PR, RR
     auto green = [&](const M16& p, const M16& r, M16& gpp, M16& gpr, M16& grr) {
+        gpp = M16{-p.re, -p.im};
+        gpr = M16{-HRP, zr};  // rows R, columns P until the sweep exchanges them
+        grr = M16{-r.re, -r.im};
+        add_diag(gpp, er, ei, nP, lane);
+        add_diag(grr, er, ei, nR, lane);
+        if (sweep32<NS>(gpp, gpr, grr, lds, lane)) return;
         M16 G[2][2] = {{M16{-p.re, -p.im}, M16{-HPR, zr}}, {M16{-HRP, zr}, M16{-r.re, -r.im}}};
         add_diag(G[0][0], er, ei, nP, lane);
         add_diag(G[1][1], er, ei, nR, lane);
         inverse16s<2, NS>(G, lds, lane);
-        const M16 t = transpose16(G[1][0], lds, lane);
         gpp = M16{-G[0][0].re, -G[0][0].im};
+        const M16 t = transpose16(G[1][0], lds, lane);
         gpr = M16{-0.5 * (G[0][1].re + t.re), -0.5 * (G[0][1].im + t.im)};
         grr = M16{-G[1][1].re, -G[1][1].im};
     };
